@@ -1650,6 +1650,7 @@ int dmrj_ctx_create(int device, dmrj_ctx** out) {
     HIP_OK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
     HIP_OK(hipEventCreateWithFlags(&c->side_in, hipEventDisableTiming));
     HIP_OK(hipEventCreateWithFlags(&c->side_out, hipEventDisableTiming));
+    HIP_OK(hipEventCreateWithFlags(&c->poll, hipEventDisableTiming));
     hipDeviceProp_t prop;
     HIP_OK(hipGetDeviceProperties(&prop, device));
     c->num_cu = prop.multiProcessorCount;
@@ -1682,6 +1683,7 @@ int dmrj_ctx_destroy(dmrj_ctx* c) {
   c->release_transients();
   if (c->side_in) (void)hipEventDestroy(c->side_in);
   if (c->side_out) (void)hipEventDestroy(c->side_out);
+  if (c->poll) (void)hipEventDestroy(c->poll);
   if (c->side) (void)hipStreamDestroy(c->side);
   for (auto& g : c->graph_exec)
     if (g) (void)hipGraphExecDestroy(g);

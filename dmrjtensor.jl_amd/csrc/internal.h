@@ -191,6 +191,7 @@ struct Context {
   // large sectors; side_in / side_out order it against the main stream
   hipStream_t side = nullptr;
   hipEvent_t side_in = nullptr, side_out = nullptr;
+  hipEvent_t poll = nullptr;  // host's look at the main stream's progress (Jacobi SVD)
   void* rocblas = nullptr;   // rocblas_handle
   // batching of the SVD's batched symmetric eigensolves: 1 = size classes by
   // the cost model, 0 = one batch padded to the largest sector, 2 = one batch
@@ -226,8 +227,8 @@ struct Context {
   size_t lds_max = 65536;  // dynamic LDS per work-group (device property)
   // tuning: preferred GEMM tile config per operation (-1 = automatic)
   int gemm_cfg_override = -1;
-  // SVD backend: 0 = batched Jacobi for small sectors + batched symmetric
-  // eigensolver of the augmented matrix for large ones, 1 = gesdd,
+  // SVD backend: 0 = batched Jacobi for small sectors + QR-preconditioned
+  // block Jacobi for large ones, 1 = gesdd,
   // 2 = gesvd, 3 = batched Jacobi for small sectors + gesvd
   int svd_backend = 0;
   double bj_calls = 0, bj_sweeps = 0;  // block-Jacobi SVD calls and sweeps
@@ -375,6 +376,48 @@ struct CompleteJob {
   double* seld = nullptr;  // 32
   int* cand = nullptr;     // 32
 };
+// ---- QR-preconditioned block Jacobi for large SVD sectors (svd_qrj.hip) ----
+struct QjJob {
+  const double* M;        // R x C, column-major, ld R
+  double* A[4];           // working panels: o x n, n x K, K x K, K x K
+  double* T[3];           // triangular factors of the block reflectors, 256 doubles a panel
+  double* nrm;            // column norms: of A0 (squares, n), then of A3 (16 per panel)
+  int* perm;              // n: column of A0 at every place of the sorted order
+  int* last;              // last Jacobi round that rotated
+  const int* kcol;        // kept columns of A3, in the order of the vectors
+  const double* kinv;     // their reciprocal norms
+  double* out;            // vectors: element i of vector k at out[i es + k vs]
+  int64_t es, vs;
+  int R, o, n, K, dir, keep;
+};
+struct QjSector {
+  // set by the caller: the sector, and the sizes of A0 (o x n; the wanted
+  // vectors have n elements), K = min(o, n)
+  const double* M = nullptr;
+  int R = 0, o = 0, n = 0, K = 0, dir = 0, index = 0;
+  // set by qj_solve: singular values descending, their columns, reciprocals
+  std::vector<double> sigma, inv;
+  std::vector<int> col;
+  // set by the caller before qj_vectors
+  int keep = 0;
+  double* out = nullptr;
+  int64_t es = 0, vs = 0;
+};
+struct QjBatch {
+  Context& c;
+  std::vector<QjSector> sec;
+  std::vector<QjJob> jobs;
+  double* work = nullptr;
+  int* ints = nullptr;
+  explicit QjBatch(Context& c_) : c(c_) {}
+  QjBatch(const QjBatch&) = delete;
+  QjBatch& operator=(const QjBatch&) = delete;
+  ~QjBatch();
+};
+bool qj_fits(int64_t R, int64_t C);  // sector sizes the register-resident kernels take
+bool qj_solve(QjBatch& q, double norm2);
+void qj_vectors(QjBatch& q);
+
 // A new tensor handle of the given kind (0 site, 1 left env, 2 right env) and
 // its device storage for the current block table (api.hip).
 ::dmrj_tensor* new_tensor(Context& c, int kind);

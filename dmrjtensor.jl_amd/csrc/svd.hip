@@ -1,8 +1,9 @@
 // Truncated SVD of a two-site tensor (fsvd! of the reference's twostep,
 // algs/DMRG.jl:387-395): the tensor is cut into centre-charge sectors, every
 // sector is decomposed by the selected backend (batched one-sided Jacobi for
-// sectors up to 64, batched symmetric eigensolves of the augmented or Gram
-// matrices, block one-sided Jacobi, or rocSOLVER's SVDs), the singular
+// sectors up to 64, QR-preconditioned block Jacobi, batched symmetric
+// eigensolves of the augmented or Gram matrices, block one-sided Jacobi, or
+// rocSOLVER's SVDs), the singular
 // values of all sectors are sorted and truncated together, and the kept
 // vectors are split into the left and right tensors.
 #include <hip/hip_runtime.h>
@@ -91,6 +92,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     double* X = nullptr;
     int bj = 0, rowsX = 0, ncolsX = 0;
     int qr = 0;  // one-factor sector solved through its LQ / QR triangle (X: K x K factor)
+    int qj = -1;   // index in the QR-preconditioned Jacobi batch
     int gram = 0;  // orthonormal factor = eigenvectors of the Gram matrix (orthonormal to working precision)
     std::vector<int> perm;
     std::vector<double> hn;
@@ -324,6 +326,37 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       }
     }
   }
+  // large sectors, default backend: QR-preconditioned block Jacobi
+  // (svd_qrj.hip) for the vectors of the side that must come out orthonormal;
+  // the other factor by the grouped GEMM below.  Sectors it does not take
+  // (longer than its register-resident slabs, or not converged within its
+  // sweep limit) and tensors whose squared norm under- or overflows go to the
+  // eigensolves of the augmented matrices.
+  QjBatch qj(c);
+  if (!z && c.svd_backend == 0 && aa2 > 1e-305 && aa2 < 1e305) {
+    for (int si : order) {
+      Sec& s = secs[si];
+      if (s.kmin == 0 || is_small[si] || !qj_fits(s.R, s.C)) continue;
+      QjSector q;
+      q.M = s.M;
+      q.R = (int)s.R;
+      q.o = (int)(dir > 0 ? s.C : s.R);
+      q.n = (int)(dir > 0 ? s.R : s.C);
+      q.K = s.kmin;
+      q.dir = dir;
+      q.index = si;
+      qj.sec.push_back(q);
+    }
+    if (!qj.sec.empty() && qj_solve(qj, aa2))
+      for (size_t b = 0; b < qj.sec.size(); ++b) {
+        Sec& s = secs[qj.sec[b].index];
+        s.qj = (int)b;
+        s.bj = 1;
+        is_small[qj.sec[b].index] = 1;  // handled
+        const double mm = (double)std::max(s.R, s.C), nn = (double)s.kmin;
+        svd_flops += 4.0 * mm * nn * nn + 8.0 * nn * nn * nn;
+      }
+  }
   // large sectors, backend 5: batched symmetric eigensolve of the Gram matrix
   // of the side that must come out orthonormal (M M^T for dir > 0, M^T M for
   // dir < 0: size n = R or C instead of R + C); eigenvalues sigma^2 carry an
@@ -400,7 +433,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       }
     }
   }
-  // large sectors, default backend: one batched symmetric eigensolve of the
+  // what the default backend has left: one batched symmetric eigensolve of the
   // augmented matrices [[0, M], [M^T, 0]] (eigenvalues +-sigma, absolute
   // accuracy eps |M| like a bidiagonal SVD, no squaring of M)
   double* aug = nullptr;
@@ -705,6 +738,8 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
           s.colsrc.push_back(gramZ + gramZoff[b] + (int64_t)(Nb - 1 - l) * Nb);
           s.coldiv.push_back(1.0);
         }
+      } else if (s.qj >= 0) {
+        for (int l = 0; l < s.kmin; ++l) hs[o + l] = qj.sec[s.qj].sigma[l];
       } else if (s.qr) {
         // LQ / QR-reduced sector: sigma descending from the extraction, the
         // orthonormal factor's vectors are the columns of X (K x K)
@@ -799,7 +834,14 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     for (int si : order) {
       Sec& s = secs[si];
       if (s.bj && s.keep > 0) {
-        for (int k = 0; k < s.keep; ++k) {
+        if (s.qj >= 0) {
+          QjSector& q = qj.sec[s.qj];
+          q.keep = s.keep;
+          q.out = dir > 0 ? s.U : s.Vt;
+          q.es = dir > 0 ? 1 : s.kmin;
+          q.vs = dir > 0 ? s.R : 1;
+        }
+        for (int k = 0; k < s.keep && s.qj < 0; ++k) {
           const double* src = s.colsrc[k];
           if (dir > 0)
             gat.push_back({src, s.U + (int64_t)k * s.R, 1, s.coldiv[k], s.rowsX, 0});
@@ -817,6 +859,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       hoff += s.kmin;
     }
     launch_bj_gather(c, gat);
+    qj_vectors(qj);
     // canonical factor: kept vectors of singular values below 1e-2 sigma_max
     // (extracted vectors are orthogonal to the rest only to about
     // eps sigma_max / sigma, so those above stay within ~1e-14; not in Gram
@@ -836,7 +879,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
         int c0 = s.keep;
         while (c0 > 0 && hs[hoff + c0 - 1] <= szero) --c0;
         int c1 = c0;
-        if (!s.gram)  // Gram eigenvectors need no re-orthonormalisation
+        if (!s.gram && s.qj < 0)  // Gram eigenvectors and Jacobi columns need no re-orthonormalisation
           while (c1 > 1 && hs[hoff + c1 - 1] < ssmall) --c1;
         const int nv = (int)(dir > 0 ? s.R : s.C);
         if (c1 < c0 && c1 >= 1) {

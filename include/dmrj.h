@@ -64,7 +64,8 @@ int dmrj_ctx_sync(dmrj_ctx* ctx);
 int dmrj_version(void);
 /* memory statistics: bytes live, bytes cached, peak bytes */
 int dmrj_ctx_memstats(dmrj_ctx* ctx, int64_t* out3);
-/* Batching of the SVD's batched symmetric eigensolves (backends 0 and 5; no
+/* Batching of the SVD's batched symmetric eigensolves (backend 5, complex
+ * tensors and what backend 0 leaves to them; no
  * counterpart in the reference, whose SVD runs sector by sector): 1 (default)
  * = sectors sorted by size and cut into batches, each padded to its own
  * largest size, where a cost model of the tridiagonalisation (fixed latency
@@ -116,11 +117,12 @@ int dmrj_ctx_graph_stats(dmrj_ctx* ctx, double* out2);
  * counterpart in the reference). */
 int dmrj_ctx_marker(dmrj_ctx* ctx, int id);
 /* SVD backend of dmrj_svd_trunc2 / dmrj_twostep: 0 (default) = batched
- * one-sided Jacobi for sectors with min(R,C) <= 64 and one batched symmetric
- * eigensolve of the augmented matrices [[0,M],[M^T,0]] for the larger ones
- * (a sector at least 1.5 times longer than the side that must come out
- * orthonormal is first reduced by a batched Householder LQ / QR to its K x K
- * triangle, whose augmented matrix has size 2K);
+ * one-sided Jacobi for sectors with min(R,C) <= 64, QR-preconditioned block
+ * Jacobi for the larger ones (both FP64 on the matrix cores); a sector longer
+ * than 2048 on a side, or one that does not converge within the sweep limit,
+ * takes a batched symmetric eigensolve of the augmented matrix [[0,M],[M^T,0]]
+ * (if at least 1.5 times longer than the side that must come out orthonormal,
+ * of its K x K LQ / QR triangle);
  * 1 = rocSOLVER gesdd per sector, 2 = gesvd per sector, 3 = batched Jacobi +
  * gesvd, 4 = batched Jacobi for small sectors + batched block one-sided
  * Jacobi (columns of M or M^T in LDS-resident block pairs) for the larger

@@ -1,0 +1,80 @@
+"""Truncated SVD of single sectors over the sizes its solver treats
+differently: remainders of the 16-column panels, one and several register
+tiles per wave, the tallest sectors of the register-resident kernels and the
+ones above them, wide and tall sectors in both directions."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+EPS = np.finfo(np.float64).eps
+
+
+def _matrix(kind, R, Cc, rng):
+    K = min(R, Cc)
+    if kind == "flat":
+        M = rng.standard_normal((R, Cc))
+    elif kind == "graded":      # both sides graded, as a two-site tensor is
+        M = np.exp(-25.0 * np.arange(R) / R)[:, None] * rng.standard_normal((R, Cc)) * \
+            np.exp(-10.0 * np.arange(Cc) / Cc)[None, :]
+        M = M[rng.permutation(R)][:, rng.permutation(Cc)]
+    elif kind == "equal":       # groups of equal columns and of zero rows
+        M = np.repeat(rng.standard_normal((R, -(-Cc // 8))), 8, axis=1)[:, :Cc]
+        M[rng.permutation(R)[:R // 5]] = 0.0
+    else:                       # isometric: all singular values equal
+        Q = np.linalg.qr(rng.standard_normal((max(R, Cc), K)))[0]
+        M = Q if R >= Cc else Q.T
+    return M / np.linalg.norm(M)
+
+
+SHAPES = [(17, 40), (33, 32), (65, 65), (66, 150), (150, 67), (127, 129), (256, 255), (257, 300), (500, 513),
+          (1024, 80), (70, 1025), (1030, 1027), (2048, 90), (90, 2048), (2049, 72)]
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("kind", ["flat", "graded", "equal", "isometric"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_svd_single_sector(pkg, ctx, shape, kind, direction):
+    R, Cc = shape
+    if max(shape) > 1000 and min(shape) > 1000 and kind != "graded":
+        pytest.skip("one large square case is enough")
+    M = _matrix(kind, R, Cc, np.random.default_rng(R * 7 + Cc))
+    t = pkg.site2_from_dense(ctx, M.reshape(R, 1, 1, Cc))
+    l, r, te, kk = C.c_void_p(), C.c_void_p(), C.c_double(), C.c_int64()
+    sv = np.zeros(4096)
+    ctx.call("dmrj_svd_trunc2", t.h, 0, 2, 0.0, direction, C.byref(l), C.byref(r), C.byref(te), C.byref(kk),
+             pkg._lib.dptr(sv), 4096)
+    L = pkg.DeviceTensor(ctx, l).to_dense()[0].reshape(R, -1)
+    Rt = pkg.DeviceTensor(ctx, r).to_dense()[0].reshape(-1, Cc)
+    n = max(R, Cc)
+    want = np.linalg.svd(M, compute_uv=False)
+    assert kk.value == min(R, Cc)
+    # backward-stable factorisations and orthogonal updates: n eps |M| each
+    assert np.max(np.abs(sv[:kk.value] - want)) <= 2 * n * EPS
+    # (vectors of sigma <= 1e-10 sigma_max are replaced by an orthonormal
+    # completion, which leaves their part of M out)
+    zero = want[want <= 1e-10 * want[0]]
+    assert np.max(np.abs(L @ Rt - M)) <= 8 * n * EPS + np.linalg.norm(zero)
+    # columns are orthogonal to the pair tolerance (1e-14 or 4 eps sqrt(n)) on
+    # top of the rounding of the back-transformation and the completion
+    Q = L if direction > 0 else Rt.T
+    assert np.max(np.abs(Q.T @ Q - np.eye(kk.value))) <= 1e-13 + 4 * n * EPS
+
+
+@pytest.mark.parametrize("scale", [1e-150, 1e-60, 1e60, 1e120])
+def test_svd_scaled(pkg, ctx, scale):
+    """The tensor's norm enters as a power of two only."""
+    M = _matrix("graded", 130, 97, np.random.default_rng(3))
+    sv = []
+    for f in (1.0, scale):
+        t = pkg.site2_from_dense(ctx, (M * f).reshape(130, 1, 1, 97))
+        l, r, te, kk = C.c_void_p(), C.c_void_p(), C.c_double(), C.c_int64()
+        s = np.zeros(128)
+        ctx.call("dmrj_svd_trunc2", t.h, 0, 2, 0.0, 1, C.byref(l), C.byref(r), C.byref(te), C.byref(kk),
+                 pkg._lib.dptr(s), 128)
+        Q = pkg.DeviceTensor(ctx, l).to_dense()[0].reshape(130, -1)
+        assert np.max(np.abs(Q.T @ Q - np.eye(97))) <= 1e-13 + 4 * 130 * EPS
+        sv.append(s[:97])
+    assert np.max(np.abs(sv[0] - sv[1])) <= 2 * 130 * EPS
