@@ -379,20 +379,20 @@ struct CompleteJob {
 // ---- QR-preconditioned block Jacobi for large SVD sectors (svd_qrj.hip) ----
 struct QjJob {
   const double* M;        // R x C, column-major, ld R
-  double* A[4];           // working panels: o x n, n x K, K x K, K x K
-  double* T[3];           // triangular factors of the block reflectors, 256 doubles a panel
-  double* nrm;            // column norms: of A0 (squares, n), then of A3 (16 per panel)
-  int* perm;              // n: column of A0 at every place of the sorted order
+  double* A[3];           // working panels: n x o, o x K, K x K
+  double* T[2];           // triangular factors of the block reflectors, 256 doubles a panel
+  double* nrm;            // column norms: of A0 (squares, o), then of A2 (16 per panel)
+  int* perm;              // o: column of A0 at every place of the sorted order
   int* last;              // last Jacobi round that rotated
-  const int* kcol;        // kept columns of A3, in the order of the vectors
+  const int* kcol;        // kept columns of A2, in the order of the vectors
   const double* kinv;     // their reciprocal norms
   double* out;            // vectors: element i of vector k at out[i es + k vs]
   int64_t es, vs;
   int R, o, n, K, dir, keep;
 };
 struct QjSector {
-  // set by the caller: the sector, and the sizes of A0 (o x n; the wanted
-  // vectors have n elements), K = min(o, n)
+  // set by the caller: the sector, and the sizes of A0 (n x o; the wanted
+  // vectors have n elements), K = min(n, o)
   const double* M = nullptr;
   int R = 0, o = 0, n = 0, K = 0, dir = 0, index = 0;
   // set by qj_solve: singular values descending, their columns, reciprocals

@@ -189,13 +189,18 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   int nsvd = 0;
   const int psvd = c.prof_begin();
   double svd_flops = 0.0;
-  // small sectors: one batched Jacobi launch; large ones: rocSOLVER gesdd
+  // small sectors: one batched Jacobi launch.  With the default backend it
+  // takes sides up to 16, above which the launches of the blocked solver are
+  // the shorter chain: bond step with sectors to 55, 2.43 ms with this kernel
+  // up to 64, 1.01 up to 32, 0.77 up to 16; to 80 (m=80 Hubbard) 2.90, 0.91,
+  // 0.88; to 18 (m=16 Heisenberg) 0.43, 0.45, 0.46.
+  const int small_side = c.svd_backend == 0 ? 16 : 64;
   std::vector<SmallSvdJob> small;
   size_t small_lds = 0;
   std::vector<char> is_small(secs.size(), 0);
   for (int si : order) {
     Sec& s = secs[si];
-    if (z || s.kmin == 0 || s.kmin > 64 || c.svd_backend == 1 || c.svd_backend == 2) continue;
+    if (z || s.kmin == 0 || s.kmin > small_side || c.svd_backend == 1 || c.svd_backend == 2) continue;
     const size_t l = small_svd_lds((int)s.R, (int)s.C);
     if (l > kSmallSvdMaxLds) continue;
     is_small[si] = 1;

@@ -1,19 +1,20 @@
 // Batched SVD of the larger charge sectors: QR-preconditioned block one-sided
 // Jacobi on the FP64 matrix cores.
 //
-// The wanted orthonormal vectors of a sector M (R x C) are the right singular
-// vectors of A0 = M^T (dir > 0: U) or A0 = M (dir < 0: V), an o x n matrix
-// with K = min(o, n).  Three unpivoted Householder factorisations precede the
+// The wanted orthonormal vectors of a sector M (R x C) are the left singular
+// vectors of A0 = M (dir > 0: U) or A0 = M^T (dir < 0: V), an n x o matrix
+// with K = min(n, o).  Two unpivoted Householder factorisations precede the
 // Jacobi sweeps (the preconditioning of Drmac and Veselic, SIAM J. Matrix
 // Anal. Appl. 29 (2008), with a column sort in place of the pivoting):
-//   A0 P = Q1 R1, A1 = R1^T;  A1 = Q2 R2, A2 = R2^T;  A2 = Q3 R3, A3 = R3^T
+//   A0 P = Q0 R0, A1 = R0^T;  A1 = Q1 R1, A2 = R1^T
 // (P orders the columns by decreasing norm).  Two-site tensors are graded on
 // both sides, so every factorisation moves A_i closer to a diagonal matrix:
 // on the 433 x 462 sector of an m=1024 Heisenberg state the sweeps fall from
-// 20 (columns sorted, no factorisation) over 10, 7 to 6, and the error of the
-// singular values from 5e-14 to 4e-16 of the largest.  Jacobi sweeps then
-// rotate the columns of A3 until they are orthogonal, A3 V = W D, and the
-// vectors are P Q2 [W; 0]: neither V nor Q1, Q3 is ever formed.
+// 20 (columns sorted, no factorisation) over 10 to 7, and the error of the
+// singular values from 5e-14 to 1e-15 of the largest.  Jacobi sweeps then
+// rotate the columns of A2 until they are orthogonal, A2 V = W D, so that
+// R1 = V D W^T, A1 = Q1 V D W^T, R0 = W D (Q1 V)^T, and the vectors are
+// Q0 [W; 0]: neither V nor Q1 nor P is needed.
 //
 // Storage: column panels of 16, row-major inside a panel, so that a 16 x 16
 // tile is 256 consecutive doubles and register r of lane l of a wave's tile
@@ -29,12 +30,14 @@
 // work-group: Gram matrix, one inner sweep, product), one for the vectors.
 // All sectors of a bond are in the same launches.
 //
-// What bounds it is latency, not bytes or flops: a bond is about 3 K/16 panel
+// What bounds it is latency, not bytes or flops: a bond is about 2 K/16 panel
 // launches of 20 to 45 us (K the largest sector; 16 dependent columns each)
 // and 7 to 8 sweeps of K/16 rounds of 15 to 45 us.  Bond step at the middle of
 // an m=1024 Heisenberg chain (sectors to 508): 31.0 ms with the batched
 // eigensolve of the augmented matrices, five launches per column of R + C,
-// 7.4 ms with this; m=2048 Hubbard (sectors to 1164): 134 and 30.7 ms.
+// 7.1 ms with this; m=2048 Hubbard (sectors to 1164): 134 and 31 ms.  A third
+// factorisation (of A2) saves a sweep and costs its panels: 7.3 and 30.7 ms, and
+// 1.06 against 0.98 ms at a single 100 x 100 sector.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -270,7 +273,7 @@ __global__ __launch_bounds__(NW * 64) void k_qj_qr(const QjJob* __restrict__ job
   __shared__ double red[NW * 256], wl[256], dots[2 * NW * 16], piv[32], sm[256], taul[16];
   const QrShared sh{red, wl, dots, piv, sm, taul};
   const QjJob& jb = jobs[blockIdx.y];
-  const int rows = which == 0 ? jb.o : which == 1 ? jb.n : jb.K, cols = which == 0 ? jb.n : jb.K;
+  const int rows = which == 0 ? jb.n : jb.o, cols = which == 0 ? jb.o : jb.K;
   const int rb = blocks16(rows), nb = blocks16(cols), np = min(rb, nb);
   const int t = s + 1 + blockIdx.x;
   if (s >= np || t >= nb) return;
@@ -351,28 +354,29 @@ __global__ __launch_bounds__(NW * 64) void k_qj_qr(const QjJob* __restrict__ job
   }
 }
 
-// Squared column norms of A0 (rows of M for dir > 0): 64 columns a group.
+// Squared column norms of A0 (columns of M for dir > 0, rows for dir < 0): 64
+// columns a group.
 __global__ __launch_bounds__(256) void k_qj_norms0(const QjJob* __restrict__ jobs) {
   __shared__ double part[4][64];
   const QjJob& jb = jobs[blockIdx.y];
   const int j0 = blockIdx.x * 64;
-  if (j0 >= jb.n) return;
+  if (j0 >= jb.o) return;
   if (j0 == 0 && threadIdx.x == 0) *jb.last = -1;
   const int w = wave_id(), lane = threadIdx.x & 63;
-  if (jb.dir > 0) {
+  if (jb.dir < 0) {
     double acc = 0.0;
-    if (j0 + lane < jb.n)
-      for (int i = w; i < jb.o; i += 4) {
+    if (j0 + lane < jb.o)
+      for (int i = w; i < jb.n; i += 4) {
         const double v = jb.M[(int64_t)(j0 + lane) + (int64_t)i * jb.R];
         acc += v * v;
       }
     part[w][lane] = acc;
     __syncthreads();
-    if (w == 0 && j0 + lane < jb.n) jb.nrm[j0 + lane] = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
+    if (w == 0 && j0 + lane < jb.o) jb.nrm[j0 + lane] = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
   } else {
-    for (int k = w; k < 64 && j0 + k < jb.n; k += 4) {
+    for (int k = w; k < 64 && j0 + k < jb.o; k += 4) {
       double acc = 0.0;
-      for (int i = lane; i < jb.o; i += 64) {
+      for (int i = lane; i < jb.n; i += 64) {
         const double v = jb.M[(int64_t)i + (int64_t)(j0 + k) * jb.R];
         acc += v * v;
       }
@@ -386,36 +390,36 @@ __global__ __launch_bounds__(256) void k_qj_norms0(const QjJob* __restrict__ job
 __global__ __launch_bounds__(256) void k_qj_rank(const QjJob* __restrict__ jobs) {
   const QjJob& jb = jobs[blockIdx.y];
   const int j = blockIdx.x * 256 + threadIdx.x;
-  if (blockIdx.x * 256 >= jb.n) return;
+  if (blockIdx.x * 256 >= jb.o) return;
   __shared__ double buf[256];
-  const double x = j < jb.n ? jb.nrm[j] : 0.0;
+  const double x = j < jb.o ? jb.nrm[j] : 0.0;
   int rank = 0;
-  for (int k0 = 0; k0 < jb.n; k0 += 256) {
+  for (int k0 = 0; k0 < jb.o; k0 += 256) {
     __syncthreads();
-    if (k0 + threadIdx.x < jb.n) buf[threadIdx.x] = jb.nrm[k0 + threadIdx.x];
+    if (k0 + threadIdx.x < jb.o) buf[threadIdx.x] = jb.nrm[k0 + threadIdx.x];
     __syncthreads();
-    const int kn = min(256, jb.n - k0);
+    const int kn = min(256, jb.o - k0);
     for (int k = 0; k < kn; ++k) rank += buf[k] > x || (buf[k] == x && k0 + k < j);
   }
-  if (j < jb.n) jb.perm[rank] = j;
+  if (j < jb.o) jb.perm[rank] = j;
 }
 
 // Panels of A0: sorted columns, scaled, zero-padded.
 __global__ __launch_bounds__(256) void k_qj_gather(const QjJob* __restrict__ jobs, double scale) {
   const QjJob& jb = jobs[blockIdx.y];
   const int p = blockIdx.x;
-  if (p >= blocks16(jb.n)) return;
-  const int rb = blocks16(jb.o), c = threadIdx.x & 15, rr = threadIdx.x >> 4;
-  const int col = p * 16 + c < jb.n ? jb.perm[p * 16 + c] : -1;
+  if (p >= blocks16(jb.o)) return;
+  const int rb = blocks16(jb.n), c = threadIdx.x & 15, rr = threadIdx.x >> 4;
+  const int col = p * 16 + c < jb.o ? jb.perm[p * 16 + c] : -1;
   double* dst = jb.A[0] + (int64_t)p * rb * 256 + threadIdx.x;
-  const int64_t cs = jb.dir > 0 ? 1 : jb.R, is = jb.dir > 0 ? jb.R : 1;
+  const int64_t cs = jb.dir > 0 ? jb.R : 1, is = jb.dir > 0 ? 1 : jb.R;
   for (int b = blockIdx.z; b < rb; b += gridDim.z) {
     const int i = b * 16 + rr;
-    dst[(int64_t)b * 256] = col >= 0 && i < jb.o ? scale * jb.M[col * cs + i * is] : 0.0;
+    dst[(int64_t)b * 256] = col >= 0 && i < jb.n ? scale * jb.M[col * cs + i * is] : 0.0;
   }
 }
 
-// One Jacobi round on A3: block pair k of the circle schedule per
+// One Jacobi round on A2: block pair k of the circle schedule per
 // work-group.  Gram matrix of the 32 columns on the matrix cores, an
 // approximate eigenbasis V of it in LDS, columns ordered by norm, and the
 // product Y V on the matrix cores.  Pairs whose columns are orthogonal already
@@ -440,8 +444,8 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
     q = t;
   }
   if (q >= npan) return;
-  double* Yp = jb.A[3] + (int64_t)p * rb * 256;
-  double* Yq = jb.A[3] + (int64_t)q * rb * 256;
+  double* Yp = jb.A[2] + (int64_t)p * rb * 256;
+  double* Yq = jb.A[2] + (int64_t)q * rb * 256;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   {
     double4_t pp = {0.0, 0.0, 0.0, 0.0}, pq = pp, qq = pp;
@@ -654,14 +658,14 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
   }
 }
 
-// Column norms of A3: one panel a group, 16 per panel in nrm.
+// Column norms of A2: one panel a group, 16 per panel in nrm.
 __global__ __launch_bounds__(256) void k_qj_norms3(const QjJob* __restrict__ jobs) {
   __shared__ double part[4][16];
   const QjJob& jb = jobs[blockIdx.y];
   const int rb = blocks16(jb.K), p = blockIdx.x;
   if (p >= rb) return;
   const int w = wave_id(), lane = threadIdx.x & 63;
-  const double* P = jb.A[3] + (int64_t)p * rb * 256 + threadIdx.x;
+  const double* P = jb.A[2] + (int64_t)p * rb * 256 + threadIdx.x;
   double acc = 0.0;
   for (int b = 0; b < rb; ++b) acc += P[(int64_t)b * 256] * P[(int64_t)b * 256];
   acc = sum_rows(acc);
@@ -672,9 +676,9 @@ __global__ __launch_bounds__(256) void k_qj_norms3(const QjJob* __restrict__ job
         sqrt(part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x]);
 }
 
-// The kept vectors: 16 normalised columns of A3 a group, the block
-// reflectors of the second factorisation applied to them from the last to the
-// first in registers, rows put back in the unsorted order.
+// The kept vectors: 16 normalised columns of A2 a group, the block
+// reflectors of the first factorisation applied to them from the last to the
+// first in registers.
 template <int NW, int TPW>
 __global__ __launch_bounds__(NW * 64) void k_qj_back(const QjJob* __restrict__ jobs) {
   __shared__ double red[NW * 256], wl[256];
@@ -687,7 +691,7 @@ __global__ __launch_bounds__(NW * 64) void k_qj_back(const QjJob* __restrict__ j
   const int k = k0 + c;
   const int src = k < jb.keep ? jb.kcol[k] : -1;
   const double inv = k < jb.keep ? jb.kinv[k] : 0.0;
-  const double* S = jb.A[3] + (int64_t)(max(src, 0) >> 4) * kb * 256 + (max(src, 0) & 15);
+  const double* S = jb.A[2] + (int64_t)(max(src, 0) >> 4) * kb * 256 + (max(src, 0) & 15);
   double4_t a[TPW];
 #pragma unroll
   for (int i = 0; i < TPW; ++i) {
@@ -697,8 +701,8 @@ __global__ __launch_bounds__(NW * 64) void k_qj_back(const QjJob* __restrict__ j
   }
   const int m = 4 * (c & 3) + (c >> 2);
   for (int s = kb - 1; s >= 0; --s) {
-    const double* V = jb.A[1] + (int64_t)s * rb * 256;
-    const double* T = jb.T[1] + (int64_t)s * 256;
+    const double* V = jb.A[0] + (int64_t)s * rb * 256;
+    const double* T = jb.T[0] + (int64_t)s * 256;
     // row blocks above s do not take part: their V is not stored
     double4_t acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -740,7 +744,7 @@ __global__ __launch_bounds__(NW * 64) void k_qj_back(const QjJob* __restrict__ j
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = 16 * (w + NW * i) + 4 * r + g;
-      if (row < jb.n) jb.out[jb.perm[row] * jb.es + k * jb.vs] = a[i][r];
+      if (row < jb.n) jb.out[row * jb.es + k * jb.vs] = a[i][r];
     }
 }
 
@@ -795,7 +799,7 @@ bool qj_solve(QjBatch& q, double norm2) {
   std::vector<QjSector>& sec = q.sec;
   const int nj = (int)sec.size();
   // largest first: a launch's grid covers the jobs that still take part
-  std::stable_sort(sec.begin(), sec.end(), [](const QjSector& a, const QjSector& b) { return a.n > b.n; });
+  std::stable_sort(sec.begin(), sec.end(), [](const QjSector& a, const QjSector& b) { return a.o > b.o; });
   // powers of two, exact: norms of order one whatever the tensor's scale
   int ex = 0;
   (void)std::frexp(std::sqrt(norm2), &ex);
@@ -808,11 +812,11 @@ bool qj_solve(QjBatch& q, double norm2) {
   for (int j = 0; j < nj; ++j) {
     const int64_t o = up16(sec[j].o), n = up16(sec[j].n), K = up16(sec[j].K), Kc = kcols(sec[j].K);
     nof[j] = nn;
-    nn += std::max(n, K);
+    nn += o;
     dof[j] = nd;
-    nd += o * n + n * Kc + 2 * K * Kc + 3 * 16 * n;
+    nd += n * o + o * Kc + K * Kc + 2 * 16 * K;
     iof[j] = ni;
-    ni += n;
+    ni += o;
   }
   q.work = (double*)c.alloc.alloc((nn + nd) * sizeof(double));
   q.ints = (int*)c.alloc.alloc(ni * sizeof(int));
@@ -826,12 +830,10 @@ bool qj_solve(QjBatch& q, double norm2) {
     b = QjJob{};
     b.M = s.M;
     b.A[0] = q.work + nn + dof[j];
-    b.A[1] = b.A[0] + o * n;
-    b.A[2] = b.A[1] + n * Kc;
-    b.A[3] = b.A[2] + K * Kc;
-    b.T[0] = b.A[3] + K * Kc;
-    b.T[1] = b.T[0] + 16 * n;
-    b.T[2] = b.T[1] + 16 * n;
+    b.A[1] = b.A[0] + n * o;
+    b.A[2] = b.A[1] + o * Kc;
+    b.T[0] = b.A[2] + K * Kc;
+    b.T[1] = b.T[0] + 16 * K;
     b.nrm = q.work + nof[j];
     b.perm = q.ints + iof[j];
     b.last = q.ints + j;
@@ -845,18 +847,19 @@ bool qj_solve(QjBatch& q, double norm2) {
     maxK = std::max(maxK, s.K);
   }
   auto* dj = (QjJob*)c.upload(q.jobs.data(), nj * sizeof(QjJob));
-  const int pn = up16(maxn) / 16, pk = up16(maxK) / 16;
-  hipLaunchKernelGGL(k_qj_norms0, dim3((maxn + 63) / 64, nj), dim3(256), 0, c.stream, dj);
-  hipLaunchKernelGGL(k_qj_rank, dim3((maxn + 255) / 256, nj), dim3(256), 0, c.stream, dj);
-  hipLaunchKernelGGL(k_qj_gather, dim3(pn, nj, std::min(16, up16(maxo) / 16)), dim3(256), 0, c.stream, dj, scale);
-  for (int which = 0; which < 3; ++which) {
-    const int rows = which == 0 ? maxo : which == 1 ? maxn : maxK;
+  const int pk = up16(maxK) / 16;
+  hipLaunchKernelGGL(k_qj_norms0, dim3((maxo + 63) / 64, nj), dim3(256), 0, c.stream, dj);
+  hipLaunchKernelGGL(k_qj_rank, dim3((maxo + 255) / 256, nj), dim3(256), 0, c.stream, dj);
+  hipLaunchKernelGGL(k_qj_gather, dim3(up16(maxo) / 16, nj, std::min(16, up16(maxn) / 16)), dim3(256), 0, c.stream,
+                     dj, scale);
+  for (int which = 0; which < 2; ++which) {
+    const int rows = which == 0 ? maxn : maxo;
     // slabs and panels of every job in this factorisation
     std::vector<int> slabs(nj), pans(nj);
     int np = 0;
     for (int j = 0; j < nj; ++j) {
-      slabs[j] = up16(which == 0 ? sec[j].n : sec[j].K) / 16;
-      pans[j] = std::min(up16(which == 0 ? sec[j].o : which == 1 ? sec[j].n : sec[j].K) / 16, slabs[j]);
+      slabs[j] = up16(which == 0 ? sec[j].o : sec[j].K) / 16;
+      pans[j] = std::min(up16(which == 0 ? sec[j].n : sec[j].o) / 16, slabs[j]);
       np = std::max(np, pans[j]);
     }
     for (int s = -1; s < np; ++s) {
@@ -874,7 +877,7 @@ bool qj_solve(QjBatch& q, double norm2) {
   // comes to the host after every half cycle of the largest while the next
   // half cycle is already queued
   const int nbmax = (std::max(2, pk) + 1) & ~1;
-  const int chunk = std::max(4, nbmax / 2);
+  const int chunk = nbmax / 2;
   const double tol = std::max(1e-14, 4.0 * 2.220446049250313e-16 * std::sqrt((double)maxK));
   const double fl = 1e-11;  // relative to |AA|, which the scaling puts in [1/2, 1)
   constexpr int kMaxSweeps = 40;
@@ -885,7 +888,7 @@ bool qj_solve(QjBatch& q, double norm2) {
     for (int k = 0; k < chunk; ++k, ++step)
       hipLaunchKernelGGL(k_qj_round, dim3(nbmax / 2, nj), dim3(512), 0, c.stream, dj, step, tol * tol, fl * fl);
   };
-  for (int k = 0; k < 5; ++k) rounds();
+  for (int k = 0; k < 10 && step < 5 * (nbmax - 1); ++k) rounds();  // five sweeps are always needed
   while (!done && step < kMaxSweeps * (nbmax - 1)) {
     const int upto = step;
     HIP_OK(hipMemcpyAsync(hlast, q.ints, nj * sizeof(int), hipMemcpyDeviceToHost, c.stream));

@@ -117,8 +117,8 @@ int dmrj_ctx_graph_stats(dmrj_ctx* ctx, double* out2);
  * counterpart in the reference). */
 int dmrj_ctx_marker(dmrj_ctx* ctx, int id);
 /* SVD backend of dmrj_svd_trunc2 / dmrj_twostep: 0 (default) = batched
- * one-sided Jacobi for sectors with min(R,C) <= 64, QR-preconditioned block
- * Jacobi for the larger ones (both FP64 on the matrix cores); a sector longer
+ * one-sided Jacobi for sectors with min(R,C) <= 16, QR-preconditioned block
+ * Jacobi for the larger ones (FP64 on the matrix cores); a sector longer
  * than 2048 on a side, or one that does not converge within the sweep limit,
  * takes a batched symmetric eigensolve of the augmented matrix [[0,M],[M^T,0]]
  * (if at least 1.5 times longer than the side that must come out orthonormal,

@@ -29,7 +29,7 @@ def _matrix(kind, R, Cc, rng):
     return M / np.linalg.norm(M)
 
 
-SHAPES = [(17, 40), (33, 32), (65, 65), (66, 150), (150, 67), (127, 129), (256, 255), (257, 300), (500, 513),
+SHAPES = [(16, 20), (20, 17), (17, 40), (33, 32), (65, 65), (66, 150), (150, 67), (127, 129), (256, 255), (257, 300), (500, 513),
           (1024, 80), (70, 1025), (1030, 1027), (2048, 90), (90, 2048), (2049, 72)]
 
 
