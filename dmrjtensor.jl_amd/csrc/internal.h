@@ -379,6 +379,7 @@ struct CompleteJob {
 // ---- QR-preconditioned block Jacobi for large SVD sectors (svd_qrj.hip) ----
 struct QjJob {
   const double* M;        // R x C, column-major, ld R
+  int64_t plane;          // distance of its imaginary plane (0 for real tensors)
   double* A[3];           // working panels: n x o, o x K, K x K
   double* T[2];           // triangular factors of the block reflectors, 256 doubles a panel
   double* nrm;            // column norms: of A0 (squares, o), then of A2 (16 per panel)
@@ -387,7 +388,7 @@ struct QjJob {
   const int* kcol;        // kept columns of A2, in the order of the vectors
   const double* kinv;     // their reciprocal norms
   double* out;            // vectors: element i of vector k at out[i es + k vs]
-  int64_t es, vs;
+  int64_t es, vs, oplane;  // (imaginary parts oplane further)
   int R, o, n, K, dir, keep;
 };
 struct QjSector {
@@ -401,7 +402,7 @@ struct QjSector {
   // set by the caller before qj_vectors
   int keep = 0;
   double* out = nullptr;
-  int64_t es = 0, vs = 0;
+  int64_t es = 0, vs = 0, oplane = 0;
 };
 struct QjBatch {
   Context& c;
@@ -409,12 +410,13 @@ struct QjBatch {
   std::vector<QjJob> jobs;
   double* work = nullptr;
   int* ints = nullptr;
-  explicit QjBatch(Context& c_) : c(c_) {}
+  const bool cplx;
+  QjBatch(Context& c_, bool cplx_) : c(c_), cplx(cplx_) {}
   QjBatch(const QjBatch&) = delete;
   QjBatch& operator=(const QjBatch&) = delete;
   ~QjBatch();
 };
-bool qj_fits(int64_t R, int64_t C);  // sector sizes the register-resident kernels take
+bool qj_fits(int64_t R, int64_t C, bool cplx);  // sector sizes the register-resident kernels take
 bool qj_solve(QjBatch& q, double norm2);
 void qj_vectors(QjBatch& q);
 

@@ -331,17 +331,17 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       }
     }
   }
-  // large sectors, default backend: QR-preconditioned block Jacobi
+  // large sectors of the default backend and all complex ones: QR-preconditioned block Jacobi
   // (svd_qrj.hip) for the vectors of the side that must come out orthonormal;
   // the other factor by the grouped GEMM below.  Sectors it does not take
   // (longer than its register-resident slabs, or not converged within its
   // sweep limit) and tensors whose squared norm under- or overflows go to the
   // eigensolves of the augmented matrices.
-  QjBatch qj(c);
-  if (!z && c.svd_backend == 0 && aa2 > 1e-305 && aa2 < 1e305) {
+  QjBatch qj(c, z);
+  if ((z || c.svd_backend == 0) && aa2 > 1e-305 && aa2 < 1e305) {
     for (int si : order) {
       Sec& s = secs[si];
-      if (s.kmin == 0 || is_small[si] || !qj_fits(s.R, s.C)) continue;
+      if (s.kmin == 0 || is_small[si] || !qj_fits(s.R, s.C, z)) continue;
       QjSector q;
       q.M = s.M;
       q.R = (int)s.R;
@@ -451,12 +451,12 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   rocblas_int* qinfo = nullptr;
   int nqr = 0;
   if (z) {
-    // complex: every sector through batched Hermitian eigensolves of
-    // [[0, M], [M^H, 0]] (eigenvalues +-sigma), batched by size (eig_classes)
+    // complex, what the block Jacobi has left: batched Hermitian eigensolves
+    // of [[0, M], [M^H, 0]] (eigenvalues +-sigma), batched by size (eig_classes)
     std::vector<int> big;
     for (int si : order) {
       Sec& s = secs[si];
-      if (s.kmin == 0) continue;
+      if (s.kmin == 0 || is_small[si]) continue;
       big.push_back(si);
     }
     if (!big.empty()) {
@@ -832,6 +832,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   {
     // block-Jacobi sectors: normalised kept columns, then the other factor
     // U^T M = D V^T (dir > 0) or M V = U D (dir < 0) in one grouped GEMM
+    BufMap planes;  // complex: the operands of those products
     std::vector<BjGather> gat;
     std::vector<GemmTask> tasks;
     std::vector<GemmSeg> segs;
@@ -845,6 +846,12 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
           q.out = dir > 0 ? s.U : s.Vt;
           q.es = dir > 0 ? 1 : s.kmin;
           q.vs = dir > 0 ? s.R : 1;
+          q.oplane = s.kmin * (dir > 0 ? s.R : s.C);
+          if (z) {
+            planes.add(s.M, s.R * s.C, true);
+            planes.add(s.U, s.R * s.kmin, true);
+            planes.add(s.Vt, s.kmin * s.C, true);
+          }
         }
         for (int k = 0; k < s.keep && s.qj < 0; ++k) {
           const double* src = s.colsrc[k];
@@ -855,10 +862,10 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
         }
         if (dir > 0) {
           tasks.push_back({s.Vt, s.kmin, s.keep, (int)s.C, (int)segs.size(), 1, 0.0});
-          segs.push_back({s.U, s.M, s.R, s.R, (int)s.R, 1, 1.0});
+          segs.push_back({s.U, s.M, s.R, s.R, (int)s.R, 1 | (z ? kSegConjA : 0), 1.0});
         } else {
           tasks.push_back({s.U, s.R, (int)s.R, s.keep, (int)segs.size(), 1, 0.0});
-          segs.push_back({s.M, s.Vt, s.R, s.kmin, (int)s.C, 2, 1.0});
+          segs.push_back({s.M, s.Vt, s.R, s.kmin, (int)s.C, 2 | (z ? kSegConjB : 0), 1.0});
         }
       }
       hoff += s.kmin;
@@ -906,6 +913,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       reorth_basis(c, rj);
       complete_basis(c, cj);
     }
+    if (z) complexify_gemm(tasks, segs, planes);
     launch_gemm(c, tasks, segs, -1);
   }
   double* dscal = (double*)c.alloc.alloc(std::max<size_t>(1, scal.size()) * sizeof(double));
@@ -942,7 +950,8 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
                        dir < 0 ? dscal + soff[qidx[Q]] : nullptr, 1.0});
     if (z)
       split.push_back({s.U + s.R * s.kmin + ro, tl->data + tl->site.size + b.off, s.R, S.dim[b.a], S.dim[b.a],
-                       s.keep, nullptr, dir < 0 ? dscal + soff[qidx[Q]] : nullptr, 1.0});
+                       s.keep, nullptr, dir < 0 && !s.bj ? dscal + soff[qidx[Q]] : nullptr,
+                       dir < 0 && s.bj ? renorm : 1.0});
   }
   for (const SiteBlock& b : tr->site.blocks) {
     const Charge Q = mid.q[b.a];
@@ -958,7 +967,8 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
                        dir > 0 ? dscal + soff[qidx[Q]] : nullptr, nullptr, 1.0});
     if (z)
       split.push_back({s.Vt + (int64_t)s.kmin * s.C + co * s.kmin, tr->data + tr->site.size + b.off, s.kmin, s.keep,
-                       s.keep, T.dim[b.b], dir > 0 ? dscal + soff[qidx[Q]] : nullptr, nullptr, 1.0});
+                       s.keep, T.dim[b.b], dir > 0 && !s.bj ? dscal + soff[qidx[Q]] : nullptr, nullptr,
+                       dir > 0 && s.bj ? renorm : 1.0});
   }
   launch_copy(c, split);
   for (auto& s : secs) {

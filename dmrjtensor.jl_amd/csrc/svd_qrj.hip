@@ -6,14 +6,14 @@
 // with K = min(n, o).  Two unpivoted Householder factorisations precede the
 // Jacobi sweeps (the preconditioning of Drmac and Veselic, SIAM J. Matrix
 // Anal. Appl. 29 (2008), with a column sort in place of the pivoting):
-//   A0 P = Q0 R0, A1 = R0^T;  A1 = Q1 R1, A2 = R1^T
+//   A0 P = Q0 R0, A1 = R0^H;  A1 = Q1 R1, A2 = R1^H
 // (P orders the columns by decreasing norm).  Two-site tensors are graded on
 // both sides, so every factorisation moves A_i closer to a diagonal matrix:
 // on the 433 x 462 sector of an m=1024 Heisenberg state the sweeps fall from
 // 20 (columns sorted, no factorisation) over 10 to 7, and the error of the
 // singular values from 5e-14 to 1e-15 of the largest.  Jacobi sweeps then
 // rotate the columns of A2 until they are orthogonal, A2 V = W D, so that
-// R1 = V D W^T, A1 = Q1 V D W^T, R0 = W D (Q1 V)^T, and the vectors are
+// R1 = V D W^H, A1 = Q1 V D W^H, R0 = W D (Q1 V)^H, and the vectors are
 // Q0 [W; 0]: neither V nor Q1 nor P is needed.
 //
 // Storage: column panels of 16, row-major inside a panel, so that a 16 x 16
@@ -114,153 +114,251 @@ __device__ __forceinline__ int blocks16(int n) { return (n + 15) >> 4; }
 
 constexpr int kGroup = 2;  // register tiles whose loads are in flight together
 
+// Complex tensors (Z) hold every tile as a real and an imaginary 16 x 16
+// plane, 512 doubles; their products are real products of the planes.
+template <bool Z>
+constexpr int kTile = Z ? 512 : 256;
+template <bool Z>
+struct Tile {  // a wave's registers of one tile (i: complex only)
+  double4_t r, i;
+};
+constexpr double4_t kZero4 = {0.0, 0.0, 0.0, 0.0};
+
+// acc += conj(a) b, acc += a b and acc -= a b, one MFMA step
+template <bool Z>
+__device__ __forceinline__ void mac_h(Tile<Z>& acc, double ar, double ai, double br, double bi) {
+  acc.r = mfma(ar, br, acc.r);
+  if constexpr (Z) {
+    acc.r = mfma(ai, bi, acc.r);
+    acc.i = mfma(ar, bi, acc.i);
+    acc.i = mfma(-ai, br, acc.i);
+  }
+}
+template <bool Z>
+__device__ __forceinline__ void mac(Tile<Z>& acc, double ar, double ai, double br, double bi) {
+  acc.r = mfma(ar, br, acc.r);
+  if constexpr (Z) {
+    acc.r = mfma(-ai, bi, acc.r);
+    acc.i = mfma(ar, bi, acc.i);
+    acc.i = mfma(ai, br, acc.i);
+  }
+}
+
 struct QrShared {
-  double* red;   // NW x 256 partial tiles
-  double* w;     // 256
-  double* dots;  // 2 x NW x 16
-  double* piv;   // 2 x 16
-  double* s;     // 256: V^T V above the diagonal
-  double* tau;   // 16
+  double* red;   // NW partial tiles
+  double* w;     // a tile
+  double* dots;  // 2 x NW x 16 (x 2 complex)
+  double* piv;   // 2 x 16 (x 2)
+  double* s;     // 256 (x 2): V^H V above the diagonal
+  double* tau;   // 16 (x 2)
 };
 
-// W = V^T A over the register tiles of the work-group's slab (tiles of
-// row blocks base + w + NW i), summed over the waves; every lane returns its
-// elements in the B operand layout.
-template <int NW, int TPW>
-__device__ __forceinline__ double4_t slab_vta(const double* V, int base, int rb, const double4_t (&a)[TPW],
-                                              const QrShared& sh) {
+// W = V^H A over the register tiles of the work-group's slab (tiles of row
+// blocks base + w + NW i, those from `first` on), summed over the waves; every
+// lane returns its elements in the B operand layout.
+template <bool Z, int NW, int TPW>
+__device__ __forceinline__ Tile<Z> slab_vha(const double* V, int base, int first, int rb, const Tile<Z> (&a)[TPW],
+                                            const QrShared& sh) {
   const int w = wave_id(), lane = threadIdx.x & 63;
-  double4_t acc = {0.0, 0.0, 0.0, 0.0};
-  // groups of tiles: the loads of a group are in flight together; tiles past
-  // the end are zero, so any tile of V will do for them
+  Tile<Z> acc = {kZero4, kZero4};
+  // groups of tiles: the loads of a group are in flight together; tiles that
+  // take no part are zeroed, so any tile of V will do for them
 #pragma unroll
   for (int i0 = 0; i0 < TPW; i0 += kGroup)
-    if (base + w + NW * i0 < rb) {
+    if (base + w + NW * i0 < rb && base + w + NW * (i0 + kGroup - 1) >= first) {
 #pragma unroll
       for (int i = i0; i < i0 + kGroup; ++i) {
-        const double* v = V + (int64_t)min(base + w + NW * i, rb - 1) * 256 + lane;
+        const int b = base + w + NW * i;
+        const double z = b >= first ? 1.0 : 0.0;  // (tiles past the end hold zeros)
+        const double* v = V + (int64_t)min(max(b, first), rb - 1) * kTile<Z> + lane;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc = mfma(v[64 * r], a[i][r], acc);
+        for (int r = 0; r < 4; ++r) mac_h<Z>(acc, z * v[64 * r], Z ? z * v[256 + 64 * r] : 0.0, a[i].r[r], Z ? a[i].i[r] : 0.0);
       }
     }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) sh.red[w * 256 + 64 * r + lane] = acc[r];
+  for (int r = 0; r < 4; ++r) {
+    sh.red[w * kTile<Z> + 64 * r + lane] = acc.r[r];
+    if constexpr (Z) sh.red[w * kTile<Z> + 256 + 64 * r + lane] = acc.i[r];
+  }
   __syncthreads();
-  if (threadIdx.x < 256) {
+  if (threadIdx.x < kTile<Z>) {
     double t = 0.0;
 #pragma unroll
-    for (int k = 0; k < NW; ++k) t += sh.red[k * 256 + threadIdx.x];
+    for (int k = 0; k < NW; ++k) t += sh.red[k * kTile<Z> + threadIdx.x];
     sh.w[threadIdx.x] = t;
   }
   __syncthreads();
-  double4_t r;
+  Tile<Z> r = {kZero4, kZero4};
 #pragma unroll
-  for (int k = 0; k < 4; ++k) r[k] = sh.w[64 * k + lane];
+  for (int k = 0; k < 4; ++k) {
+    r.r[k] = sh.w[64 * k + lane];
+    if constexpr (Z) r.i[k] = sh.w[256 + 64 * k + lane];
+  }
   return r;
 }
 
 // A -= V Y on the register tiles; Y's register s holds row 4 (l/16) + s of
 // column l%16, the reduction index order of V's four consecutive elements.
-template <int NW, int TPW>
-__device__ __forceinline__ void slab_sub(const double* V, int base, int rb, double4_t (&a)[TPW], double4_t Y) {
+template <bool Z, int NW, int TPW>
+__device__ __forceinline__ void slab_sub(const double* V, int base, int first, int rb, Tile<Z> (&a)[TPW],
+                                         const Tile<Z>& Y) {
   const int w = wave_id(), lane = threadIdx.x & 63;
 #pragma unroll
   for (int i0 = 0; i0 < TPW; i0 += kGroup)
-    if (base + w + NW * i0 < rb) {
+    if (base + w + NW * i0 < rb && base + w + NW * (i0 + kGroup - 1) >= first) {
 #pragma unroll
       for (int i = i0; i < i0 + kGroup; ++i) {
         const int b = base + w + NW * i;
-        const double z = b < rb ? -1.0 : 0.0;  // tiles past the end stay zero
-        const double2_t* v =
-            (const double2_t*)(V + (int64_t)min(b, rb - 1) * 256 + (lane & 15) * 16 + 4 * (lane >> 4));
+        const double z = b >= first && b < rb ? -1.0 : 0.0;  // other tiles stay as they are
+        const double2_t* v = (const double2_t*)(V + (int64_t)min(max(b, first), rb - 1) * kTile<Z> +
+                                                (lane & 15) * 16 + 4 * (lane >> 4));
         const double2_t v0 = v[0], v1 = v[1];
-        a[i] = mfma(z * v0[0], Y[0], a[i]);
-        a[i] = mfma(z * v0[1], Y[1], a[i]);
-        a[i] = mfma(z * v1[0], Y[2], a[i]);
-        a[i] = mfma(z * v1[1], Y[3], a[i]);
+        double2_t u0 = {0.0, 0.0}, u1 = u0;
+        if constexpr (Z) {
+          u0 = v[128];
+          u1 = v[129];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          mac<Z>(a[i], z * (k < 2 ? v0[k & 1] : v1[k & 1]), z * (k < 2 ? u0[k & 1] : u1[k & 1]), Y.r[k],
+                 Z ? Y.i[k] : 0.0);
       }
     }
 }
 
 // One column of a panel: Householder reflector of column J (pivot in row J of
-// the pivot tile, tile 0 of wave pw) and its application to the columns
-// right of it.  One reduction gives the products of column J with all 16
-// columns: the norm, the update coefficients and the inner products of the
+// the pivot tile, tile 0 of the wave with `top`) and its application to the
+// columns right of it.  One reduction gives the products of column J with all
+// 16 columns: the norm, the update coefficients and the inner products of the
 // reflectors that the triangular factor needs.
-template <int J, int NW, int TPW>
-__device__ __forceinline__ void panel_column(double4_t (&a)[TPW], int nt, bool top, const QrShared& sh) {
+template <bool Z, int J, int NW, int TPW>
+__device__ __forceinline__ void panel_column(Tile<Z> (&a)[TPW], int nt, bool top, const QrShared& sh) {
+  constexpr int kP = Z ? 2 : 1;
   const int w = wave_id(), lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  double4_t dots = {0.0, 0.0, 0.0, 0.0};
+  double4_t dr = kZero4, di = kZero4;
 #pragma unroll
   for (int i = 0; i < TPW; ++i)
     if (i < nt) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const double x = row_bcast<J>(a[i][r]);
-        const double y = (i == 0 && top && 4 * r + g <= J) ? 0.0 : a[i][r];
-        dots[r] = fma(x, y, dots[r]);
+        const bool out = i == 0 && top && 4 * r + g <= J;
+        const double x = row_bcast<J>(a[i].r[r]);
+        const double y = out ? 0.0 : a[i].r[r];
+        dr[r] = fma(x, y, dr[r]);
+        if constexpr (Z) {
+          const double xi = row_bcast<J>(a[i].i[r]);
+          const double yi = out ? 0.0 : a[i].i[r];
+          dr[r] = fma(xi, yi, dr[r]);
+          di[r] = fma(x, yi, di[r]);
+          di[r] = fma(-xi, y, di[r]);
+        }
       }
     }
-  const double dot = sum_rows((dots[0] + dots[1]) + (dots[2] + dots[3]));
-  double* d = sh.dots + (J & 1) * NW * 16;
-  double* pv = sh.piv + (J & 1) * 16;
+  double* d = sh.dots + (J & 1) * NW * 16 * kP;
+  double* pv = sh.piv + (J & 1) * 16 * kP;
+  const double dot = sum_rows((dr[0] + dr[1]) + (dr[2] + dr[3]));
   if (g == 0) d[w * 16 + c] = dot;
-  if (top && g == (J & 3)) pv[c] = a[0][J >> 2];
+  if (top && g == (J & 3)) pv[c] = a[0].r[J >> 2];
+  if constexpr (Z) {
+    const double dotz = sum_rows((di[0] + di[1]) + (di[2] + di[3]));
+    if (g == 0) d[NW * 16 + w * 16 + c] = dotz;
+    if (top && g == (J & 3)) pv[16 + c] = a[0].i[J >> 2];
+  }
   __syncthreads();
-  double part[4] = {0.0, 0.0, 0.0, 0.0};
+  double part[4] = {0.0, 0.0, 0.0, 0.0}, partz[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int k = 0; k < NW; ++k) part[k & 3] += d[k * 16 + c];
+  for (int k = 0; k < NW; ++k) {
+    part[k & 3] += d[k * 16 + c];
+    if constexpr (Z) partz[k & 3] += d[NW * 16 + k * 16 + c];
+  }
   const double tot = (part[0] + part[1]) + (part[2] + part[3]);
-  const double pr = pv[c];
+  const double totz = (partz[0] + partz[1]) + (partz[2] + partz[3]);
+  const double pr = pv[c], prz = Z ? pv[16 + c] : 0.0;
   const double xn = row_bcast<J>(tot), alpha = row_bcast<J>(pr);
-  double tau = 0.0, beta = alpha, scale = 0.0;
-  if (xn > 0.0) {
-    const double h = fma(alpha, alpha, xn);
+  const double alphaz = Z ? row_bcast<J>(prz) : 0.0;
+  double tau = 0.0, tauz = 0.0, beta = alpha, scale = 0.0, scalez = 0.0;
+  const double xa = Z ? fma(alphaz, alphaz, xn) : xn;
+  if (xa > 0.0) {
+    const double h = fma(alpha, alpha, xa);
     const double ri = copysign(fast_rsqrt(h), -alpha);  // 1 / beta
     beta = h * ri;
     tau = fma(-alpha, ri, 1.0);
-    scale = fast_rcp(alpha - beta);
+    if constexpr (Z) {
+      tauz = -alphaz * ri;
+      const double u = alpha - beta, q = fast_rcp(fma(u, u, alphaz * alphaz));
+      scale = u * q;
+      scalez = -alphaz * q;
+    } else {
+      scale = fast_rcp(alpha - beta);
+    }
   }
-  const double vc = fma(scale, tot, pr);   // v_J . column c (c < J: the column is v_c)
-  const double wc = c > J ? tau * vc : 0.0;
+  // v_J^H column c (c < J: the column is v_c), and conj(tau) of it right of J
+  double vc = fma(scale, tot, pr), vcz = 0.0;
+  if constexpr (Z) {
+    vc = fma(scalez, totz, vc);
+    vcz = prz + scale * totz - scalez * tot;
+  }
+  double wc = tau * vc, wcz = 0.0;
+  if constexpr (Z) {
+    wc = fma(tauz, vcz, wc);
+    wcz = tau * vcz - tauz * vc;
+  }
+  wc = c > J ? wc : 0.0;
+  wcz = c > J ? wcz : 0.0;
   if (w == 0 && g == 0) {
     if (c < J) sh.s[c * 16 + J] = vc;
     if (c == J) sh.tau[J] = tau;
+    if constexpr (Z) {
+      if (c < J) sh.s[256 + c * 16 + J] = -vcz;
+      if (c == J) sh.tau[16 + J] = tauz;
+    }
   }
   // column J becomes the reflector, x + (scale - 1) x, the columns right of it
   // lose w_c scale x: one multiply-add with a coefficient per column.  The
   // broadcasts of the first pass are made again: held across the barrier they
   // would take as many registers as the tiles.
-  const double coef = c == J ? scale - 1.0 : -wc * scale;
+  const double coef = c == J ? scale - 1.0 : -(wc * scale - (Z ? wcz * scalez : 0.0));
+  const double coefz = Z ? (c == J ? scalez : -(wc * scalez + wcz * scale)) : 0.0;
 #pragma unroll
   for (int i = 0; i < TPW; ++i)
     if (i < nt) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        double x = a[i][r];
+        const int row = 4 * r + g;
+        double x = a[i].r[r];
         asm volatile("" : "+v"(x));
-        const double y = fma(coef, row_bcast<J>(x), x);
-        if (i == 0 && top) {
-          const int row = 4 * r + g;
-          a[i][r] = row > J ? y : row == J ? (c == J ? beta : x - wc) : x;
-        } else {
-          a[i][r] = y;
+        const double xj = row_bcast<J>(x);
+        double y = fma(coef, xj, x);
+        if constexpr (Z) {
+          double z = a[i].i[r];
+          asm volatile("" : "+v"(z));
+          const double zj = row_bcast<J>(z);
+          y = fma(-coefz, zj, y);
+          const double yz = fma(coefz, xj, fma(coef, zj, z));
+          if (i == 0 && top)
+            a[i].i[r] = row > J ? yz : row == J ? (c == J ? 0.0 : z - wcz) : z;
+          else
+            a[i].i[r] = yz;
         }
+        if (i == 0 && top)
+          a[i].r[r] = row > J ? y : row == J ? (c == J ? beta : x - wc) : x;
+        else
+          a[i].r[r] = y;
       }
     }
 }
 
-template <int J, int NW, int TPW>
-__device__ __forceinline__ void panel_columns(double4_t (&a)[TPW], int nt, bool top, const QrShared& sh) {
+template <bool Z, int J, int NW, int TPW>
+__device__ __forceinline__ void panel_columns(Tile<Z> (&a)[TPW], int nt, bool top, const QrShared& sh) {
   if constexpr (J < 16) {
-    panel_column<J, NW, TPW>(a, nt, top, sh);
-    panel_columns<J + 1, NW, TPW>(a, nt, top, sh);
+    panel_column<Z, J, NW, TPW>(a, nt, top, sh);
+    panel_columns<Z, J + 1, NW, TPW>(a, nt, top, sh);
   }
 }
 
 }  // namespace
 
-// One step of factorisation `which` (A[which] = Q R, A[which + 1] = R^T): the
+// One step of factorisation `which` (A[which] = Q R, A[which + 1] = R^H): the
 // block reflector of panel s applied to the slabs right of it, and panel
 // s + 1 factorised by its slab's group.  s = -1 factorises panel 0.
 //
@@ -268,9 +366,10 @@ __device__ __forceinline__ void panel_columns(double4_t (&a)[TPW], int nt, bool 
 // of 16): read once, written once, V read from L2 twice (once per operand
 // layout).  The step's length is that of the group that goes on to the
 // panel: 16 columns of one reduction and one barrier each.
-template <int NW, int TPW>
+template <bool Z, int NW, int TPW>
 __global__ __launch_bounds__(NW * 64) void k_qj_qr(const QjJob* __restrict__ jobs, int which, int s) {
-  __shared__ double red[NW * 256], wl[256], dots[2 * NW * 16], piv[32], sm[256], taul[16];
+  constexpr int kT = kTile<Z>, kP = Z ? 2 : 1;
+  __shared__ double red[NW * kT], wl[kT], dots[2 * NW * 16 * kP], piv[32 * kP], sm[256 * kP], taul[16 * kP];
   const QrShared sh{red, wl, dots, piv, sm, taul};
   const QjJob& jb = jobs[blockIdx.y];
   const int rows = which == 0 ? jb.n : jb.o, cols = which == 0 ? jb.o : jb.K;
@@ -279,32 +378,42 @@ __global__ __launch_bounds__(NW * 64) void k_qj_qr(const QjJob* __restrict__ job
   if (s >= np || t >= nb) return;
   const int w = wave_id(), lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int base = max(s, 0);
-  double* P = jb.A[which] + (int64_t)t * rb * 256;
-  double4_t a[TPW];
+  double* P = jb.A[which] + (int64_t)t * rb * kT;
+  Tile<Z> a[TPW];
 #pragma unroll
   for (int i = 0; i < TPW; ++i) {
     const int b = base + w + NW * i;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) a[i][r] = b < rb ? P[(int64_t)b * 256 + 64 * r + lane] : 0.0;
+    for (int r = 0; r < 4; ++r) {
+      a[i].r[r] = b < rb ? P[(int64_t)b * kT + 64 * r + lane] : 0.0;
+      if constexpr (Z) a[i].i[r] = b < rb ? P[(int64_t)b * kT + 256 + 64 * r + lane] : 0.0;
+    }
   }
   double* An = jb.A[which + 1];
   const int rbn = nb;  // row blocks of the next matrix
   if (s >= 0) {
-    const double* V = jb.A[which] + (int64_t)s * rb * 256;
-    const double* T = jb.T[which] + (int64_t)s * 256;
-    const double4_t W = slab_vta<NW, TPW>(V, base, rb, a, sh);
-    // Y = T^T W, its rows ordered for slab_sub: row i = 4r + g of the product is row 4g + r of Y
+    const double* V = jb.A[which] + (int64_t)s * rb * kT;
+    const double* T = jb.T[which] + (int64_t)s * kT;
+    const Tile<Z> W = slab_vha<Z, NW, TPW>(V, base, base, rb, a, sh);
+    // Y = T^H W, its rows ordered for slab_sub: row i = 4r + g of the product is row 4g + r of Y
     const int m = 4 * (c & 3) + (c >> 2);
-    double4_t Y = {0.0, 0.0, 0.0, 0.0};
+    Tile<Z> Y = {kZero4, kZero4};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) Y = mfma(T[(4 * k + g) * 16 + m], W[k], Y);
-    slab_sub<NW, TPW>(V, base, rb, a, Y);
-    if (w == 0) {  // rows 16 s .. of R are final: transposed into the next matrix
-      double* q = An + (int64_t)s * rbn * 256 + (int64_t)t * 256 + c * 16 + g;
+    for (int k = 0; k < 4; ++k) {
+      const double* tk = T + (4 * k + g) * 16 + m;
+      mac_h<Z>(Y, tk[0], Z ? tk[256] : 0.0, W.r[k], Z ? W.i[k] : 0.0);
+    }
+    slab_sub<Z, NW, TPW>(V, base, base, rb, a, Y);
+    if (w == 0) {  // rows 16 s .. of R are final: conjugate-transposed into the next matrix
+      double* q = An + ((int64_t)s * rbn + t) * kT + c * 16 + g;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        q[4 * r] = a[0][r];
-        a[0][r] = 0.0;
+        q[4 * r] = a[0].r[r];
+        a[0].r[r] = 0.0;
+        if constexpr (Z) {
+          q[256 + 4 * r] = -a[0].i[r];
+          a[0].i[r] = 0.0;
+        }
       }
     }
   }
@@ -312,14 +421,18 @@ __global__ __launch_bounds__(NW * 64) void k_qj_qr(const QjJob* __restrict__ job
   const int pw = s >= 0 ? 1 : 0;  // wave of the pivot tile
   if (factor) {
     const bool top = w == pw;
-    panel_columns<0, NW, TPW>(a, (rb - base - w + NW - 1) / NW, top, sh);
+    panel_columns<Z, 0, NW, TPW>(a, (rb - base - w + NW - 1) / NW, top, sh);
     if (top) {
-      double* q = An + (int64_t)t * rbn * 256 + (int64_t)t * 256 + c * 16 + g;
+      double* q = An + ((int64_t)t * rbn + t) * kT + c * 16 + g;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = 4 * r + g;
-        q[4 * r] = row <= c ? a[0][r] : 0.0;
-        a[0][r] = row > c ? a[0][r] : row == c ? 1.0 : 0.0;
+        q[4 * r] = row <= c ? a[0].r[r] : 0.0;
+        a[0].r[r] = row > c ? a[0].r[r] : row == c ? 1.0 : 0.0;
+        if constexpr (Z) {
+          q[256 + 4 * r] = row <= c ? -a[0].i[r] : 0.0;
+          a[0].i[r] = row > c ? a[0].i[r] : 0.0;
+        }
       }
     }
   }
@@ -328,29 +441,41 @@ __global__ __launch_bounds__(NW * 64) void k_qj_qr(const QjJob* __restrict__ job
     const int b = base + w + NW * i;
     if (b < rb && !(s >= 0 && b == s)) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) P[(int64_t)b * 256 + 64 * r + lane] = a[i][r];
+      for (int r = 0; r < 4; ++r) {
+        P[(int64_t)b * kT + 64 * r + lane] = a[i].r[r];
+        if constexpr (Z) P[(int64_t)b * kT + 256 + 64 * r + lane] = a[i].i[r];
+      }
     }
   }
   if (!factor) return;
   __syncthreads();
-  // T = (diag(1/tau) + strictly upper V^T V)^-1, one column per lane
+  // T = (diag(1/tau) + strictly upper V^H V)^-1, one column per lane
   if (w == 0 && g == 0) {
-    double x[16];
+    double x[16], xz[16];
 #pragma unroll
     for (int i = 15; i >= 0; --i) {
-      double acc0 = 0.0, acc1 = 0.0;
+      double acc[2] = {0.0, 0.0}, accz[2] = {0.0, 0.0};
 #pragma unroll
       for (int k = i + 1; k < 16; ++k) {
-        if (k & 1)
-          acc1 += sm[i * 16 + k] * x[k];
-        else
-          acc0 += sm[i * 16 + k] * x[k];
+        const double sr = sm[i * 16 + k];
+        acc[k & 1] += sr * x[k];
+        if constexpr (Z) {
+          const double si = sm[256 + i * 16 + k];
+          acc[k & 1] -= si * xz[k];
+          accz[k & 1] += sr * xz[k] + si * x[k];
+        }
       }
-      x[i] = i == c ? taul[i] : i < c ? -taul[i] * (acc0 + acc1) : 0.0;
+      const double sr = acc[0] + acc[1], si = accz[0] + accz[1];
+      const double tr = taul[i], ti = Z ? taul[16 + i] : 0.0;
+      x[i] = i == c ? tr : i < c ? -(tr * sr - ti * si) : 0.0;
+      xz[i] = i == c ? ti : i < c ? -(tr * si + ti * sr) : 0.0;
     }
-    double* T = jb.T[which] + (int64_t)t * 256;
+    double* T = jb.T[which] + (int64_t)t * kT;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) T[i * 16 + c] = x[i];
+    for (int i = 0; i < 16; ++i) {
+      T[i * 16 + c] = x[i];
+      if constexpr (Z) T[256 + i * 16 + c] = xz[i];
+    }
   }
 }
 
@@ -362,13 +487,14 @@ __global__ __launch_bounds__(256) void k_qj_norms0(const QjJob* __restrict__ job
   const int j0 = blockIdx.x * 64;
   if (j0 >= jb.o) return;
   if (j0 == 0 && threadIdx.x == 0) *jb.last = -1;
-  const int w = wave_id(), lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const double* Mi = jb.M + jb.plane;  // imaginary plane (the real one itself for real tensors)
   if (jb.dir < 0) {
     double acc = 0.0;
     if (j0 + lane < jb.o)
       for (int i = w; i < jb.n; i += 4) {
-        const double v = jb.M[(int64_t)(j0 + lane) + (int64_t)i * jb.R];
-        acc += v * v;
+        const int64_t e = (int64_t)(j0 + lane) + (int64_t)i * jb.R;
+        acc += jb.M[e] * jb.M[e] + Mi[e] * Mi[e];
       }
     part[w][lane] = acc;
     __syncthreads();
@@ -377,8 +503,8 @@ __global__ __launch_bounds__(256) void k_qj_norms0(const QjJob* __restrict__ job
     for (int k = w; k < 64 && j0 + k < jb.o; k += 4) {
       double acc = 0.0;
       for (int i = lane; i < jb.n; i += 64) {
-        const double v = jb.M[(int64_t)i + (int64_t)(j0 + k) * jb.R];
-        acc += v * v;
+        const int64_t e = (int64_t)i + (int64_t)(j0 + k) * jb.R;
+        acc += jb.M[e] * jb.M[e] + Mi[e] * Mi[e];
       }
       for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
       if (lane == 0) jb.nrm[j0 + k] = acc;
@@ -405,17 +531,21 @@ __global__ __launch_bounds__(256) void k_qj_rank(const QjJob* __restrict__ jobs)
 }
 
 // Panels of A0: sorted columns, scaled, zero-padded.
+template <bool Z>
 __global__ __launch_bounds__(256) void k_qj_gather(const QjJob* __restrict__ jobs, double scale) {
   const QjJob& jb = jobs[blockIdx.y];
   const int p = blockIdx.x;
   if (p >= blocks16(jb.o)) return;
   const int rb = blocks16(jb.n), c = threadIdx.x & 15, rr = threadIdx.x >> 4;
   const int col = p * 16 + c < jb.o ? jb.perm[p * 16 + c] : -1;
-  double* dst = jb.A[0] + (int64_t)p * rb * 256 + threadIdx.x;
+  double* dst = jb.A[0] + (int64_t)p * rb * kTile<Z> + threadIdx.x;
   const int64_t cs = jb.dir > 0 ? jb.R : 1, is = jb.dir > 0 ? 1 : jb.R;
   for (int b = blockIdx.z; b < rb; b += gridDim.z) {
     const int i = b * 16 + rr;
-    dst[(int64_t)b * 256] = col >= 0 && i < jb.n ? scale * jb.M[col * cs + i * is] : 0.0;
+    const bool in = col >= 0 && i < jb.n;
+    const double* m = jb.M + col * cs + i * is;
+    dst[(int64_t)b * kTile<Z>] = in ? scale * m[0] : 0.0;
+    if constexpr (Z) dst[(int64_t)b * kTile<Z> + 256] = in ? scale * m[jb.plane] : 0.0;
   }
 }
 
@@ -425,11 +555,13 @@ __global__ __launch_bounds__(256) void k_qj_gather(const QjJob* __restrict__ job
 // product Y V on the matrix cores.  Pairs whose columns are orthogonal already
 // (relative to tol; norms below `floor` count as `floor`) stop after the Gram
 // matrix.  A sector stops when a whole cycle of its rounds rotated nothing.
+template <bool Z>
 __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs, int step, double tol2,
                                                   double floor2) {
-  constexpr int kW = 8, kU = 4, kLd = 33;  // waves, row blocks in flight per wave, leading dimension
-  __shared__ double red[kW][3][256];
-  __shared__ double G[2][32 * kLd], V[32 * kLd];
+  // waves, row blocks in flight per wave, planes, leading dimension and size of a 32 x 32 matrix in LDS
+  constexpr int kW = 8, kU = Z ? 2 : 4, kP = Z ? 2 : 1, kLd = 33, kM = 32 * kLd, kT = kTile<Z>;
+  __shared__ double red[kW * 3 * kT];   // partial Gram tiles, then four matrices
+  __shared__ double G[kP * kM];
   __shared__ double cn[32];
   __shared__ int order[32];
   const QjJob& jb = jobs[blockIdx.y];
@@ -444,18 +576,18 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
     q = t;
   }
   if (q >= npan) return;
-  double* Yp = jb.A[2] + (int64_t)p * rb * 256;
-  double* Yq = jb.A[2] + (int64_t)q * rb * 256;
+  double* Yp = jb.A[2] + (int64_t)p * rb * kT;
+  double* Yq = jb.A[2] + (int64_t)q * rb * kT;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   {
-    double4_t pp = {0.0, 0.0, 0.0, 0.0}, pq = pp, qq = pp;
+    Tile<Z> pp = {kZero4, kZero4}, pq = pp, qq = pp;
     for (int b0 = w; b0 < rb; b0 += kU * kW) {
-      double x[kU][4], y[kU][4];
+      double x[kU][4 * kP], y[kU][4 * kP];
 #pragma unroll
       for (int u = 0; u < kU; ++u) {
-        const int64_t o = (int64_t)min(b0 + u * kW, rb - 1) * 256 + lane;
+        const int64_t o = (int64_t)min(b0 + u * kW, rb - 1) * kT + lane;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < 4 * kP; ++r) {
           x[u][r] = Yp[o + 64 * r];
           y[u][r] = Yq[o + 64 * r];
         }
@@ -465,28 +597,36 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
         if (b0 + u * kW < rb) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            pp = mfma(x[u][r], x[u][r], pp);
-            pq = mfma(x[u][r], y[u][r], pq);
-            qq = mfma(y[u][r], y[u][r], qq);
+            const double xr = x[u][r], yr = y[u][r], xi = Z ? x[u][(4 + r) % (4 * kP)] : 0.0,
+                         yi = Z ? y[u][(4 + r) % (4 * kP)] : 0.0;
+            mac_h<Z>(pp, xr, xi, xr, xi);
+            mac_h<Z>(pq, xr, xi, yr, yi);
+            mac_h<Z>(qq, yr, yi, yr, yi);
           }
         }
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      red[w][0][64 * r + lane] = pp[r];
-      red[w][1][64 * r + lane] = pq[r];
-      red[w][2][64 * r + lane] = qq[r];
+      double* d = red + w * 3 * kT + 64 * r + lane;
+      d[0] = pp.r[r];
+      d[kT] = pq.r[r];
+      d[2 * kT] = qq.r[r];
+      if constexpr (Z) {
+        d[256] = pp.i[r];
+        d[kT + 256] = pq.i[r];
+        d[2 * kT + 256] = qq.i[r];
+      }
     }
   }
   __syncthreads();
-  for (int e = tid; e < 768; e += 512) {
+  for (int e = tid; e < 3 * kT; e += 512) {
     double t = 0.0;
-    const int m = e >> 8, x = e & 255;
+    const int m = e / kT, im = Z ? (e >> 8) & 1 : 0, x = e & 255;
 #pragma unroll
-    for (int k = 0; k < kW; ++k) t += red[k][m][x];
+    for (int k = 0; k < kW; ++k) t += red[k * 3 * kT + e];
     const int i = (x >> 4) + (m == 2 ? 16 : 0), j = (x & 15) + (m >= 1 ? 16 : 0);
-    G[0][i * kLd + j] = t;
-    if (m == 1) G[0][j * kLd + i] = t;
+    G[im * kM + i * kLd + j] = t;
+    if (m == 1) G[im * kM + j * kLd + i] = im ? -t : t;
   }
   __syncthreads();
   constexpr double eps2 = 2.220446049250313e-16 * 2.220446049250313e-16;
@@ -494,44 +634,60 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int i = (tid >> 5) + 16 * h, j = tid & 31;
-    const double gi = G[0][i * kLd + i], gj = G[0][j * kLd + j], x = G[0][i * kLd + j];
-    act |= i < j && x * x > tol2 * fmax(gi, gj) * fmax(fmin(gi, gj), floor2);
+    const double gi = G[i * kLd + i], gj = G[j * kLd + j], x = G[i * kLd + j], y = Z ? G[(kP - 1) * kM + i * kLd + j] : 0.0;
+    act |= i < j && x * x + y * y > tol2 * fmax(gi, gj) * fmax(fmin(gi, gj), floor2);
   }
   if (!__syncthreads_or(act)) return;
   if (tid == 0) *jb.last = step;
   // Inner solve, all pairs at once: X holds the Jacobi tangents of every pair
   // (scaled down where a column of X exceeds kCap in the 2-norm), V the
-  // orthogonal polar factor of I + X by Newton-Schulz steps V += V (I - V^T V) / 2
-  // on the matrix cores, repeated on V^T G V while the rotations were large.
+  // unitary polar factor of I + X by Newton-Schulz steps V += V (I - V^H V) / 2
+  // on the matrix cores, repeated on V^H G V while the rotations were large.
   // Its off-diagonal rest is of second order, as after a cyclic sweep of
   // rotations, at a fraction of the latency: a sweep is 31 dependent rounds of
   // LDS traffic, 46000 cycles, this 8000 to 33000, and one outer sweep fewer
-  // on the sectors of an m=1024 Heisenberg state.
+  // on the sectors of an m=1024 Heisenberg state.  (A cosine applied to a
+  // column would also scale it by its rounding error, and those factors add up
+  // over the rounds: 3e-14 of the singular values of a 200 x 200 Gaussian
+  // matrix, against 1.5e-15.)
   constexpr double kCap = 0.7, kSmall = 0.25;
   constexpr int kRepeats = 2, kNewton = 12;
-  double* E = G[1];
-  double* Vt = &red[0][0][0];      // the products so far
-  double* Tm = Vt + 32 * kLd;      // scratch
+  double* V = red;             // this repeat's factor
+  double* Vt = V + kP * kM;    // the products so far
+  double* Tm = Vt + kP * kM;   // scratch
+  double* E = Tm + kP * kM;    // (I - V^H V) / 2
   const int ti = (w >> 1) & 1, tj = w & 1;  // waves 0..3: a 16 x 16 tile each
-  auto mul = [&](const double* A, bool tA, const double* B, double4_t acc) {
+  const bool mine = w < 4;
+  auto mul = [&](const double* A, bool tA, const double* B, Tile<Z> acc) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const int kk = 4 * k + g;
-      acc = mfma(tA ? A[kk * kLd + 16 * ti + c] : A[(16 * ti + c) * kLd + kk], B[kk * kLd + 16 * tj + c], acc);
+      const double* a = tA ? A + kk * kLd + 16 * ti + c : A + (16 * ti + c) * kLd + kk;
+      const double* b = B + kk * kLd + 16 * tj + c;
+      if (tA)
+        mac_h<Z>(acc, a[0], Z ? a[(kP - 1) * kM] : 0.0, b[0], Z ? b[(kP - 1) * kM] : 0.0);
+      else
+        mac<Z>(acc, a[0], Z ? a[(kP - 1) * kM] : 0.0, b[0], Z ? b[(kP - 1) * kM] : 0.0);
     }
     return acc;
   };
   auto get = [&](const double* D) {
-    double4_t v;
+    Tile<Z> v;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = D[(16 * ti + 4 * r + g) * kLd + 16 * tj + c];
+    for (int r = 0; r < 4; ++r) {
+      v.r[r] = D[(16 * ti + 4 * r + g) * kLd + 16 * tj + c];
+      v.i[r] = Z ? D[(kP - 1) * kM + (16 * ti + 4 * r + g) * kLd + 16 * tj + c] : 0.0;
+    }
     return v;
   };
-  auto put = [&](double* D, double4_t v) {
+  auto put = [&](double* D, const Tile<Z>& v) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) D[(16 * ti + 4 * r + g) * kLd + 16 * tj + c] = v[r];
+    for (int r = 0; r < 4; ++r) {
+      D[(16 * ti + 4 * r + g) * kLd + 16 * tj + c] = v.r[r];
+      if constexpr (Z) D[kM + (16 * ti + 4 * r + g) * kLd + 16 * tj + c] = v.i[r];
+    }
   };
-  const double4_t zero4 = {0.0, 0.0, 0.0, 0.0};
+  const Tile<Z> zero = {kZero4, kZero4};
   double cap = kCap;
   for (int it = 0; it < kRepeats;) {
     // tangents in single precision (any nearby V serves), and the order of the
@@ -539,26 +695,37 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int i = (tid >> 5) + 16 * h, j = tid & 31;
-      const double gi = G[0][i * kLd + i], gj = G[0][j * kLd + j], x = G[0][i * kLd + j], d = gj - gi;
-      const bool go = i != j && x * x > fmax(eps2 * gi * gj, 1e-280);
-      const float f = (float)(d * __builtin_amdgcn_rcp(go ? 2.0 * x : 1.0));
-      const bool neg = f < 0.0f || (f == 0.0f && (i > j) != (x < 0.0));
-      const float t = jacobi_tangent(fabsf(f));
-      V[i * kLd + j] = i == j ? 1.0 : go ? (double)(neg ? -t : t) : 0.0;
+      const double gi = G[i * kLd + i], gj = G[j * kLd + j], x = G[i * kLd + j], d = gj - gi;
+      if constexpr (Z) {
+        const double y = G[kM + i * kLd + j], q2 = x * x + y * y;
+        const bool go = i != j && q2 > fmax(eps2 * gi * gj, 1e-280);
+        const double ri = fast_rsqrt(go ? q2 : 1.0);   // 1 / |g_ij|
+        const float f = (float)(0.5 * d * ri);
+        const bool neg = f < 0.0f || (f == 0.0f && i > j);
+        const double t = go ? (double)jacobi_tangent(fabsf(f)) * ri : 0.0;
+        V[i * kLd + j] = i == j ? 1.0 : neg ? -t * x : t * x;
+        V[kM + i * kLd + j] = i == j ? 0.0 : neg ? -t * y : t * y;
+      } else {
+        const bool go = i != j && x * x > fmax(eps2 * gi * gj, 1e-280);
+        const float f = (float)(d * __builtin_amdgcn_rcp(go ? 2.0 * x : 1.0));
+        const bool neg = f < 0.0f || (f == 0.0f && (i > j) != (x < 0.0));
+        const float t = jacobi_tangent(fabsf(f));
+        V[i * kLd + j] = i == j ? 1.0 : go ? (double)(neg ? -t : t) : 0.0;
+      }
       const unsigned long long m = __ballot(gj > gi || (gj == gi && j < i));
       if (j == 0) order[__popc((unsigned)(lane < 32 ? m : m >> 32))] = i;
     }
     __syncthreads();
-    // X is skew: I - V^T V = X^2, and V + X^2 / 2 is orthogonal up to X^4 / 4
-    double4_t v = zero4, e = zero4;
-    if (w < 4) {
+    // X is skew: I - V^H V = X^2, and V + X^2 / 2 is unitary up to X^4 / 4
+    Tile<Z> v = zero, e = zero;
+    if (mine) {
       v = get(V);
-      e = mul(V, true, V, zero4);
+      e = mul(V, true, V, zero);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const bool one = ti == tj && 4 * r + g == c;
-        e[r] = (one ? 1.0 : 0.0) - e[r];
-        if (one) cn[16 * ti + c] = -e[r];  // squared norms of the columns of X
+        e.r[r] = (one ? 1.0 : 0.0) - e.r[r];
+        if (one) cn[16 * ti + c] = -e.r[r];  // squared norms of the columns of X
       }
     }
     __syncthreads();
@@ -566,12 +733,13 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
 #pragma unroll
     for (int k = 0; k < 32; ++k) mx = fmax(mx, cn[k]);
     const bool large = mx > kSmall * kSmall;
-    if (w < 4) {
+    if (mine) {
       const double a2 = mx > cap * cap ? cap * cap / mx : 1.0, a1 = sqrt(a2);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const bool one = ti == tj && 4 * r + g == c;
-        v[r] = (one ? 1.0 : a1 * v[r]) + 0.5 * a2 * e[r];
+        v.r[r] = (one ? 1.0 : a1 * v.r[r]) + 0.5 * a2 * e.r[r];
+        if constexpr (Z) v.i[r] = a1 * v.i[r] - 0.5 * a2 * e.i[r];
       }
       put(V, v);
     }
@@ -583,23 +751,27 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
     bool conv = dev < 1e-17;
     for (int nt = 0; nt < kNewton && !conv; ++nt) {
       int big = 0;
-      if (w < 4) {
-        e = mul(V, true, V, zero4);
+      if (mine) {
+        e = mul(V, true, V, zero);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          e[r] = (ti == tj && 4 * r + g == c ? 1.0 : 0.0) - e[r];
-          big |= fabs(e[r]) > 1e-8;
+          e.r[r] = (ti == tj && 4 * r + g == c ? 0.5 : 0.0) - 0.5 * e.r[r];
+          big |= fabs(e.r[r]) > 5e-9;
+          if constexpr (Z) {
+            e.i[r] *= -0.5;
+            big |= fabs(e.i[r]) > 5e-9;
+          }
         }
-        put(E, 0.5 * e);
+        put(E, e);
       }
       if (dev < 1e-8)
         conv = !__syncthreads_or(big);
       else
         __syncthreads();
       dev *= 0.75 * dev;
-      if (w < 4) v = mul(V, false, E, get(V));
+      if (mine) v = mul(V, false, E, get(V));
       __syncthreads();
-      if (w < 4) put(V, v);
+      if (mine) put(V, v);
       __syncthreads();
     }
     if (!conv) {
@@ -610,64 +782,77 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
       continue;
     }
     if (it > 0) {
-      if (w < 4) v = mul(Vt, false, V, zero4);
+      if (mine) v = mul(Vt, false, V, zero);
       __syncthreads();
-      if (w < 4) put(Vt, v);
-    } else if (w < 4) {
+      if (mine) put(Vt, v);
+    } else if (mine) {
       put(Vt, get(V));
     }
     if (!large || ++it == kRepeats) break;
-    if (w < 4) put(Tm, mul(G[0], false, V, zero4));
+    if (mine) put(Tm, mul(G, false, V, zero));
     __syncthreads();
-    if (w < 4) put(G[0], mul(V, true, Tm, zero4));
+    if (mine) put(G, mul(V, true, Tm, zero));
     __syncthreads();
   }
   __syncthreads();
-  double vb[2][8];
+  double vb[2][8], vi[2][8];
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      vb[h][k] = Vt[((k >> 2) * 16 + 4 * g + (k & 3)) * kLd + order[16 * h + c]];
-  for (int b0 = w; b0 < rb; b0 += 2 * kW) {
-    double2_t x[2][4];
+    for (int k = 0; k < 8; ++k) {
+      const int e = ((k >> 2) * 16 + 4 * g + (k & 3)) * kLd + order[16 * h + c];
+      vb[h][k] = Vt[e];
+      vi[h][k] = Z ? Vt[(kP - 1) * kM + e] : 0.0;
+    }
+  constexpr int kV = Z ? 1 : 2;  // row blocks in flight per wave
+  for (int b0 = w; b0 < rb; b0 += kV * kW) {
+    double2_t x[kV][4 * kP];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int64_t o = (int64_t)min(b0 + u * kW, rb - 1) * 256 + c * 16 + 4 * g;
-      x[u][0] = *(const double2_t*)(Yp + o);
-      x[u][1] = *(const double2_t*)(Yp + o + 2);
-      x[u][2] = *(const double2_t*)(Yq + o);
-      x[u][3] = *(const double2_t*)(Yq + o + 2);
+    for (int u = 0; u < kV; ++u) {
+      const int64_t o = (int64_t)min(b0 + u * kW, rb - 1) * kT + c * 16 + 4 * g;
+#pragma unroll
+      for (int h = 0; h < kP; ++h) {
+        x[u][4 * h + 0] = *(const double2_t*)(Yp + o + 256 * h);
+        x[u][4 * h + 1] = *(const double2_t*)(Yp + o + 256 * h + 2);
+        x[u][4 * h + 2] = *(const double2_t*)(Yq + o + 256 * h);
+        x[u][4 * h + 3] = *(const double2_t*)(Yq + o + 256 * h + 2);
+      }
     }
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < kV; ++u)
       if (b0 + u * kW < rb) {
-        double4_t yp = {0.0, 0.0, 0.0, 0.0}, yq = yp;
+        Tile<Z> yp = zero, yq = zero;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-          yp = mfma(x[u][k >> 1][k & 1], vb[0][k], yp);
-          yq = mfma(x[u][k >> 1][k & 1], vb[1][k], yq);
+          const double xr = x[u][k >> 1][k & 1], xi = Z ? x[u][4 * (kP - 1) + (k >> 1)][k & 1] : 0.0;
+          mac<Z>(yp, xr, xi, vb[0][k], vi[0][k]);
+          mac<Z>(yq, xr, xi, vb[1][k], vi[1][k]);
         }
-        const int64_t o = (int64_t)(b0 + u * kW) * 256 + lane;
+        const int64_t o = (int64_t)(b0 + u * kW) * kT + lane;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          Yp[o + 64 * r] = yp[r];
-          Yq[o + 64 * r] = yq[r];
+          Yp[o + 64 * r] = yp.r[r];
+          Yq[o + 64 * r] = yq.r[r];
+          if constexpr (Z) {
+            Yp[o + 256 + 64 * r] = yp.i[r];
+            Yq[o + 256 + 64 * r] = yq.i[r];
+          }
         }
       }
   }
 }
 
 // Column norms of A2: one panel a group, 16 per panel in nrm.
-__global__ __launch_bounds__(256) void k_qj_norms3(const QjJob* __restrict__ jobs) {
+template <bool Z>
+__global__ __launch_bounds__(256) void k_qj_norms2(const QjJob* __restrict__ jobs) {
   __shared__ double part[4][16];
   const QjJob& jb = jobs[blockIdx.y];
   const int rb = blocks16(jb.K), p = blockIdx.x;
   if (p >= rb) return;
-  const int w = wave_id(), lane = threadIdx.x & 63;
-  const double* P = jb.A[2] + (int64_t)p * rb * 256 + threadIdx.x;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const double* P = jb.A[2] + (int64_t)p * rb * kTile<Z> + threadIdx.x;
   double acc = 0.0;
-  for (int b = 0; b < rb; ++b) acc += P[(int64_t)b * 256] * P[(int64_t)b * 256];
+  for (int b = 0; b < rb * (Z ? 2 : 1); ++b) acc += P[(int64_t)b * 256] * P[(int64_t)b * 256];
   acc = sum_rows(acc);
   if (lane < 16) part[w][lane] = acc;
   __syncthreads();
@@ -679,9 +864,10 @@ __global__ __launch_bounds__(256) void k_qj_norms3(const QjJob* __restrict__ job
 // The kept vectors: 16 normalised columns of A2 a group, the block
 // reflectors of the first factorisation applied to them from the last to the
 // first in registers.
-template <int NW, int TPW>
+template <bool Z, int NW, int TPW>
 __global__ __launch_bounds__(NW * 64) void k_qj_back(const QjJob* __restrict__ jobs) {
-  __shared__ double red[NW * 256], wl[256];
+  constexpr int kT = kTile<Z>;
+  __shared__ double red[NW * kT], wl[kT];
   const QrShared sh{red, wl, nullptr, nullptr, nullptr, nullptr};
   const QjJob& jb = jobs[blockIdx.y];
   const int k0 = blockIdx.x * 16;
@@ -691,52 +877,28 @@ __global__ __launch_bounds__(NW * 64) void k_qj_back(const QjJob* __restrict__ j
   const int k = k0 + c;
   const int src = k < jb.keep ? jb.kcol[k] : -1;
   const double inv = k < jb.keep ? jb.kinv[k] : 0.0;
-  const double* S = jb.A[2] + (int64_t)(max(src, 0) >> 4) * kb * 256 + (max(src, 0) & 15);
-  double4_t a[TPW];
+  const double* S = jb.A[2] + (int64_t)(max(src, 0) >> 4) * kb * kT + (max(src, 0) & 15);
+  Tile<Z> a[TPW];
 #pragma unroll
   for (int i = 0; i < TPW; ++i) {
     const int b = w + NW * i;
+    const bool in = b < kb && src >= 0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) a[i][r] = b < kb && src >= 0 ? inv * S[(int64_t)b * 256 + (4 * r + g) * 16] : 0.0;
+    for (int r = 0; r < 4; ++r) {
+      a[i].r[r] = in ? inv * S[(int64_t)b * kT + (4 * r + g) * 16] : 0.0;
+      if constexpr (Z) a[i].i[r] = in ? inv * S[(int64_t)b * kT + 256 + (4 * r + g) * 16] : 0.0;
+    }
   }
   const int m = 4 * (c & 3) + (c >> 2);
   for (int s = kb - 1; s >= 0; --s) {
-    const double* V = jb.A[0] + (int64_t)s * rb * 256;
-    const double* T = jb.T[0] + (int64_t)s * 256;
+    const double* V = jb.A[0] + (int64_t)s * rb * kT;
+    const double* T = jb.T[0] + (int64_t)s * kT + m * 16 + g;
     // row blocks above s do not take part: their V is not stored
-    double4_t acc = {0.0, 0.0, 0.0, 0.0};
+    const Tile<Z> W = slab_vha<Z, NW, TPW>(V, 0, s, rb, a, sh);
+    Tile<Z> Y = {kZero4, kZero4};
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      const int b = w + NW * i;
-      const double z = b >= s && b < rb ? 1.0 : 0.0;
-      const double* v = V + (int64_t)min(max(b, s), rb - 1) * 256 + lane;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc = mfma(v[64 * r], z * a[i][r], acc);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) red[w * 256 + 64 * r + lane] = acc[r];
-    __syncthreads();
-    if (threadIdx.x < 256) {
-      double t = 0.0;
-#pragma unroll
-      for (int j = 0; j < NW; ++j) t += red[j * 256 + threadIdx.x];
-      wl[threadIdx.x] = t;
-    }
-    __syncthreads();
-    double4_t Y = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) Y = mfma(T[m * 16 + 4 * j + g], wl[64 * j + lane], Y);
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      const int b = w + NW * i;
-      const double z = b >= s && b < rb ? -1.0 : 0.0;
-      const double2_t* v = (const double2_t*)(V + (int64_t)min(max(b, s), rb - 1) * 256 + c * 16 + 4 * g);
-      const double2_t v0 = v[0], v1 = v[1];
-      a[i] = mfma(z * v0[0], Y[0], a[i]);
-      a[i] = mfma(z * v0[1], Y[1], a[i]);
-      a[i] = mfma(z * v1[0], Y[2], a[i]);
-      a[i] = mfma(z * v1[1], Y[3], a[i]);
-    }
+    for (int j = 0; j < 4; ++j) mac<Z>(Y, T[4 * j], Z ? T[256 + 4 * j] : 0.0, W.r[j], Z ? W.i[j] : 0.0);
+    slab_sub<Z, NW, TPW>(V, 0, s, rb, a, Y);
   }
   if (k >= jb.keep) return;
 #pragma unroll
@@ -744,7 +906,10 @@ __global__ __launch_bounds__(NW * 64) void k_qj_back(const QjJob* __restrict__ j
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = 16 * (w + NW * i) + 4 * r + g;
-      if (row < jb.n) jb.out[row * jb.es + k * jb.vs] = a[i][r];
+      if (row < jb.n) {
+        jb.out[row * jb.es + k * jb.vs] = a[i].r[r];
+        if constexpr (Z) jb.out[jb.oplane + row * jb.es + k * jb.vs] = a[i].i[r];
+      }
     }
 }
 
@@ -757,33 +922,41 @@ constexpr int max_rows() {
   return 16 * NW * TPW;
 }
 
+template <bool Z>
 void launch_qr_step(Context& c, const QjJob* dj, int rows, int which, int s, dim3 grid) {
   if (rows <= max_rows<8, 2>())
-    hipLaunchKernelGGL((k_qj_qr<8, 2>), grid, dim3(512), 0, c.stream, dj, which, s);
+    hipLaunchKernelGGL((k_qj_qr<Z, 8, 2>), grid, dim3(512), 0, c.stream, dj, which, s);
   else if (rows <= max_rows<8, 4>())
-    hipLaunchKernelGGL((k_qj_qr<8, 4>), grid, dim3(512), 0, c.stream, dj, which, s);
+    hipLaunchKernelGGL((k_qj_qr<Z, 8, 4>), grid, dim3(512), 0, c.stream, dj, which, s);
+  else if constexpr (Z)
+    hipLaunchKernelGGL((k_qj_qr<true, 8, 8>), grid, dim3(512), 0, c.stream, dj, which, s);
   else if (rows <= max_rows<16, 4>())
-    hipLaunchKernelGGL((k_qj_qr<16, 4>), grid, dim3(1024), 0, c.stream, dj, which, s);
+    hipLaunchKernelGGL((k_qj_qr<false, 16, 4>), grid, dim3(1024), 0, c.stream, dj, which, s);
   else
-    hipLaunchKernelGGL((k_qj_qr<16, 8>), grid, dim3(1024), 0, c.stream, dj, which, s);
+    hipLaunchKernelGGL((k_qj_qr<false, 16, 8>), grid, dim3(1024), 0, c.stream, dj, which, s);
 }
 
+template <bool Z>
 void launch_back(Context& c, const QjJob* dj, int rows, dim3 grid) {
   if (rows <= max_rows<8, 2>())
-    hipLaunchKernelGGL((k_qj_back<8, 2>), grid, dim3(512), 0, c.stream, dj);
+    hipLaunchKernelGGL((k_qj_back<Z, 8, 2>), grid, dim3(512), 0, c.stream, dj);
   else if (rows <= max_rows<8, 4>())
-    hipLaunchKernelGGL((k_qj_back<8, 4>), grid, dim3(512), 0, c.stream, dj);
+    hipLaunchKernelGGL((k_qj_back<Z, 8, 4>), grid, dim3(512), 0, c.stream, dj);
+  else if constexpr (Z)
+    hipLaunchKernelGGL((k_qj_back<true, 8, 8>), grid, dim3(512), 0, c.stream, dj);
   else if (rows <= max_rows<16, 4>())
-    hipLaunchKernelGGL((k_qj_back<16, 4>), grid, dim3(1024), 0, c.stream, dj);
+    hipLaunchKernelGGL((k_qj_back<false, 16, 4>), grid, dim3(1024), 0, c.stream, dj);
   else
-    hipLaunchKernelGGL((k_qj_back<16, 8>), grid, dim3(1024), 0, c.stream, dj);
+    hipLaunchKernelGGL((k_qj_back<false, 16, 8>), grid, dim3(1024), 0, c.stream, dj);
 }
 
 int up16(int n) { return (n + 15) / 16 * 16; }
 
 }  // namespace
 
-bool qj_fits(int64_t R, int64_t C) { return std::max(R, C) <= max_rows<16, 8>(); }
+bool qj_fits(int64_t R, int64_t C, bool cplx) {
+  return std::max(R, C) <= (cplx ? max_rows<8, 8>() : max_rows<16, 8>());
+}
 
 QjBatch::~QjBatch() {
   c.alloc.release(work);
@@ -806,6 +979,8 @@ bool qj_solve(QjBatch& q, double norm2) {
   const double scale = std::ldexp(1.0, -ex);
   // doubles: the norms of all sectors (one copy to the host), then the
   // matrices; ints: the round counters of all sectors, then the orders
+  const bool z = q.cplx;
+  const int zf = z ? 2 : 1;
   int64_t nd = 0, ni = nj, nn = 0;
   std::vector<int64_t> dof(nj), iof(nj), nof(nj);
   auto kcols = [](int K) { return (int64_t)std::max(up16(K), 32); };  // at least two panels
@@ -814,7 +989,7 @@ bool qj_solve(QjBatch& q, double norm2) {
     nof[j] = nn;
     nn += o;
     dof[j] = nd;
-    nd += n * o + o * Kc + K * Kc + 2 * 16 * K;
+    nd += zf * (n * o + o * Kc + K * Kc + 2 * 16 * K);
     iof[j] = ni;
     ni += o;
   }
@@ -830,10 +1005,11 @@ bool qj_solve(QjBatch& q, double norm2) {
     b = QjJob{};
     b.M = s.M;
     b.A[0] = q.work + nn + dof[j];
-    b.A[1] = b.A[0] + n * o;
-    b.A[2] = b.A[1] + o * Kc;
-    b.T[0] = b.A[2] + K * Kc;
-    b.T[1] = b.T[0] + 16 * K;
+    b.A[1] = b.A[0] + zf * n * o;
+    b.A[2] = b.A[1] + zf * o * Kc;
+    b.T[0] = b.A[2] + zf * K * Kc;
+    b.T[1] = b.T[0] + zf * 16 * K;
+    b.plane = z ? (int64_t)s.n * s.o : 0;
     b.nrm = q.work + nof[j];
     b.perm = q.ints + iof[j];
     b.last = q.ints + j;
@@ -850,8 +1026,11 @@ bool qj_solve(QjBatch& q, double norm2) {
   const int pk = up16(maxK) / 16;
   hipLaunchKernelGGL(k_qj_norms0, dim3((maxo + 63) / 64, nj), dim3(256), 0, c.stream, dj);
   hipLaunchKernelGGL(k_qj_rank, dim3((maxo + 255) / 256, nj), dim3(256), 0, c.stream, dj);
-  hipLaunchKernelGGL(k_qj_gather, dim3(up16(maxo) / 16, nj, std::min(16, up16(maxn) / 16)), dim3(256), 0, c.stream,
-                     dj, scale);
+  const dim3 gg(up16(maxo) / 16, nj, std::min(16, up16(maxn) / 16));
+  if (z)
+    hipLaunchKernelGGL(k_qj_gather<true>, gg, dim3(256), 0, c.stream, dj, scale);
+  else
+    hipLaunchKernelGGL(k_qj_gather<false>, gg, dim3(256), 0, c.stream, dj, scale);
   for (int which = 0; which < 2; ++which) {
     const int rows = which == 0 ? maxn : maxo;
     // slabs and panels of every job in this factorisation
@@ -869,7 +1048,10 @@ bool qj_solve(QjBatch& q, double norm2) {
           gx = std::max(gx, s < 0 ? 1 : slabs[j] - s - 1);
           gy = j + 1;
         }
-      if (gx > 0) launch_qr_step(c, dj, rows, which, s, dim3(gx, gy));
+      if (gx > 0 && z)
+        launch_qr_step<true>(c, dj, rows, which, s, dim3(gx, gy));
+      else if (gx > 0)
+        launch_qr_step<false>(c, dj, rows, which, s, dim3(gx, gy));
     }
   }
   HIP_OK(hipGetLastError());
@@ -886,7 +1068,10 @@ bool qj_solve(QjBatch& q, double norm2) {
   int* hlast = (int*)c.host_sigma((nj + 1) / 2 + 1);
   auto rounds = [&]() {
     for (int k = 0; k < chunk; ++k, ++step)
-      hipLaunchKernelGGL(k_qj_round, dim3(nbmax / 2, nj), dim3(512), 0, c.stream, dj, step, tol * tol, fl * fl);
+      if (z)
+        hipLaunchKernelGGL(k_qj_round<true>, dim3(nbmax / 2, nj), dim3(512), 0, c.stream, dj, step, tol * tol, fl * fl);
+      else
+        hipLaunchKernelGGL(k_qj_round<false>, dim3(nbmax / 2, nj), dim3(512), 0, c.stream, dj, step, tol * tol, fl * fl);
   };
   for (int k = 0; k < 10 && step < 5 * (nbmax - 1); ++k) rounds();  // five sweeps are always needed
   while (!done && step < kMaxSweeps * (nbmax - 1)) {
@@ -903,7 +1088,10 @@ bool qj_solve(QjBatch& q, double norm2) {
   }
   HIP_OK(hipGetLastError());
   if (!done) return false;
-  hipLaunchKernelGGL(k_qj_norms3, dim3(pk, nj), dim3(256), 0, c.stream, dj);
+  if (z)
+    hipLaunchKernelGGL(k_qj_norms2<true>, dim3(pk, nj), dim3(256), 0, c.stream, dj);
+  else
+    hipLaunchKernelGGL(k_qj_norms2<false>, dim3(pk, nj), dim3(256), 0, c.stream, dj);
   double* h = c.host_sigma(nn);
   HIP_OK(hipMemcpyAsync(h, q.work, nn * sizeof(double), hipMemcpyDeviceToHost, c.stream));
   HIP_OK(hipStreamSynchronize(c.stream));
@@ -950,9 +1138,13 @@ void qj_vectors(QjBatch& q) {
     b.es = s.es;
     b.vs = s.vs;
     b.keep = s.keep;
+    b.oplane = s.oplane;
   }
   auto* dj = (QjJob*)c.upload(q.jobs.data(), nj * sizeof(QjJob));
-  launch_back(c, dj, maxn, dim3((maxkeep + 15) / 16, nj));
+  if (q.cplx)
+    launch_back<true>(c, dj, maxn, dim3((maxkeep + 15) / 16, nj));
+  else
+    launch_back<false>(c, dj, maxn, dim3((maxkeep + 15) / 16, nj));
   HIP_OK(hipGetLastError());
 }
 

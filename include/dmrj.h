@@ -135,7 +135,8 @@ int dmrj_ctx_marker(dmrj_ctx* ctx, int id);
  * R + C), the other factor by a grouped GEMM with M: faster, exactly
  * orthonormal factor, singular values with absolute error ~eps |M|^2 (not
  * the FP64 drop-in's accuracy: small sigma and truncation errors near a
- * cutoff differ from LAPACK's).  Complex tensors always use a
+ * cutoff differ from LAPACK's).  Complex tensors of
+ * sides up to 1024 always use the QR-preconditioned block Jacobi, longer ones a
  * batched Hermitian eigensolve of [[0,M],[M^H,0]]. */
 int dmrj_ctx_set_svd_backend(dmrj_ctx* ctx, int mode);
 /* out2 = {SVD calls that used the block one-sided Jacobi, total sweeps of

@@ -78,3 +78,61 @@ def test_svd_scaled(pkg, ctx, scale):
         assert np.max(np.abs(Q.T @ Q - np.eye(97))) <= 1e-13 + 4 * 130 * EPS
         sv.append(s[:97])
     assert np.max(np.abs(sv[0] - sv[1])) <= 2 * 130 * EPS
+
+
+def _complex_matrix(kind, R, Cc, rng):
+    M = rng.standard_normal((R, Cc)) + 1j * rng.standard_normal((R, Cc))
+    if kind == "graded":
+        M = np.exp(-25.0 * np.arange(R) / R)[:, None] * M * np.exp(-10.0 * np.arange(Cc) / Cc)[None, :]
+    return M / np.linalg.norm(M)
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("kind", ["flat", "graded"])
+@pytest.mark.parametrize("shape", [(1, 1), (3, 5), (16, 17), (33, 32), (70, 40), (130, 257), (300, 280), (600, 513),
+                                   (1024, 40), (1030, 40)])
+def test_complex_svd_single_sector(pkg, ctx, shape, kind, direction):
+    """ComplexF64 sectors: same bounds; vectors of sigma <= 1e-10 sigma_max keep
+    the extracted form (no completion), so their orthogonality is not checked."""
+    R, Cc = shape
+    M = _complex_matrix(kind, R, Cc, np.random.default_rng(R * 7 + Cc))
+    t = pkg.site2_from_dense(ctx, M.reshape(R, 1, 1, Cc))
+    l, r, te, kk = C.c_void_p(), C.c_void_p(), C.c_double(), C.c_int64()
+    sv = np.zeros(4096)
+    ctx.call("dmrj_svd_trunc2", t.h, 0, 2, 0.0, direction, C.byref(l), C.byref(r), C.byref(te), C.byref(kk),
+             pkg._lib.dptr(sv), 4096)
+    L = pkg.DeviceTensor(ctx, l).to_dense()[0].reshape(R, -1)
+    Rt = pkg.DeviceTensor(ctx, r).to_dense()[0].reshape(-1, Cc)
+    n = max(R, Cc)
+    want = np.linalg.svd(M, compute_uv=False)
+    assert kk.value == min(R, Cc)
+    assert np.max(np.abs(sv[:kk.value] - want)) <= 2 * n * EPS
+    assert np.max(np.abs(L @ Rt - M)) <= 8 * n * EPS
+    big = want > 1e-10 * want[0]
+    Q = (L if direction > 0 else Rt.conj().T)[:, big]
+    assert np.max(np.abs(Q.conj().T @ Q - np.eye(big.sum()))) <= 1e-13 + 4 * n * EPS
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+def test_complex_svd_sectors_of_different_sizes(pkg, ctx, direction):
+    """Charge sectors of 3 to 67 rows in one call: every vector is finite and
+    the product of the factors is the tensor (a batched Hermitian eigensolve
+    of such sectors, padded to one size, has returned NaN vectors)."""
+    rng = np.random.default_rng(11)
+    dims = {-2: 12, 0: 40, 2: 27, 4: 3}
+    q = np.array([[c] for c in sorted(dims) for _ in range(dims[c])], dtype=np.int32)
+    m = len(q)
+    qp = np.array([[1], [-1]], dtype=np.int32)
+    A = rng.standard_normal((m, 2, 2, m)) + 1j * rng.standard_normal((m, 2, 2, m))
+    ok = (q[:, None, None, None, 0] + qp[None, :, None, None, 0] + qp[None, None, :, None, 0] == q[None, None, None, :, 0])
+    A = np.where(ok, A, 0.0)
+    A /= np.linalg.norm(A)
+    t = pkg.site2_from_dense(ctx, A, q, qp, qp, q, 1)
+    l, r, te, kk = C.c_void_p(), C.c_void_p(), C.c_double(), C.c_int64()
+    sv = np.zeros(4096)
+    ctx.call("dmrj_svd_trunc2", t.h, 0, 2, 0.0, direction, C.byref(l), C.byref(r), C.byref(te), C.byref(kk),
+             pkg._lib.dptr(sv), 4096)
+    L = pkg.DeviceTensor(ctx, l).to_dense(1)[0]
+    Rt = pkg.DeviceTensor(ctx, r).to_dense(1)[0]
+    assert np.all(np.isfinite(L)) and np.all(np.isfinite(Rt))
+    assert np.max(np.abs(np.tensordot(L, Rt, axes=(2, 0)) - A)) <= 8 * 2 * m * EPS
