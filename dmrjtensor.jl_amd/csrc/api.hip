@@ -150,33 +150,70 @@ Allocator::~Allocator() {
 }
 
 // ====================================================================== staging
-void* Context::upload(const void* host, size_t bytes) {
-  const size_t r = (bytes + 255) / 256 * 256;
-  if (stage.used + r > stage.cap) {
-    // all earlier staged copies must have landed before the buffer is reused
-    HIP_OK(hipStreamSynchronize(stream));
-    stage.used = 0;
-    if (r > stage.cap) {
-      if (stage.base) HIP_OK(hipHostFree(stage.base));
-      stage.cap = std::max(r * 2, stage.cap * 2);
-      HIP_OK(hipHostMalloc((void**)&stage.base, stage.cap, hipHostMallocDefault));
-    }
+static Stage new_stage(Context& c, size_t cap) {
+  Stage s;
+  if (hipMalloc((void**)&s.d, cap) != hipSuccess) {
+    (void)hipGetLastError();
+    c.alloc.trim();
+    HIP_OK(hipMalloc((void**)&s.d, cap));
   }
-  char* h = stage.base + stage.used;
+  const hipError_t e = hipHostMalloc((void**)&s.h, cap, hipHostMallocDefault);
+  if (e != hipSuccess) {
+    (void)hipFree(s.d);
+    HIP_OK(e);
+  }
+  s.cap = cap;
+  return s;
+}
+
+void* Context::stage_put(const void* host, size_t bytes) {
+  const size_t r = std::max<size_t>(256, (bytes + 255) / 256 * 256);
+  if (stage.used + r > stage.cap) {
+    // earlier tables keep their block until the stream has been synchronised
+    stage_flush();
+    const size_t cap = std::max<size_t>(std::max<size_t>(2 * r, 2 * stage.cap), 8 << 20);
+    if (stage.cap) stage_old.push_back(stage);
+    stage = Stage();
+    stage = new_stage(*this, cap);
+  }
+  char* h = stage.h + stage.used;
   if (host && bytes)
     std::memcpy(h, host, bytes);
   else
     std::memset(h, 0, r);
+  void* d = stage.d + stage.used;
   stage.used += r;
-  void* d = alloc.alloc(r);
-  HIP_OK(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, stream));
-  // the device copy is returned to the pool right away: later users of the
-  // same memory are ordered after the kernels that read it (single stream)
-  transient.push_back(d);
   return d;
 }
 
-void Context::stage_reset() { stage.used = 0; }
+void Context::stage_flush() {
+  if (stage.used == stage.sent) return;
+  HIP_OK(hipMemcpyAsync(stage.d + stage.sent, stage.h + stage.sent, stage.used - stage.sent, hipMemcpyHostToDevice,
+                        stream));
+  stage.sent = stage.used;
+}
+
+void* Context::upload(const void* host, size_t bytes) {
+  void* d = stage_put(host, bytes);
+  stage_flush();
+  return d;
+}
+
+void Context::stage_reset() {
+  for (Stage& o : stage_old) {
+    (void)hipFree(o.d);
+    (void)hipHostFree(o.h);
+  }
+  stage_old.clear();
+  stage.used = stage.sent = 0;
+}
+
+void Context::stage_trim() {
+  if (stage_old.empty() && 2 * stage.used <= stage.cap) return;
+  HIP_OK(hipStreamSynchronize(stream));
+  release_transients();
+  stage_reset();
+}
 
 void Context::release_transients() {
   for (void* p : transient) alloc.release(p);
@@ -628,6 +665,7 @@ void run_heff(Context& c, const HeffPlan& p, int prec = DMRJ_PREC_F64) {
 // topology matches (same kernels, new arguments), else re-instantiated.
 template <class F>
 void run_captured(Context& c, F&& body, double flops, int slot = 0) {
+  c.stage_flush();  // tables are not part of the graph
   HIP_OK(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
   try {
     body();
@@ -929,16 +967,23 @@ EnvPlan plan_right(Context& c, const EnvMeta& R, const double* Rd, const SiteMet
 }
 
 void run_env(Context& c, EnvPlan& p) {
-  launch_gemm_arith(c, p.t1, p.s1, -1, c.env_prec);
-  launch_mix(c, p.md, p.mt);
-  launch_gemm_arith(c, p.t3, p.s3, -1, c.env_prec);
+  // the tables of the three launches go over in one copy (a left and a right
+  // update of m = 16 Heisenberg environments: 62 us with one copy per launch,
+  // 31 with this; Hubbard m = 1024: 232 and 182)
+  const GemmPrep g1 = prepare_gemm_arith(c, p.t1, p.s1, -1, c.env_prec);
+  const MixLaunch m = prepare_mix(c, p.md, p.mt);
+  const GemmPrep g3 = prepare_gemm_arith(c, p.t3, p.s3, -1, c.env_prec);
+  issue_gemm_arith(c, g1);
+  issue_mix_timed(c, m);
+  issue_gemm_arith(c, g3);
   c.flops_env += p.flops;
   c.alloc.release(p.X);
   c.alloc.release(p.Y);
 }
 
 // ================================================================ theta = AL*AR
-dmrj_tensor* make_theta(Context& c, const Tensor& AL, const Tensor& AR) {
+// prep: the product's launch is only prepared, for the caller to issue
+dmrj_tensor* make_theta(Context& c, const Tensor& AL, const Tensor& AR, GemmPrep* prep = nullptr) {
   if (AL.kind != 0 || AR.kind != 0 || AL.site.d1 != 0 || AR.site.d1 != 0)
     throw Error(DMRJ_ERR_ARG, "theta2 needs two MPS tensors");
   const SiteMeta& L = AL.site;
@@ -984,7 +1029,10 @@ dmrj_tensor* make_theta(Context& c, const Tensor& AL, const Tensor& AR) {
     bm.add(t->data, m.size, true);
     complexify_gemm(tasks, segs, bm);
   }
-  launch_gemm(c, tasks, segs, -1);
+  if (prep)
+    *prep = prepare_gemm_arith(c, tasks, segs, -1, 0);
+  else
+    launch_gemm(c, tasks, segs, -1);
   return t;
 }
 
@@ -1002,7 +1050,8 @@ dmrj_tensor* lanczos2(Context& c, const Tensor& L, const Tensor& R, const Tensor
   const bool correct = (precision & DMRJ_PREC_CORRECT) != 0;
   if (L.kind != 1 || R.kind != 2) throw Error(DMRJ_ERR_ARG, "lanczos2: bad environment handles");
   if (L.cplx || R.cplx || AL.cplx || AR.cplx) throw Error(DMRJ_ERR_ARG, "lanczos2 takes real tensors");
-  dmrj_tensor* th = make_theta(c, AL, AR);
+  GemmPrep theta;
+  dmrj_tensor* th = make_theta(c, AL, AR, &theta);
   const SiteMeta& x = th->site;
   const int64_t n = x.size;
   FusedMpo f = fuse_two(W1, W2);
@@ -1021,6 +1070,7 @@ dmrj_tensor* lanczos2(Context& c, const Tensor& L, const Tensor& R, const Tensor
     h3 = prepare_heff(c, p, DMRJ_PREC_F64);          // H AA' in FP64
   }
   const bool graph = c.graph_mode != 0;
+  issue_gemm_arith(c, theta);
   auto step = [&]() {
     issue_heff(c, h1, !graph);
     {
@@ -1579,10 +1629,11 @@ double read_scalar(Context& c, int slot) {
 }
 
 template <class F>
-int guard(dmrj_ctx* ctx, F&& f) {
+int guard(dmrj_ctx* ctx, F&& f, bool trim = true) {
   if (!ctx) return DMRJ_ERR_ARG;
   try {
     HIP_OK(hipSetDevice(ctx->device));
+    if (trim) ctx->stage_trim();
     f();
     return DMRJ_OK;
   } catch (const Error& e) {
@@ -1664,8 +1715,6 @@ int dmrj_ctx_create(int device, dmrj_ctx** out) {
     HIP_OK(hipHostMalloc((void**)&c->hscal, S_COUNT * sizeof(double), hipHostMallocDefault));
     HIP_OK(hipMalloc((void**)&c->partial, 4 * kDotPartials * sizeof(double)));
     c->noalloc = noalloc_scratch(device);
-    c->stage.cap = 8 << 20;
-    HIP_OK(hipHostMalloc((void**)&c->stage.base, c->stage.cap, hipHostMallocDefault));
     for (auto& e : c->graph_done) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   } catch (const Error& e) {
     delete c;
@@ -1694,7 +1743,11 @@ int dmrj_ctx_destroy(dmrj_ctx* c) {
   if (c->partial) (void)hipFree(c->partial);
   if (c->hscal) (void)hipHostFree(c->hscal);
   if (c->hsig) (void)hipHostFree(c->hsig);
-  if (c->stage.base) (void)hipHostFree(c->stage.base);
+  c->stage_old.push_back(c->stage);
+  for (Stage& o : c->stage_old) {
+    if (o.d) (void)hipFree(o.d);
+    if (o.h) (void)hipHostFree(o.h);
+  }
   c->alloc.trim();
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -2475,7 +2528,7 @@ int dmrj_dots_noalloc(dmrj_ctx* c, int npairs, const dmrj_tensor* const* xs, con
       const double* yp[1] = {ys[p]->data};
       launch_dots_buf(*c, 1, xp, yp, xs[p]->nstore(), out_dev + p, c->noalloc + (int64_t)p * kDotPartials);
     }
-  });
+  }, false);  // stages nothing and may be under the caller's capture: no synchronisation
 }
 
 int dmrj_site_apply_op(dmrj_ctx* c, const dmrj_tensor* A, const double* op, const int32_t* dqL, const int32_t* dqR,

@@ -387,25 +387,40 @@ void issue_gemm(Context& c, const GemmLaunch& g) {
     issue_gemm_f64(c, g);
 }
 
-void launch_gemm_arith(Context& c, const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs, int cfg,
-                       int arith) {
-  if (tasks.empty()) return;
+GemmPrep prepare_gemm_arith(Context& c, const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs,
+                            int cfg, int arith) {
+  GemmPrep p;
+  if (tasks.empty()) return p;
   if (cfg < 0) cfg = pick_gemm_cfg(c, tasks, segs, arith);
   if (arith == 0) c.last_gemm_cfg = cfg;
-  GemmLaunch g = prepare_gemm(c, tasks, segs, cfg, arith);
-  if (g.ntiles == 0) return;
+  p.g = prepare_gemm(c, tasks, segs, cfg, arith);
+  if (c.prof) {
+    p.flops = gemm_flops(tasks, segs);
+    p.bytes = gemm_bytes(tasks, segs);
+  }
+  return p;
+}
+
+void issue_gemm_arith(Context& c, const GemmPrep& p) {
+  if (p.g.ntiles == 0) return;
   // one-kernel forms are timed by their own dispatch (hipExtLaunchKernelGGL
   // events); the FP16 form (scale pre-pass + GEMM) by events around both
+  const int arith = p.g.arith;
   const int kind = arith == 1 ? KIND_GEMM_LP : (arith == 2 ? KIND_GEMM_F16 : KIND_GEMM_F64);
   if (arith == 2) {
     const int ps = c.prof_begin();
-    issue_gemm(c, g);
-    if (ps >= 0) c.prof_end(ps, kind, gemm_flops(tasks, segs), gemm_bytes(tasks, segs));
+    issue_gemm(c, p.g);
+    if (ps >= 0) c.prof_end(ps, kind, p.flops, p.bytes);
   } else {
     const int ps = c.prof_begin_ext();
-    issue_gemm(c, g);
-    c.prof_end_ext(ps, kind, gemm_flops(tasks, segs), gemm_bytes(tasks, segs));
+    issue_gemm(c, p.g);
+    c.prof_end_ext(ps, kind, p.flops, p.bytes);
   }
+}
+
+void launch_gemm_arith(Context& c, const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs, int cfg,
+                       int arith) {
+  issue_gemm_arith(c, prepare_gemm_arith(c, tasks, segs, cfg, arith));
 }
 
 }  // namespace dmrj

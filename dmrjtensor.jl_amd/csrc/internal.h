@@ -178,9 +178,13 @@ struct Allocator {
   ~Allocator();
 };
 
-struct HostStage {   // pinned staging memory for plan uploads
-  char* base = nullptr;
-  size_t cap = 0, used = 0;
+// Staging memory for plan tables: a pinned host block and its device mirror.
+// Tables are written at the same offset of both; everything put since the
+// last flush goes over in one copy.
+struct Stage {
+  char* h = nullptr;
+  char* d = nullptr;
+  size_t cap = 0, used = 0, sent = 0;
 };
 
 struct Context {
@@ -198,8 +202,9 @@ struct Context {
   // per sector (dmrj_ctx_set_eig_batching)
   int eig_batching = 1;
   Allocator alloc;
-  HostStage stage;
-  std::vector<void*> transient;  // device copies of plan tables, freed at sync points
+  Stage stage;
+  std::vector<Stage> stage_old;  // full blocks whose tables may still be in use
+  std::vector<void*> transient;  // device scratch of prepared launches, freed at sync points
   std::string err;
   double* scal = nullptr;       // device scalars for Lanczos
   double* hscal = nullptr;      // pinned mirror
@@ -272,8 +277,20 @@ struct Context {
   int prof_begin_ext();
   void prof_end_ext(int slot, int kind, double flops, double bytes);
   void prof_resolve();                             // after a stream sync
-  void* upload(const void* host, size_t bytes);   // staged async copy, returns device ptr
+  // Device address of a copy of a host table.  stage_put only writes it to the
+  // staging block: it is on the device once stage_flush has been called, which
+  // every issue_* / launch_* helper does before its kernel, so the tables of
+  // launches prepared together share one copy (a copy is a 2.7 us kernel of
+  // its own on the stream: 35 of them were 96 of 670 us of a bond step with
+  // sectors up to 55).  upload = put and flush.  Tables stay valid until
+  // stage_reset, which follows a synchronisation of the stream.
+  void* stage_put(const void* host, size_t bytes);
+  void stage_flush();
+  void* upload(const void* host, size_t bytes);
   void stage_reset();
+  // Called where a library call begins: bounds the staging memory by
+  // synchronising when more than half a block is in use.
+  void stage_trim();
   void release_transients();
 };
 
@@ -408,8 +425,10 @@ struct QjBatch {
   Context& c;
   std::vector<QjSector> sec;
   std::vector<QjJob> jobs;
+  QjJob* dj = nullptr;  // device job table
   double* work = nullptr;
   int* ints = nullptr;
+  int64_t nn = 0, nd = 0;  // doubles of work: column norms of all sectors, matrices
   const bool cplx;
   QjBatch(Context& c_, bool cplx_) : c(c_), cplx(cplx_) {}
   QjBatch(const QjBatch&) = delete;
@@ -417,6 +436,7 @@ struct QjBatch {
   ~QjBatch();
 };
 bool qj_fits(int64_t R, int64_t C, bool cplx);  // sector sizes the register-resident kernels take
+void qj_prepare(QjBatch& q);
 bool qj_solve(QjBatch& q, double norm2);
 void qj_vectors(QjBatch& q);
 
@@ -444,6 +464,15 @@ void launch_aug_extract_z(Context& c, const std::vector<AugJobZ>& jobs);
 void launch_gemm(Context& c, const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs,
                  int cfg);
 void launch_mix(Context& c, const std::vector<MixDst>& dsts, const std::vector<MixTerm>& terms);
+// Block copies: tables prepared first, or prepared and launched.
+struct CopyLaunch {
+  const CopyWork* work = nullptr;
+  const CopyOp* ops = nullptr;
+  int nwork = 0, grid = 0;
+  double bytes = 0.0;
+};
+CopyLaunch prepare_copy(Context& c, const std::vector<CopyOp>& ops);
+void issue_copy(Context& c, const CopyLaunch& l);
 void launch_copy(Context& c, const std::vector<CopyOp>& ops);
 void launch_fill(Context& c, double* p, int64_t n, double v);
 void launch_marker(Context& c, int id);
@@ -552,7 +581,15 @@ double gemm_bytes(const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>
 int autotune_gemm(Context& c, const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs, int arith);
 // override > autotuner > heuristic
 int pick_gemm_cfg(Context& c, const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs, int arith);
-// one grouped GEMM in the given arithmetic (tile shape picked when cfg < 0)
+// One grouped GEMM in the given arithmetic (tile shape picked when cfg < 0):
+// prepared (tables staged), issued later, or both at once.
+struct GemmPrep {
+  GemmLaunch g;
+  double flops = 0.0, bytes = 0.0;  // (only while profiling)
+};
+GemmPrep prepare_gemm_arith(Context& c, const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs,
+                            int cfg, int arith);
+void issue_gemm_arith(Context& c, const GemmPrep& p);
 void launch_gemm_arith(Context& c, const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs, int cfg,
                        int arith);
 // Descriptor tables of one mix launch, already on the device.
@@ -565,6 +602,7 @@ struct MixLaunch {
 };
 MixLaunch prepare_mix(Context& c, const std::vector<MixDst>& dsts, const std::vector<MixTerm>& terms);
 void issue_mix(Context& c, const MixLaunch& m);
+void issue_mix_timed(Context& c, const MixLaunch& m);
 struct SmallSvdJob {
   const double* M;
   double* U;
@@ -610,9 +648,9 @@ __device__ __forceinline__ double ld_global(const double* p) {
 
 // The host arrays of one launch (tile list, tasks, segments, work lists,
 // FP16 plane tables) packed into one blob, each at a 256-byte aligned offset,
-// so that they reach the device in a single staged copy instead of one per
-// array.  add() returns an array's byte offset in the blob; commit() uploads
-// the blob once and returns its device address.
+// so that they are staged together.  add() returns an array's byte offset in
+// the blob; commit() puts the blob into the staging block and returns its
+// device address (valid on the device after the next stage_flush).
 struct UploadPack {
   std::vector<char> blob;
   size_t add(const void* p, size_t bytes) {
@@ -621,7 +659,7 @@ struct UploadPack {
     if (p && bytes) std::memcpy(blob.data() + o, p, bytes);
     return o;
   }
-  char* commit(Context& c) { return (char*)c.upload(blob.data(), blob.size()); }
+  char* commit(Context& c) { return (char*)c.stage_put(blob.data(), blob.size()); }
 };
 
 }  // namespace dmrj

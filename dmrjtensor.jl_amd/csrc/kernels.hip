@@ -810,6 +810,7 @@ int gemm_occupancy_f64(int cfg) {
 
 void issue_gemm_f64(Context& c, const GemmLaunch& g) {
   if (g.ntiles <= 0) return;
+  c.stage_flush();
   switch (g.cfg) {
     case 0: gemm_f64_kernel_launch<32, 32>(c, g); break;
     case 1: gemm_f64_kernel_launch<64, 64>(c, g); break;
@@ -851,6 +852,7 @@ MixLaunch prepare_mix(Context& c, const std::vector<MixDst>& dsts, const std::ve
 
 void issue_mix(Context& c, const MixLaunch& m) {
   if (m.nwork <= 0) return;
+  c.stage_flush();
   hipLaunchKernelGGL(k_mix, dim3(m.grid), dim3(kThreads), 0, c.stream, m.work, m.nwork, m.dsts, m.terms);
   HIP_OK(hipGetLastError());
 }
@@ -868,38 +870,47 @@ void launch_marker(Context& c, int id) {
   HIP_OK(hipGetLastError());
 }
 
-void launch_mix(Context& c, const std::vector<MixDst>& dsts, const std::vector<MixTerm>& terms) {
-  MixLaunch m = prepare_mix(c, dsts, terms);
+void issue_mix_timed(Context& c, const MixLaunch& m) {
   if (m.nwork <= 0) return;
   const int ps = c.prof_begin();
   issue_mix(c, m);
   if (ps >= 0) c.prof_end(ps, KIND_MIX, m.flops, m.bytes);
 }
 
-void launch_copy(Context& c, const std::vector<CopyOp>& ops) {
-  if (ops.empty()) return;
+void launch_mix(Context& c, const std::vector<MixDst>& dsts, const std::vector<MixTerm>& terms) {
+  issue_mix_timed(c, prepare_mix(c, dsts, terms));
+}
+
+CopyLaunch prepare_copy(Context& c, const std::vector<CopyOp>& ops) {
+  CopyLaunch l;
   std::vector<CopyWork> work;
   for (size_t i = 0; i < ops.size(); ++i) {
     const int64_t n = (int64_t)ops[i].rows * ops[i].cols;
     for (int64_t e = 0; e < n; e += kMixChunk) work.push_back({(int)i, 0, e});
   }
-  if (work.empty()) return;
+  if (work.empty()) return l;
   UploadPack up;
   const size_t ow = up.add(work.data(), work.size() * sizeof(CopyWork));
   const size_t oo = up.add(ops.data(), ops.size() * sizeof(CopyOp));
   char* base = up.commit(c);
-  auto* dw = (CopyWork*)(base + ow);
-  auto* dops = (CopyOp*)(base + oo);
-  const int grid = (int)std::min<size_t>(work.size(), (size_t)c.num_cu * 8);
-  const int ps = c.prof_begin();
-  hipLaunchKernelGGL(k_copy, dim3(grid), dim3(kThreads), 0, c.stream, dw, (int)work.size(), dops);
-  HIP_OK(hipGetLastError());
-  if (ps >= 0) {
-    double bytes = 0.0;
-    for (const auto& o : ops) bytes += 8.0 * o.rows * (double)o.cols * (o.src ? 2.0 : 1.0);
-    c.prof_end(ps, KIND_COPY, 0.0, bytes);
-  }
+  l.work = (const CopyWork*)(base + ow);
+  l.ops = (const CopyOp*)(base + oo);
+  l.nwork = (int)work.size();
+  l.grid = (int)std::min<size_t>(work.size(), (size_t)c.num_cu * 8);
+  for (const auto& o : ops) l.bytes += 8.0 * o.rows * (double)o.cols * (o.src ? 2.0 : 1.0);
+  return l;
 }
+
+void issue_copy(Context& c, const CopyLaunch& l) {
+  if (l.nwork <= 0) return;
+  c.stage_flush();
+  const int ps = c.prof_begin();
+  hipLaunchKernelGGL(k_copy, dim3(l.grid), dim3(kThreads), 0, c.stream, l.work, l.nwork, l.ops);
+  HIP_OK(hipGetLastError());
+  if (ps >= 0) c.prof_end(ps, KIND_COPY, 0.0, l.bytes);
+}
+
+void launch_copy(Context& c, const std::vector<CopyOp>& ops) { issue_copy(c, prepare_copy(c, ops)); }
 
 void launch_fill(Context& c, double* p, int64_t n, double v) {
   if (n <= 0) return;

@@ -638,6 +638,7 @@ int gemm_occupancy_f16(int cfg) {
 
 void issue_gemm_f16_prep(Context& c, const GemmLaunch& g) {
   if (g.ntiles <= 0) return;
+  c.stage_flush();
   auto check = [] {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) throw Error(-3, std::string("HIP: ") + hipGetErrorString(e));
@@ -668,6 +669,7 @@ void issue_gemm_f16_prep(Context& c, const GemmLaunch& g) {
 
 void issue_gemm_f16_main(Context& c, const GemmLaunch& g) {
   if (g.ntiles <= 0) return;
+  c.stage_flush();
   if (g.presplit) {
     switch (g.cfg) {
       case 0: gemm_f16p_kernel_launch<32, 32>(c, g); break;
@@ -760,6 +762,7 @@ int gemm_occupancy_lp(int cfg) {
 
 void issue_gemm_lp(Context& c, const GemmLaunch& g) {
   if (g.ntiles <= 0) return;
+  c.stage_flush();
   switch (g.cfg) {
     case 0: gemm_lp_kernel_launch<32, 32>(c, g); break;
     case 1: gemm_lp_kernel_launch<64, 64>(c, g); break;

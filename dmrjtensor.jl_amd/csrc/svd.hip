@@ -209,6 +209,29 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     const double mm = (double)std::max(s.R, s.C), nn = (double)std::min(s.R, s.C);
     svd_flops += 4.0 * mm * nn * nn + 8.0 * nn * nn * nn;
   }
+  // larger sectors of the default backend and all complex ones: QR-preconditioned block Jacobi
+  // (svd_qrj.hip) for the vectors of the side that must come out orthonormal;
+  // the other factor by the grouped GEMM below.  Sectors it does not take
+  // (longer than its register-resident slabs, or not converged within its
+  // sweep limit) and tensors whose squared norm under- or overflows go to the
+  // eigensolves of the augmented matrices.
+  QjBatch qj(c, z);
+  if ((z || c.svd_backend == 0) && aa2 > 1e-305 && aa2 < 1e305) {
+    for (int si : order) {
+      Sec& s = secs[si];
+      if (s.kmin == 0 || is_small[si] || !qj_fits(s.R, s.C, z)) continue;
+      QjSector q;
+      q.M = s.M;
+      q.R = (int)s.R;
+      q.o = (int)(dir > 0 ? s.C : s.R);
+      q.n = (int)(dir > 0 ? s.R : s.C);
+      q.K = s.kmin;
+      q.dir = dir;
+      q.index = si;
+      qj.sec.push_back(q);
+    }
+    qj_prepare(qj);
+  }
   const bool small_on_side = launch_svd_small(c, small, small_lds);
   // every exit from here on, exceptions included, orders the main stream
   // after the side-stream kernel, so no later synchronisation of the main
@@ -331,37 +354,15 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       }
     }
   }
-  // large sectors of the default backend and all complex ones: QR-preconditioned block Jacobi
-  // (svd_qrj.hip) for the vectors of the side that must come out orthonormal;
-  // the other factor by the grouped GEMM below.  Sectors it does not take
-  // (longer than its register-resident slabs, or not converged within its
-  // sweep limit) and tensors whose squared norm under- or overflows go to the
-  // eigensolves of the augmented matrices.
-  QjBatch qj(c, z);
-  if ((z || c.svd_backend == 0) && aa2 > 1e-305 && aa2 < 1e305) {
-    for (int si : order) {
-      Sec& s = secs[si];
-      if (s.kmin == 0 || is_small[si] || !qj_fits(s.R, s.C, z)) continue;
-      QjSector q;
-      q.M = s.M;
-      q.R = (int)s.R;
-      q.o = (int)(dir > 0 ? s.C : s.R);
-      q.n = (int)(dir > 0 ? s.R : s.C);
-      q.K = s.kmin;
-      q.dir = dir;
-      q.index = si;
-      qj.sec.push_back(q);
+  if (!qj.sec.empty() && qj_solve(qj, aa2))
+    for (size_t b = 0; b < qj.sec.size(); ++b) {
+      Sec& s = secs[qj.sec[b].index];
+      s.qj = (int)b;
+      s.bj = 1;
+      is_small[qj.sec[b].index] = 1;  // handled
+      const double mm = (double)std::max(s.R, s.C), nn = (double)s.kmin;
+      svd_flops += 4.0 * mm * nn * nn + 8.0 * nn * nn * nn;
     }
-    if (!qj.sec.empty() && qj_solve(qj, aa2))
-      for (size_t b = 0; b < qj.sec.size(); ++b) {
-        Sec& s = secs[qj.sec[b].index];
-        s.qj = (int)b;
-        s.bj = 1;
-        is_small[qj.sec[b].index] = 1;  // handled
-        const double mm = (double)std::max(s.R, s.C), nn = (double)s.kmin;
-        svd_flops += 4.0 * mm * nn * nn + 8.0 * nn * nn * nn;
-      }
-  }
   // large sectors, backend 5: batched symmetric eigensolve of the Gram matrix
   // of the side that must come out orthonormal (M M^T for dir > 0, M^T M for
   // dir < 0: size n = R or C instead of R + C); eigenvalues sigma^2 carry an
@@ -829,13 +830,13 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     }
   }
   mid.finish();
+  // block-Jacobi sectors: normalised kept columns, then the other factor
+  // U^T M = D V^T (dir > 0) or M V = U D (dir < 0) in one grouped GEMM
+  BufMap planes;  // complex: the operands of those products
+  std::vector<BjGather> gat;
+  std::vector<GemmTask> tasks;
+  std::vector<GemmSeg> segs;
   {
-    // block-Jacobi sectors: normalised kept columns, then the other factor
-    // U^T M = D V^T (dir > 0) or M V = U D (dir < 0) in one grouped GEMM
-    BufMap planes;  // complex: the operands of those products
-    std::vector<BjGather> gat;
-    std::vector<GemmTask> tasks;
-    std::vector<GemmSeg> segs;
     int64_t hoff = 0;
     for (int si : order) {
       Sec& s = secs[si];
@@ -870,55 +871,8 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       }
       hoff += s.kmin;
     }
-    launch_bj_gather(c, gat);
-    qj_vectors(qj);
-    // canonical factor: kept vectors of singular values below 1e-2 sigma_max
-    // (extracted vectors are orthogonal to the rest only to about
-    // eps sigma_max / sigma, so those above stay within ~1e-14; not in Gram
-    // sectors, whose factor is a set of eigenvectors) re-orthonormalised in
-    // place, then an orthonormal
-    // completion for numerically zero singular values (sigma <= 1e-10
-    // sigma_max); the latter carry no weight
-    double smax = 0.0;
-    for (int64_t i = 0; i < n; ++i) smax = std::max(smax, ents[i].v);
-    const double szero = 1e-10 * smax;
-    const double ssmall = 1e-2 * smax;
-    std::vector<CompleteJob> cj, rj;
-    hoff = 0;
-    for (int si : order) {
-      Sec& s = secs[si];
-      if (s.keep > 0) {
-        int c0 = s.keep;
-        while (c0 > 0 && hs[hoff + c0 - 1] <= szero) --c0;
-        int c1 = c0;
-        if (!s.gram && s.qj < 0)  // Gram eigenvectors and Jacobi columns need no re-orthonormalisation
-          while (c1 > 1 && hs[hoff + c1 - 1] < ssmall) --c1;
-        const int nv = (int)(dir > 0 ? s.R : s.C);
-        if (c1 < c0 && c1 >= 1) {
-          if (dir > 0)
-            rj.push_back({s.U, s.R, 1, nv, c1, c0});
-          else
-            rj.push_back({s.Vt, 1, s.kmin, nv, c1, c0});
-        }
-        if (c0 < s.keep) {
-          if (dir > 0)
-            cj.push_back({s.U, s.R, 1, nv, c0, s.keep});
-          else
-            cj.push_back({s.Vt, 1, s.kmin, nv, c0, s.keep});
-        }
-      }
-      hoff += s.kmin;
-    }
-    if (!z) {
-      reorth_basis(c, rj);
-      complete_basis(c, cj);
-    }
-    if (z) complexify_gemm(tasks, segs, planes);
-    launch_gemm(c, tasks, segs, -1);
   }
-  double* dscal = (double*)c.alloc.alloc(std::max<size_t>(1, scal.size()) * sizeof(double));
-  HIP_OK(hipMemcpyAsync(dscal, scal.data(), std::max<size_t>(1, scal.size()) * sizeof(double),
-                        hipMemcpyHostToDevice, c.stream));
+  const double* dscal = (const double*)c.stage_put(scal.data(), scal.size() * sizeof(double));
   auto* tl = new_tensor(c, 0);
   auto* tr = new_tensor(c, 0);
   tl->nq = tr->nq = AA.nq;
@@ -970,7 +924,56 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
                        s.keep, T.dim[b.b], dir > 0 && !s.bj ? dscal + soff[qidx[Q]] : nullptr, nullptr,
                        dir > 0 && s.bj ? renorm : 1.0});
   }
-  launch_copy(c, split);
+  if (z) complexify_gemm(tasks, segs, planes);
+  const GemmPrep gp = prepare_gemm_arith(c, tasks, segs, -1, 0);
+  const CopyLaunch sp = prepare_copy(c, split);
+  {
+    launch_bj_gather(c, gat);
+    qj_vectors(qj);
+    // canonical factor: kept vectors of singular values below 1e-2 sigma_max
+    // (extracted vectors are orthogonal to the rest only to about
+    // eps sigma_max / sigma, so those above stay within ~1e-14; not in Gram
+    // sectors, whose factor is a set of eigenvectors) re-orthonormalised in
+    // place, then an orthonormal
+    // completion for numerically zero singular values (sigma <= 1e-10
+    // sigma_max); the latter carry no weight
+    double smax = 0.0;
+    for (int64_t i = 0; i < n; ++i) smax = std::max(smax, ents[i].v);
+    const double szero = 1e-10 * smax;
+    const double ssmall = 1e-2 * smax;
+    std::vector<CompleteJob> cj, rj;
+    int64_t hoff = 0;
+    for (int si : order) {
+      Sec& s = secs[si];
+      if (s.keep > 0) {
+        int c0 = s.keep;
+        while (c0 > 0 && hs[hoff + c0 - 1] <= szero) --c0;
+        int c1 = c0;
+        if (!s.gram && s.qj < 0)  // Gram eigenvectors and Jacobi columns need no re-orthonormalisation
+          while (c1 > 1 && hs[hoff + c1 - 1] < ssmall) --c1;
+        const int nv = (int)(dir > 0 ? s.R : s.C);
+        if (c1 < c0 && c1 >= 1) {
+          if (dir > 0)
+            rj.push_back({s.U, s.R, 1, nv, c1, c0});
+          else
+            rj.push_back({s.Vt, 1, s.kmin, nv, c1, c0});
+        }
+        if (c0 < s.keep) {
+          if (dir > 0)
+            cj.push_back({s.U, s.R, 1, nv, c0, s.keep});
+          else
+            cj.push_back({s.Vt, 1, s.kmin, nv, c0, s.keep});
+        }
+      }
+      hoff += s.kmin;
+    }
+    if (!z) {
+      reorth_basis(c, rj);
+      complete_basis(c, cj);
+    }
+    issue_gemm_arith(c, gp);
+    issue_copy(c, sp);
+  }
   for (auto& s : secs) {
     c.alloc.release(s.M);
     c.alloc.release(s.U);
@@ -986,7 +989,6 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   c.alloc.release(gramE);
   c.alloc.release(graminfo);
   c.alloc.release(info);
-  c.alloc.release(dscal);
   res.L = tl;
   res.R = tr;
   return res;

@@ -963,20 +963,14 @@ QjBatch::~QjBatch() {
   c.alloc.release(ints);
 }
 
-// Factorisations, Jacobi sweeps and column norms of all sectors; sigma and
-// col of every sector receive the column norms (unscaled) in descending order
-// and the column each belongs to.  Returns false when a sector did not
-// converge within the sweep limit.
-bool qj_solve(QjBatch& q, double norm2) {
+// Orders the sectors, allocates and stages the job table.
+void qj_prepare(QjBatch& q) {
+  if (q.sec.empty()) return;
   Context& c = q.c;
   std::vector<QjSector>& sec = q.sec;
   const int nj = (int)sec.size();
   // largest first: a launch's grid covers the jobs that still take part
   std::stable_sort(sec.begin(), sec.end(), [](const QjSector& a, const QjSector& b) { return a.o > b.o; });
-  // powers of two, exact: norms of order one whatever the tensor's scale
-  int ex = 0;
-  (void)std::frexp(std::sqrt(norm2), &ex);
-  const double scale = std::ldexp(1.0, -ex);
   // doubles: the norms of all sectors (one copy to the host), then the
   // matrices; ints: the round counters of all sectors, then the orders
   const bool z = q.cplx;
@@ -995,9 +989,9 @@ bool qj_solve(QjBatch& q, double norm2) {
   }
   q.work = (double*)c.alloc.alloc((nn + nd) * sizeof(double));
   q.ints = (int*)c.alloc.alloc(ni * sizeof(int));
-  launch_fill(c, q.work + nn, nd, 0.0);
+  q.nn = nn;
+  q.nd = nd;
   q.jobs.resize(nj);
-  int maxo = 0, maxn = 0, maxK = 0;
   for (int j = 0; j < nj; ++j) {
     QjJob& b = q.jobs[j];
     const QjSector& s = sec[j];
@@ -1018,11 +1012,33 @@ bool qj_solve(QjBatch& q, double norm2) {
     b.n = s.n;
     b.K = s.K;
     b.dir = s.dir;
+  }
+  q.dj = (QjJob*)c.stage_put(q.jobs.data(), nj * sizeof(QjJob));
+}
+
+// Factorisations, Jacobi sweeps and column norms of all sectors; sigma and
+// col of every sector receive the column norms (unscaled) in descending order
+// and the column each belongs to.  Returns false when a sector did not
+// converge within the sweep limit.
+bool qj_solve(QjBatch& q, double norm2) {
+  Context& c = q.c;
+  std::vector<QjSector>& sec = q.sec;
+  const int nj = (int)sec.size();
+  // powers of two, exact: norms of order one whatever the tensor's scale
+  int ex = 0;
+  (void)std::frexp(std::sqrt(norm2), &ex);
+  const double scale = std::ldexp(1.0, -ex);
+  const bool z = q.cplx;
+  const int64_t nn = q.nn;
+  int maxo = 0, maxn = 0, maxK = 0;
+  for (const QjSector& s : sec) {
     maxo = std::max(maxo, s.o);
     maxn = std::max(maxn, s.n);
     maxK = std::max(maxK, s.K);
   }
-  auto* dj = (QjJob*)c.upload(q.jobs.data(), nj * sizeof(QjJob));
+  QjJob* dj = q.dj;
+  c.stage_flush();
+  launch_fill(c, q.work + nn, q.nd, 0.0);
   const int pk = up16(maxK) / 16;
   hipLaunchKernelGGL(k_qj_norms0, dim3((maxo + 63) / 64, nj), dim3(256), 0, c.stream, dj);
   hipLaunchKernelGGL(k_qj_rank, dim3((maxo + 255) / 256, nj), dim3(256), 0, c.stream, dj);
@@ -1097,7 +1113,7 @@ bool qj_solve(QjBatch& q, double norm2) {
   HIP_OK(hipStreamSynchronize(c.stream));
   for (int j = 0; j < nj; ++j) {
     QjSector& s = sec[j];
-    const double* v = h + nof[j];
+    const double* v = h + (q.jobs[j].nrm - q.work);
     s.col.resize(up16(s.K));
     for (int i = 0; i < (int)s.col.size(); ++i) s.col[i] = i;
     std::stable_sort(s.col.begin(), s.col.end(), [&](int a, int b) { return v[a] > v[b]; });
@@ -1140,7 +1156,8 @@ void qj_vectors(QjBatch& q) {
     b.keep = s.keep;
     b.oplane = s.oplane;
   }
-  auto* dj = (QjJob*)c.upload(q.jobs.data(), nj * sizeof(QjJob));
+  auto* dj = (QjJob*)c.stage_put(q.jobs.data(), nj * sizeof(QjJob));
+  c.stage_flush();
   if (q.cplx)
     launch_back<true>(c, dj, maxn, dim3((maxkeep + 15) / 16, nj));
   else
