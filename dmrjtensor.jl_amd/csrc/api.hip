@@ -1154,60 +1154,31 @@ dmrj_tensor* krylov_expm(Context& c, const Tensor& L, const Tensor& R, const Ten
   double* w = (double*)c.alloc.alloc((size_t)nv * sizeof(double));
   double* xin = (double*)c.alloc.alloc((size_t)nv * sizeof(double));  // fixed input of the prepared H_eff
   double* sc = (double*)c.alloc.alloc(256 * sizeof(double));  // alpha[0..63], beta[64..127], work[128..]
-  double* gs = (double*)c.alloc.alloc((size_t)(2 * 64 * 256 + 128) * sizeof(double));  // CGS partials, coefs
-  launch_fill(c, sc, 256, 0.0);
-  // v0 = x / |x|
-  {
-    const double* xs[1] = {x.data};
-    launch_dots(c, 1, xs, xs, x.nstore(), c.scal + S_OC);
-    launch_lz_scalar(c, 0);
-    if (zv && !x.cplx) launch_fill(c, V + n, m.size, 0.0);
-    HIP_OK(hipMemcpyAsync(V, x.data, x.nstore() * sizeof(double), hipMemcpyDeviceToDevice, c.stream));
-    launch_scale_dev(c, V, ne, c.scal + S_INVOC);
-  }
+  double* gs = (double*)c.alloc.alloc((size_t)4 * 64 * kKrylovBlocks * sizeof(double));  // partial sums
   double *T1 = nullptr, *T3 = nullptr;
   const int zmask = zv ? ((L.cplx ? 1 : 0) | 2 | (R.cplx ? 4 : 0)) : 0;
-  HIP_OK(hipMemcpyAsync(xin, V, ne * sizeof(double), hipMemcpyDeviceToDevice, c.stream));
   HeffPlan p = plan_heff(c, m, xin, w, L.env, L.data, R.env, R.data, f, &T1, &T3, zmask);
   const HeffLaunch hl = prepare_heff(c, p, prec);  // descriptor tables stay valid until the final sync
+  launch_krylov_first(c, x.data, x.nstore(), ne, V, xin, sc);  // v_0 = x / |x|
   // the whole iteration is a fixed kernel sequence on device scalars: with
   // graphs on it is captured and launched as one graph
   const bool graph = c.graph_mode != 0;
-  // short vectors: everything after H_eff in one single-work-group launch,
-  // which also writes v_{j+1} into the fixed input buffer
-  const bool fused = ne <= kKrylovFusedMax;
+  // what follows an H_eff application, up to v_{j+1} in the fixed input
+  // buffer: one work-group for short vectors, else four launches
+  const bool fused = ne <= kKrylovTailMax;
   auto iterate = [&]() {
-  for (int j = 0; j < r; ++j) {
-    double* vj = V + (size_t)j * nv;
-    if (j > 0 && !fused) HIP_OK(hipMemcpyAsync(xin, vj, ne * sizeof(double), hipMemcpyDeviceToDevice, c.stream));
-    issue_heff(c, hl, !graph);
-    if (fused) {
-      launch_krylov_tail(c, V, nv, j, w, m.size, zv ? 1 : 0, sc, xin, j == r - 1 ? 1 : 0);
-      continue;
+    for (int j = 0; j < r; ++j) {
+      issue_heff(c, hl, !graph);
+      if (fused) {
+        launch_krylov_tail(c, V, nv, j, w, m.size, zv ? 1 : 0, sc, xin, j == r - 1 ? 1 : 0);
+      } else if (j < r - 1) {
+        launch_krylov_step(c, V, nv, j, w, m.size, zv ? 1 : 0, sc, xin, gs);
+      } else {  // alpha_j = Re <v_j, w> (real for a Hermitian H_eff)
+        const double* xs[1] = {V + (size_t)j * nv};
+        const double* ys[1] = {w};
+        launch_dots(c, 1, xs, ys, ne, sc + j);
+      }
     }
-    // alpha_j = Re <v_j, w> (real for a Hermitian H_eff)
-    {
-      const double* xs[1] = {vj};
-      const double* ys[1] = {w};
-      launch_dots(c, 1, xs, ys, ne, sc + j);
-    }
-    if (j == r - 1) break;
-    // w -= <v_i, w> v_i for all i <= j: two block passes of classical
-    // Gram-Schmidt (this removes alpha_j v_j and beta_{j-1} v_{j-1} as well)
-    for (int pass = 0; pass < 2; ++pass)
-      launch_cgs_pass(c, w, V, nv, m.size, j + 1, zv ? 1 : 0, gs, gs + 2 * 64 * 256);
-    {
-      const double* xs[1] = {w};
-      launch_dots(c, 1, xs, xs, ne, sc + 130);
-    }
-    // beta_j = |w|, v_{j+1} = w / beta_j (zero when the Krylov space is exhausted)
-    HIP_OK(hipMemcpyAsync(c.scal + S_PP, sc + 130, sizeof(double), hipMemcpyDeviceToDevice, c.stream));
-    launch_lz_scalar(c, 2);
-    HIP_OK(hipMemcpyAsync(sc + 64 + j, c.scal + S_B1, sizeof(double), hipMemcpyDeviceToDevice, c.stream));
-    double* vn = V + (size_t)(j + 1) * nv;
-    HIP_OK(hipMemcpyAsync(vn, w, ne * sizeof(double), hipMemcpyDeviceToDevice, c.stream));
-    launch_scale_dev(c, vn, ne, c.scal + S_INVB);
-  }
   };
   if (graph)
     run_captured(c, iterate, r * hl.flops_alg, slot);
@@ -1225,14 +1196,8 @@ dmrj_tensor* krylov_expm(Context& c, const Tensor& L, const Tensor& R, const Ten
   out->site = m;
   out->cplx = zout ? 1 : 0;
   alloc_data(c, *out);
-  if (!zv) {
-    launch_combine(c, out->data, V, n, m.size, dcoef, r);
-    if (zout) launch_combine(c, out->data + m.size, V, n, m.size, dcoef + r, r);
-  } else {
-    // planes of the Krylov basis: plane 2j = Re v_j, plane 2j+1 = Im v_j, stride n
-    launch_combine(c, out->data, V, n, m.size, dcoef, 2 * r);
-    launch_combine(c, out->data + m.size, V, n, m.size, dcoef + 2 * r, 2 * r);
-  }
+  // complex basis planes: plane 2j = Re v_j, plane 2j+1 = Im v_j, stride n
+  launch_combine(c, out->data, zout ? out->data + m.size : nullptr, V, n, m.size, dcoef, zv ? 2 * r : r);
   double hout[3] = {0.0, (double)r, 0.0};
   const bool need = energy != nullptr || kdim != nullptr;
   if (need) {

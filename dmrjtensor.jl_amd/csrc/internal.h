@@ -476,17 +476,18 @@ void issue_copy(Context& c, const CopyLaunch& l);
 void launch_copy(Context& c, const std::vector<CopyOp>& ops);
 void launch_fill(Context& c, double* p, int64_t n, double v);
 void launch_marker(Context& c, int id);
-// One block classical Gram-Schmidt pass: w -= sum_{i<k} <v_i, w> v_i (v_i at
-// V + i nv; complex: split planes of n elements).  partial: 2 k 256 doubles,
-// coef: 2 k doubles.
-void launch_cgs_pass(Context& c, double* w, const double* V, int64_t nv, int64_t n, int k, int cplx,
-                     double* partial, double* coef);
-// One Krylov iteration after the H_eff application in a single work-group
-// (alpha_j to sc[j]; unless last: two Gram-Schmidt passes against v_0..v_j,
-// beta_j to sc[64 + j], v_{j+1} to V and xin) for short vectors.
+// Krylov iteration: the first vector, and what follows an H_eff application
+// (alpha_j to sc[j], two Gram-Schmidt passes against v_0..v_j, beta_j to
+// sc[64 + j], v_{j+1} to V and xin); tail: one work-group, up to kKrylovTailMax
+// stored elements (last: alpha_j only); step: four launches, any length, work:
+// 256 kKrylovBlocks doubles.
+constexpr int64_t kKrylovTailMax = 4096;
+constexpr int kKrylovBlocks = 512;
+void launch_krylov_first(Context& c, const double* x, int64_t ns, int64_t ne, double* V, double* xin, double* sc);
 void launch_krylov_tail(Context& c, double* V, int64_t nv, int j, double* w, int64_t n, int cplx, double* sc,
                         double* xin, int last);
-constexpr int64_t kKrylovFusedMax = 16384;  // stored elements of a Krylov vector for the one-work-group path
+void launch_krylov_step(Context& c, double* V, int64_t nv, int j, double* w, int64_t n, int cplx, double* sc,
+                        double* xin, double* work);
 constexpr int kDotPartials = 256;  // per-pair partial sums of launch_dots
 // launch_dots with the partials in `partial` (npairs * kDotPartials doubles)
 void launch_dots_buf(Context& c, int npairs, const double* const* xs, const double* const* ys, int64_t n,
@@ -498,7 +499,8 @@ void launch_scale_dev(Context& c, double* x, int64_t n, const double* coef);
 void launch_comb_dev(Context& c, double* out, const double* a, const double* b, int64_t n,
                      const double* ca, const double* cb);
 void launch_lz_scalar(Context& c, int stage);
-void launch_combine(Context& c, double* out, const double* V, int64_t ld, int64_t n, const double* coef, int k);
+void launch_combine(Context& c, double* out, double* out2, const double* V, int64_t ld, int64_t n,
+                    const double* coef, int k);
 // exp(pf T) e1 (or the lowest Ritz vector) coefficients of a Krylov space on
 // the device: sc = {alpha[0..64), beta[64..128)}; coef receives 2r (real
 // Krylov vectors) or 4r (complex) weights, outs {lowest Ritz value, k, flag}

@@ -232,9 +232,29 @@ struct DotArgs {
   const double* y[4];
 };
 
+__device__ inline double lane_get(double v, int i) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), i),
+                          __builtin_amdgcn_readlane(__double2loint(v), i));
+}
+
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+  return v + __hiloint2double(hi, lo);
+}
+
+// sum over the wave, in every lane: inside the rows of 16 lanes by shifts,
+// across them by broadcasts of their last lanes (six dependent additions of
+// VALU latency instead of six of LDS-permute latency)
 __device__ inline double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
+  v = dpp_add<0x111, 0xf>(v);
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);
+  v = dpp_add<0x143, 0xc>(v);
+  return lane_get(v, 63);
 }
 
 __global__ __launch_bounds__(kThreads) void k_dot_partial(DotArgs args, int64_t n, double* partial) {
@@ -271,189 +291,319 @@ __global__ __launch_bounds__(kThreads) void k_dot_final(const double* partial, d
   }
 }
 
-// Block classical Gram-Schmidt pass of the Krylov reorthogonalisation:
-// coef_i = <v_i, w> for all i < k in one pair of launches (deterministic
-// two-level reduction), then w -= sum_i coef_i v_i in one launch.  Real:
-// vectors of n elements.  Complex (split planes, stride nv >= 2n): <v, w> =
-// (vr.wr + vi.wi) + i (vr.wi - vi.wr) and w -= c v on both planes.
-__global__ __launch_bounds__(kThreads) void k_vdots_partial(const double* __restrict__ V, int64_t nv,
-                                                            const double* __restrict__ w, int64_t n, int cplx,
-                                                            double* __restrict__ partial) {
-  const double* __restrict__ v = V + (int64_t)blockIdx.y * nv;
-  double re = 0.0, im = 0.0;
-  for (int64_t e = blockIdx.x * (int64_t)kThreads + threadIdx.x; e < n; e += (int64_t)gridDim.x * kThreads) {
-    if (cplx) {
-      const double vr = v[e], vi = v[n + e], wr = w[e], wi = w[n + e];
-      re += vr * wr + vi * wi;
-      im += vr * wi - vi * wr;
-    } else {
-      re += v[e] * w[e];
-    }
-  }
-  __shared__ double red[2][kThreads / 64];
-  re = wave_sum(re);
-  im = wave_sum(im);
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x >> 6] = re;
-    red[1][threadIdx.x >> 6] = im;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double a = 0.0, b = 0.0;
-    for (int i = 0; i < kThreads / 64; ++i) {
-      a += red[0][i];
-      b += red[1][i];
-    }
-    const int64_t o = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 2;
-    partial[o] = a;
-    partial[o + 1] = b;
-  }
-}
-
-__global__ __launch_bounds__(kThreads) void k_vdots_final(const double* __restrict__ partial, int nblk,
-                                                          double* __restrict__ coef) {
-  const int i = blockIdx.x;
-  double re = 0.0, im = 0.0;
-  for (int b = threadIdx.x; b < nblk; b += kThreads) {
-    re += partial[((int64_t)i * nblk + b) * 2];
-    im += partial[((int64_t)i * nblk + b) * 2 + 1];
-  }
-  __shared__ double red[2][kThreads / 64];
-  re = wave_sum(re);
-  im = wave_sum(im);
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x >> 6] = re;
-    red[1][threadIdx.x >> 6] = im;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double a = 0.0, b = 0.0;
-    for (int t = 0; t < kThreads / 64; ++t) {
-      a += red[0][t];
-      b += red[1][t];
-    }
-    coef[2 * i] = a;
-    coef[2 * i + 1] = b;
-  }
-}
-
-__global__ void k_cgs_sub(double* __restrict__ w, const double* __restrict__ V, int64_t nv, int64_t n, int k,
-                          int cplx, const double* __restrict__ coef) {
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
-    double ar = 0.0, ai = 0.0;
-    for (int i = 0; i < k; ++i) {
-      const double* v = V + (int64_t)i * nv;
-      const double cr = coef[2 * i];
-      if (cplx) {
-        const double ci = coef[2 * i + 1], vr = v[e], vi = v[n + e];
-        ar += cr * vr - ci * vi;
-        ai += cr * vi + ci * vr;
-      } else {
-        ar += cr * v[e];
-      }
-    }
-    w[e] -= ar;
-    if (cplx) w[n + e] -= ai;
-  }
-}
-
-// One Krylov iteration after the H_eff application, in one work-group, for
-// short vectors (the latency of a dozen dependent launches dominates there):
-// alpha_j = Re <v_j, w> -> sc[j]; unless last: two classical Gram-Schmidt
-// passes of w against v_0..v_j (coefficients of a pass from the same w, then
-// one subtraction, as the multi-launch passes), beta_j = |w| -> sc[64 + j],
-// v_{j+1} = w / beta_j (zero when beta_j <= 1e-10) written to V and to the
+// ---------------------------------------------------------------- Krylov step
+// Everything between two H_eff applications of a Krylov iteration: alpha_j =
+// Re <v_j, w>, two classical Gram-Schmidt passes of w against v_0..v_j (the
+// coefficients of a pass from the same w, then one subtraction; alpha_j is the
+// real part of the first pass's last one), beta_j = |w|, v_{j+1} = w / beta_j
+// (zero when beta_j <= 1e-10, the space is exhausted), written to V and to the
 // fixed H_eff input xin.  Complex vectors: real plane then imaginary plane of
 // n elements each, <v, w> = sum conj(v) w.
-__global__ __launch_bounds__(kThreads) void k_krylov_tail(double* __restrict__ V, int64_t nv, int j,
-                                                          double* __restrict__ w, int64_t n, int cplx,
-                                                          double* __restrict__ sc, double* __restrict__ xin,
-                                                          int last) {
-  __shared__ double red[2][kThreads / 64];
-  __shared__ double coef[2 * 64];
-  const int tid = threadIdx.x;
-  const int64_t ne = cplx ? 2 * n : n;
-  auto block_sum2 = [&](double a, double b, double& A, double& B) {
-    a = wave_sum(a);
-    b = wave_sum(b);
-    if ((tid & 63) == 0) {
-      red[0][tid >> 6] = a;
-      red[1][tid >> 6] = b;
+//
+// A piece of w is held in LDS and every wave takes whole vectors of the basis
+// (several waves one vector when there are few), so a pass has one barrier
+// however many vectors there are.  One work-group up to 4096 stored elements
+// (complex two-site step at m = 12: 11.9 us with one barrier pair per vector,
+// 6.9 now), above that four launches (m = 96, 18432 complex elements: 57 us of
+// 16 launches before, 35 now).
+
+// acc[i P + part] (first piece: set, else add) = the dots of the m elements
+// from e0 of v_0..v_{k-1} with the piece wl (imaginary plane at wl + ldw)
+template <int NW>
+__device__ inline void krylov_dots(const double* __restrict__ V, int64_t nv, int64_t n, int cplx, int k,
+                                   const double* wl, int ldw, int64_t e0, int m, double2* acc, bool first) {
+  const int P = k < NW ? NW / k : 1, wv = threadIdx.x >> 6, part = wv % P, lane = threadIdx.x & 63;
+  for (int i = wv / P; i < k; i += NW / P) {
+    const double* v = V + (int64_t)i * nv + e0;
+    double re = 0.0, im = 0.0;
+    if (cplx) {
+#pragma unroll 4
+      for (int e = 64 * part + lane; e < m; e += 64 * P) {
+        const double vr = v[e], vi = v[n + e], wr = wl[e], wi = wl[ldw + e];
+        re += vr * wr + vi * wi;
+        im += vr * wi - vi * wr;
+      }
+      im = wave_sum(im);
+    } else {
+#pragma unroll 8
+      for (int e = 64 * part + lane; e < m; e += 64 * P) re += v[e] * wl[e];
     }
-    __syncthreads();
-    A = 0.0;
-    B = 0.0;
-    for (int i = 0; i < kThreads / 64; ++i) {
-      A += red[0][i];
-      B += red[1][i];
+    re = wave_sum(re);
+    if (lane == 0) {
+      double2* d = acc + i * P + part;
+      *d = first ? make_double2(re, im) : make_double2(d->x + re, d->y + im);
     }
-    __syncthreads();
-  };
-  double A, B;
-  {
-    const double* vj = V + (int64_t)j * nv;
-    double a = 0.0;
-    for (int64_t e = tid; e < ne; e += kThreads) a += vj[e] * w[e];
-    block_sum2(a, 0.0, A, B);
-    if (tid == 0) sc[j] = A;
   }
-  if (last) return;
-  for (int pass = 0; pass < 2; ++pass) {
-    for (int i = 0; i <= j; ++i) {
-      const double* v = V + (int64_t)i * nv;
-      double re = 0.0, im = 0.0;
-      for (int64_t e = tid; e < n; e += kThreads) {
-        if (cplx) {
-          const double vr = v[e], vi = v[n + e], wr = w[e], wi = w[n + e];
-          re += vr * wr + vi * wi;
-          im += vr * wi - vi * wr;
-        } else {
-          re += v[e] * w[e];
-        }
-      }
-      block_sum2(re, im, A, B);
-      if (tid == 0) {
-        coef[2 * i] = A;
-        coef[2 * i + 1] = B;
-      }
+}
+
+// element e of sum_i coef_i v_i
+__device__ inline double2 krylov_project(const double* __restrict__ V, int64_t nv, int64_t n, int cplx, int k,
+                                         const double2* coef, int64_t e) {
+  double ar = 0.0, ai = 0.0;
+  const double* v = V + e;
+  if (cplx) {
+#pragma unroll 4
+    for (int i = 0; i < k; ++i) {
+      const double vr = v[(int64_t)i * nv], vi = v[(int64_t)i * nv + n];
+      const double2 c = coef[i];
+      ar += c.x * vr - c.y * vi;
+      ai += c.x * vi + c.y * vr;
     }
-    __syncthreads();
-    for (int64_t e = tid; e < n; e += kThreads) {
-      double ar = 0.0, ai = 0.0;
-      for (int i = 0; i <= j; ++i) {
-        const double* v = V + (int64_t)i * nv;
-        const double cr = coef[2 * i];
-        if (cplx) {
-          const double ci = coef[2 * i + 1], vr = v[e], vi = v[n + e];
-          ar += cr * vr - ci * vi;
-          ai += cr * vi + ci * vr;
-        } else {
-          ar += cr * v[e];
-        }
-      }
-      w[e] -= ar;
-      if (cplx) w[n + e] -= ai;
-    }
-    __syncthreads();
+  } else {
+#pragma unroll 8
+    for (int i = 0; i < k; ++i) ar += coef[i].x * v[(int64_t)i * nv];
   }
+  return make_double2(ar, ai);
+}
+
+constexpr int kTailThreads = 1024;
+constexpr size_t kKrylovTailLds = 60 << 10;  // dynamic LDS of the one-work-group kernel
+
+// Short vectors: one launch of one work-group.  VL: the basis fits into LDS
+// beside w, so that the one memory latency of the kernel is that of all loads
+// at once.
+template <bool VL>
+__global__ __launch_bounds__(kTailThreads) void k_krylov_tail(double* __restrict__ Vg, int64_t nv, int j,
+                                                              const double* __restrict__ w, int64_t n, int cplx,
+                                                              double* __restrict__ sc, double* __restrict__ xin,
+                                                              int last) {
+  constexpr int NW = kTailThreads / 64;
+  extern __shared__ double wl[];
+  __shared__ double2 acc[64], coef[64];
+  __shared__ double red[NW];
+  const int tid = threadIdx.x, m = (int)n, ne = cplx ? 2 * m : m;
+  const int k = last ? 1 : j + 1;  // the last iteration only asks for alpha_j
+  const int P = k < NW ? NW / k : 1;
+  const double* B = last ? Vg + (int64_t)j * nv : Vg;
+  if constexpr (VL) {
+    for (int e = tid; e < ne; e += kTailThreads) {
+      wl[e] = w[e];
+#pragma unroll 8
+      for (int i = 0; i < k; ++i) wl[(i + 1) * ne + e] = B[(int64_t)i * nv + e];
+    }
+  } else {
+    for (int e = tid; e < ne; e += kTailThreads) wl[e] = w[e];
+  }
+  const double* V = VL ? wl + ne : B;
+  const int64_t ld = VL ? ne : nv;
+  __syncthreads();
   double s2 = 0.0;
-  for (int64_t e = tid; e < ne; e += kThreads) s2 += w[e] * w[e];
-  block_sum2(s2, 0.0, A, B);
-  const double b = sqrt(A);
+  for (int pass = 0; pass < 2; ++pass) {
+    krylov_dots<NW>(V, ld, m, cplx, k, wl, m, 0, m, acc, true);
+    __syncthreads();
+    if (tid < k) {
+      double2 t = acc[tid * P];
+      for (int q = 1; q < P; ++q) {
+        t.x += acc[tid * P + q].x;
+        t.y += acc[tid * P + q].y;
+      }
+      coef[tid] = t;
+      if (pass == 0 && tid == k - 1) sc[j] = t.x;
+    }
+    if (last) return;
+    __syncthreads();
+    for (int e = tid; e < m; e += kTailThreads) {
+      const double2 a = krylov_project(V, ld, m, cplx, k, coef, e);
+      const double x = wl[e] - a.x, y = cplx ? wl[m + e] - a.y : 0.0;
+      wl[e] = x;
+      if (cplx) wl[m + e] = y;
+      if (pass == 1) s2 += x * x + y * y;
+    }
+    if (pass == 0) __syncthreads();
+  }
+  s2 = wave_sum(s2);
+  if ((tid & 63) == 0) red[tid >> 6] = s2;
+  __syncthreads();
+  double t = 0.0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) t += red[i];
+  const double b = sqrt(t);
   const double invb = b > 1e-10 ? 1.0 / b : 0.0;
   if (tid == 0) sc[64 + j] = b;
-  double* vn = V + (int64_t)(j + 1) * nv;
-  for (int64_t e = tid; e < ne; e += kThreads) {
-    const double x = w[e] * invb;
+  double* vn = Vg + (int64_t)(j + 1) * nv;
+  for (int e = tid; e < ne; e += kTailThreads) {
+    const double x = wl[e] * invb;
     vn[e] = x;
     xin[e] = x;
   }
 }
 
+// Longer vectors: four launches over many work-groups, each of which owns the
+// same range of elements in all of them.  A launch starts by summing the
+// partial sums of the one before it (every work-group all of them, from L2):
+//   0: dots of w                                      -> pa
+//   1: coefficients from pa, subtract, dots of the new w -> pb
+//   2: coefficients from pb, subtract, squared norm   -> pa
+//   3: beta from pa, v_{j+1} and xin
+constexpr int kKrylovPiece = 1024;
+
+template <int STEP>
+__global__ __launch_bounds__(kThreads) void k_krylov_step(double* __restrict__ V, int64_t nv, int j,
+                                                          double* __restrict__ w, int64_t n, int cplx,
+                                                          double* __restrict__ sc, double* __restrict__ xin,
+                                                          const double2* __restrict__ pin,
+                                                          double2* __restrict__ pout) {
+  constexpr int NW = kThreads / 64;
+  __shared__ double wl[2 * kKrylovPiece];
+  __shared__ double2 acc[64], coef[64];
+  __shared__ double red[NW];
+  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, k = j + 1;
+  const int nblk = gridDim.x;
+  const int64_t per = ((n + nblk - 1) / nblk + 63) / 64 * 64;
+  const int64_t lo = min(n, blockIdx.x * per), hi = min(n, lo + per);
+  if constexpr (STEP == 1 || STEP == 2) {
+    for (int i = wv; i < k; i += NW) {
+      double re = 0.0, im = 0.0;
+      for (int b = lane; b < nblk; b += 64) {
+        const double2 p = pin[(int64_t)i * nblk + b];
+        re += p.x;
+        im += p.y;
+      }
+      re = wave_sum(re);
+      im = wave_sum(im);
+      if (lane == 0) coef[i] = make_double2(re, im);
+    }
+    __syncthreads();
+    if (STEP == 1 && blockIdx.x == 0 && tid == 0) sc[j] = coef[j].x;
+  }
+  if constexpr (STEP == 3) {
+    double t = 0.0;
+    for (int b = tid; b < nblk; b += kThreads) t += pin[b].x;
+    t = wave_sum(t);
+    if (lane == 0) red[wv] = t;
+    __syncthreads();
+    t = 0.0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) t += red[i];
+    const double b = sqrt(t);
+    const double invb = b > 1e-10 ? 1.0 / b : 0.0;
+    if (blockIdx.x == 0 && tid == 0) sc[64 + j] = b;
+    double* vn = V + (int64_t)(j + 1) * nv;
+    for (int64_t e = lo + tid; e < hi; e += kThreads) {
+      const double x = w[e] * invb;
+      vn[e] = x;
+      xin[e] = x;
+      if (cplx) {
+        const double y = w[n + e] * invb;
+        vn[n + e] = y;
+        xin[n + e] = y;
+      }
+    }
+    return;
+  }
+  double s2 = 0.0;
+  for (int64_t e0 = lo; e0 < hi; e0 += kKrylovPiece) {
+    const int m = (int)min((int64_t)kKrylovPiece, hi - e0);
+    if (e0 > lo) __syncthreads();
+    for (int e = tid; e < m; e += kThreads) {
+      double x = w[e0 + e], y = cplx ? w[n + e0 + e] : 0.0;
+      if constexpr (STEP != 0) {
+        const double2 a = krylov_project(V, nv, n, cplx, k, coef, e0 + e);
+        x -= a.x;
+        y -= a.y;
+        w[e0 + e] = x;
+        if (cplx) w[n + e0 + e] = y;
+        if (STEP == 2) s2 += x * x + y * y;
+      }
+      if constexpr (STEP != 2) {
+        wl[e] = x;
+        wl[kKrylovPiece + e] = y;
+      }
+    }
+    if constexpr (STEP != 2) {
+      __syncthreads();
+      krylov_dots<NW>(V, nv, n, cplx, k, wl, kKrylovPiece, e0, m, acc, e0 == lo);
+    }
+  }
+  __syncthreads();
+  if constexpr (STEP == 2) {
+    s2 = wave_sum(s2);
+    if (lane == 0) red[wv] = s2;
+    __syncthreads();
+    if (tid == 0) {
+      double t = 0.0;
+      for (int i = 0; i < NW; ++i) t += red[i];
+      pout[blockIdx.x] = make_double2(t, 0.0);
+    }
+  } else if (tid < k) {
+    const int P = k < NW ? NW / k : 1;
+    double2 t = make_double2(0.0, 0.0);
+    for (int q = 0; q < P && lo < hi; ++q) {
+      t.x += acc[tid * P + q].x;
+      t.y += acc[tid * P + q].y;
+    }
+    pout[(int64_t)tid * nblk + blockIdx.x] = t;
+  }
+}
+
+void launch_krylov_step(Context& c, double* V, int64_t nv, int j, double* w, int64_t n, int cplx, double* sc,
+                        double* xin, double* work) {
+  if (j < 0 || j >= 64) throw Error(-1, "krylov step: vector index out of range");
+  if (n <= 0) return;
+  const int nblk = (int)std::min<int64_t>(kKrylovBlocks, (n + kKrylovPiece - 1) / kKrylovPiece);
+  double2* pa = (double2*)work;
+  double2* pb = pa + 64 * kKrylovBlocks;
+  const dim3 g(nblk), t(kThreads);
+  hipLaunchKernelGGL(k_krylov_step<0>, g, t, 0, c.stream, V, nv, j, w, n, cplx, sc, xin, pb, pa);
+  hipLaunchKernelGGL(k_krylov_step<1>, g, t, 0, c.stream, V, nv, j, w, n, cplx, sc, xin, pa, pb);
+  hipLaunchKernelGGL(k_krylov_step<2>, g, t, 0, c.stream, V, nv, j, w, n, cplx, sc, xin, pb, pa);
+  hipLaunchKernelGGL(k_krylov_step<3>, g, t, 0, c.stream, V, nv, j, w, n, cplx, sc, xin, pa, pb);
+  HIP_OK(hipGetLastError());
+}
+
 void launch_krylov_tail(Context& c, double* V, int64_t nv, int j, double* w, int64_t n, int cplx, double* sc,
                         double* xin, int last) {
-  if (j < 0 || j >= 64) throw Error(-1, "krylov tail: vector index out of range");
-  hipLaunchKernelGGL(k_krylov_tail, dim3(1), dim3(kThreads), 0, c.stream, V, nv, j, w, n, cplx, sc, xin, last);
+  if (j < 0 || j >= 64 || (cplx ? 2 * n : n) > kKrylovTailMax)
+    throw Error(-1, "krylov tail: vector index or length out of range");
+  const size_t wb = (cplx ? 2 * n : n) * sizeof(double), vb = wb * (last ? 1 : j + 1);
+  const dim3 t(kTailThreads);
+  if (wb + vb <= kKrylovTailLds)
+    hipLaunchKernelGGL(k_krylov_tail<true>, dim3(1), t, wb + vb, c.stream, V, nv, j, w, n, cplx, sc, xin, last);
+  else
+    hipLaunchKernelGGL(k_krylov_tail<false>, dim3(1), t, wb, c.stream, V, nv, j, w, n, cplx, sc, xin, last);
+  HIP_OK(hipGetLastError());
+}
+
+// The first vector: V and xin = x / |x| (an imaginary plane of zeros when the
+// basis is complex and x is not: ne > ns), the scalars of the iteration
+// cleared.  NRM: |x|^2 of a short x by every work-group itself, else from *n2.
+template <bool NRM>
+__global__ __launch_bounds__(kTailThreads) void k_krylov_first(const double* __restrict__ x, int64_t ns, int64_t ne,
+                                                               const double* __restrict__ n2, double* __restrict__ V,
+                                                               double* __restrict__ xin, double* __restrict__ sc) {
+  __shared__ double red[kTailThreads / 64];
+  double t = 0.0;
+  if constexpr (NRM) {
+    for (int64_t e = threadIdx.x; e < ns; e += kTailThreads) t += x[e] * x[e];
+    t = wave_sum(t);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
+    __syncthreads();
+    t = 0.0;
+#pragma unroll
+    for (int i = 0; i < kTailThreads / 64; ++i) t += red[i];
+  } else {
+    t = *n2;
+  }
+  const double inv = 1.0 / sqrt(t);
+  for (int64_t e = blockIdx.x * (int64_t)kTailThreads + threadIdx.x; e < ne; e += (int64_t)gridDim.x * kTailThreads) {
+    const double v = e < ns ? x[e] * inv : 0.0;
+    V[e] = v;
+    xin[e] = v;
+  }
+  if (blockIdx.x == 0 && threadIdx.x < 256) sc[threadIdx.x] = 0.0;
+}
+
+void launch_krylov_first(Context& c, const double* x, int64_t ns, int64_t ne, double* V, double* xin, double* sc) {
+  const dim3 t(kTailThreads);
+  if (ne <= kKrylovTailMax) {
+    hipLaunchKernelGGL(k_krylov_first<true>, dim3(1), t, 0, c.stream, x, ns, ne, nullptr, V, xin, sc);
+  } else {
+    const double* xs[1] = {x};
+    launch_dots(c, 1, xs, xs, ns, c.scal + S_OC);
+    const int64_t g = std::min<int64_t>((ne + kTailThreads - 1) / kTailThreads, 4 * c.num_cu);
+    hipLaunchKernelGGL(k_krylov_first<false>, dim3((unsigned)g), t, 0, c.stream, x, ns, ne, c.scal + S_OC, V, xin,
+                       sc);
+  }
   HIP_OK(hipGetLastError());
 }
 
@@ -557,186 +707,156 @@ void launch_mfma_probe(Context& c, double* out) {
   HIP_OK(hipGetLastError());
 }
 
-// out[i] = sum_j c[j] * V[j*ld + i] (Krylov vector combination)
-__global__ void k_combine(double* out, const double* V, int64_t ld, int64_t n, const double* c, int k) {
+// out[i] = sum_j c[j] V[j ld + i]; with out2: out2[i] = sum_j c[k + j] V[j ld + i] beside it
+__global__ void k_combine(double* __restrict__ out, double* __restrict__ out2, const double* __restrict__ V,
+                          int64_t ld, int64_t n, const double* __restrict__ c, int k) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    double acc = 0.0;
-    for (int j = 0; j < k; ++j) acc += c[j] * V[(int64_t)j * ld + i];
-    out[i] = acc;
+    double a = 0.0, b = 0.0;
+#pragma unroll 4
+    for (int j = 0; j < k; ++j) {
+      const double v = V[(int64_t)j * ld + i];
+      a += c[j] * v;
+      if (out2) b += c[k + j] * v;
+    }
+    out[i] = a;
+    if (out2) out2[i] = b;
   }
 }
 
 // Coefficients of the Krylov exponential / Ritz vector on the device (one
 // wave; the Krylov dimension is at most 64, typically 2..12):
 //   k = the Krylov dimension used (first beta_j <= 1e-10 ends the space),
-//   T = Q diag(lam) Q^T by parallel-order Jacobi (FP64, the tridiagonal of
-//   alpha in sc[0..], beta in sc[64..]): each step rotates k/2 disjoint index
-//   pairs of a round-robin schedule at once (columns, then rows), k-1 steps
-//   per sweep, until the off-diagonal part is at the matrix's rounding level,
+//   T = Q diag(lam) Q^T by the QL algorithm with implicit shifts (FP64, the
+//   tridiagonal of alpha in sc[0..], beta in sc[64..]),
 //   c = Q exp(pf lam) Q^T e1 with the complex prefactor pf = (pf_re, pf_im),
 //   or (ritz) the eigenvector of the lowest lam signed to c_1 >= 0.
 // coef: real Krylov vectors: c_re[0..r), c_im[r..2r); complex Krylov vectors
 // (split planes, basis planes 2j = Re v_j, 2j+1 = Im v_j): the plane weights
 // of Re out in [0..2r) and of Im out in [2r..4r).  Entries j >= k are zero.
 // outs: {lowest Ritz value, k, 1 if an alpha/beta was non-finite}.
-// Dynamic LDS: 2 r^2 doubles (the matrix and its eigenvectors).
-__device__ inline void kc_pair(int n, int s, int i, int& p, int& q) {  // round robin of n (even) players
-  if (i == 0) {
-    p = s;
-    q = n - 1;
-  } else {
-    p = (s + i) % (n - 1);
-    q = (s - i + (n - 1)) % (n - 1);
-  }
-  if (p > q) {
-    const int t = p;
-    p = q;
-    q = t;
-  }
+//
+// Bound by the latency of the chain of plane rotations, about 0.85 k^2 of
+// them: diagonal and off-diagonal live in the lanes (entry i in lane i, read as
+// scalars), every lane runs the same chain and turns its own row of Q.  39 us
+// at k = 12 against 86 of a parallel-order Jacobi in LDS.
+__device__ inline double rsqrt_newton(double h) {
+  double y = __builtin_amdgcn_rsq(h);
+  y = fma(0.5 * y, fma(-h * y, y, 1.0), y);
+  return fma(0.5 * y, fma(-h * y, y, 1.0), y);
 }
 
 __global__ __launch_bounds__(64) void k_krylov_coef(const double* __restrict__ sc, int r, double pf_re,
                                                      double pf_im, int ritz, int zv, double* __restrict__ coef,
                                                      double* __restrict__ outs) {
-  extern __shared__ double kc_lds[];
-  __shared__ int sk, sbad, simin;
-  __shared__ double scs[32], ssn[32];
-  __shared__ int sp[32], sq[32];
+  __shared__ double Q[64 * 64];  // Q[i][t]: component t of eigenvector i
   const int t = threadIdx.x;
-  if (t == 0) {
-    int k = r, bad = 0;
-    for (int j = 0; j + 1 < r; ++j) {
-      if (!isfinite(sc[64 + j]) || !isfinite(sc[j])) bad = 1;
-      if (sc[64 + j] <= 1e-10) {
-        k = j + 1;
-        break;
-      }
-    }
-    sk = k;
-    sbad = bad;
-  }
-  __syncthreads();
-  const int k = sk, bad = sbad;
-  double* A = kc_lds;
-  double* Q = kc_lds + (int64_t)k * k;
-  for (int e = t; e < k * k; e += 64) {
-    A[e] = 0.0;
-    Q[e] = 0.0;
-  }
-  __syncthreads();
-  for (int i = t; i < k; i += 64) {
-    A[i + i * k] = sc[i];
-    if (i + 1 < k) A[i + (i + 1) * k] = A[(i + 1) + i * k] = sc[64 + i];
-    Q[i + i * k] = 1.0;
-  }
-  __syncthreads();
-  const int K = (k + 1) & ~1;  // even number of players; player k of an odd k is idle
-  const int npair = K / 2;
-  for (int sweep = 0; sweep < 100 && !bad && k > 1; ++sweep) {
-    double off = 0.0, dia = 0.0;  // off: both triangles
-    for (int e = t; e < k * k; e += 64) {
-      const double v = A[e];
-      if (e % k == e / k)
-        dia += v * v;
-      else
-        off += v * v;
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-      off += __shfl_xor(off, o, 64);
-      dia += __shfl_xor(dia, o, 64);
-    }
-    // lane 0's sums decide for all lanes (the butterfly may round differently
-    // per lane), so the loop and its barriers stay uniform
-    off = __shfl(off, 0, 64);
-    dia = __shfl(dia, 0, 64);
-    if (off <= 2e-30 * (dia + off) || off < 1e-300) break;
-    for (int st = 0; st < K - 1; ++st) {
-      if (t < npair) {
-        int p, q;
-        kc_pair(K, st, t, p, q);
-        double cs = 1.0, sn = 0.0;
-        if (q < k) {
-          const double apq = A[p + q * k];
-          if (apq != 0.0) {
-            const double app = A[p + p * k], aqq = A[q + q * k];
-            const double theta = (aqq - app) / (2.0 * apq);
-            const double tt = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-            cs = 1.0 / sqrt(tt * tt + 1.0);
-            sn = tt * cs;
+  double d = t < r ? sc[t] : 0.0, e = t + 1 < r ? sc[64 + t] : 0.0;
+  const unsigned long long ends = __ballot(t + 1 < r && e <= 1e-10);
+  const int k = ends ? __builtin_ctzll(ends) + 1 : r;
+  const bool bad = __ballot(t < k && t + 1 < r && (!isfinite(d) || !isfinite(e))) != 0;
+  if (t >= k) d = 0.0;
+  if (t + 1 >= k) e = 0.0;
+  for (int i = 0; i < k; ++i) Q[i * 64 + t] = i == t ? 1.0 : 0.0;
+  // a power of two that brings the largest entry to order one
+  double mx = fmax(fabs(d), fabs(e));
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+  int ex = 0;
+  if (mx > 0.0 && mx < 1e308) (void)frexp(mx, &ex);
+  ex = max(-1000, min(1000, ex));
+  d = ldexp(d, -ex);
+  e = ldexp(e, -ex);
+  for (int l = 0; l < k && !bad; ++l) {
+    for (int iter = 0; iter < 80; ++iter) {
+      // the block [l, m] ends at the first negligible coupling (a NaN ends it too)
+      const double dn = __shfl_down(d, 1, 64);
+      const unsigned long long neg =
+          __ballot(!(fabs(e) > 2.220446049250313e-16 * (fabs(d) + fabs(dn))) || t >= k - 1) >> l;
+      const int m = l + __builtin_ctzll(neg);
+      if (m == l) break;
+      const double dl = lane_get(d, l), el = lane_get(e, l);
+      double g = (lane_get(d, l + 1) - dl) / (2.0 * el);
+      g = lane_get(d, m) - dl + el / (g + copysign(sqrt(g * g + 1.0), g));
+      double s = 1.0, c = 1.0, p = 0.0, z = Q[m * 64 + t];
+      int i = m - 1;
+      for (; i >= l; --i) {
+        const double ei = lane_get(e, i), di = lane_get(d, i), dj = lane_get(d, i + 1), zi = Q[i * 64 + t];
+        const double f = s * ei, b = c * ei, h = f * f + g * g;
+        if (!(h > 1e-280)) {  // the rotation is undefined: the block splits here
+          if (t == i + 1) {
+            d = dj - p;
+            e = 0.0;
           }
+          Q[(i + 1) * 64 + t] = z;
+          break;
         }
-        sp[t] = p;
-        sq[t] = q;
-        scs[t] = cs;
-        ssn[t] = sn;
+        const double y = rsqrt_newton(h);
+        s = f * y;
+        c = g * y;
+        g = dj - p;
+        const double q = (di - g) * s + 2.0 * c * b;
+        p = s * q;
+        if (t == i + 1) {
+          d = g + p;
+          e = h * y;
+        }
+        g = c * q - b;
+        Q[(i + 1) * 64 + t] = s * zi + c * z;
+        z = c * zi - s * z;
       }
-      __syncthreads();
-      for (int e = t; e < npair * k; e += 64) {  // columns p, q of A and of Q
-        const int pi = e / k, rr = e % k;
-        const int p = sp[pi], q = sq[pi];
-        if (q >= k) continue;
-        const double cs = scs[pi], sn = ssn[pi];
-        double x = A[rr + p * k], y = A[rr + q * k];
-        A[rr + p * k] = cs * x - sn * y;
-        A[rr + q * k] = sn * x + cs * y;
-        x = Q[rr + p * k];
-        y = Q[rr + q * k];
-        Q[rr + p * k] = cs * x - sn * y;
-        Q[rr + q * k] = sn * x + cs * y;
+      if (t == m) e = 0.0;
+      if (i < l) {
+        Q[l * 64 + t] = z;
+        if (t == l) {
+          d = dl - p;
+          e = g;
+        }
       }
-      __syncthreads();
-      for (int e = t; e < npair * k; e += 64) {  // rows p, q of A
-        const int pi = e / k, rr = e % k;
-        const int p = sp[pi], q = sq[pi];
-        if (q >= k) continue;
-        const double cs = scs[pi], sn = ssn[pi];
-        const double x = A[p + rr * k], y = A[q + rr * k];
-        A[p + rr * k] = cs * x - sn * y;
-        A[q + rr * k] = sn * x + cs * y;
-      }
-      __syncthreads();
     }
   }
+  __syncthreads();
+  d = ldexp(d, ex);
+  // lowest value, the first of equal ones; not a number if any is not finite
+  double emin = t < k ? d : __builtin_inf();
+  int imin = t;
+  for (int o = 32; o > 0; o >>= 1) {
+    const double v = __shfl_xor(emin, o, 64);
+    const int i = __shfl_xor(imin, o, 64);
+    if (v < emin || (v == emin && i < imin)) {
+      emin = v;
+      imin = i;
+    }
+  }
+  emin = lane_get(emin, 0);
+  imin = __builtin_amdgcn_readfirstlane(imin);
+  if (__ballot(t < k && !isfinite(d)) != 0) emin = __builtin_nan("");
   if (t == 0) {
-    double emin = A[0];
-    int imin = 0;
-    for (int i = 1; i < k; ++i)
-      if (A[i + i * k] < emin) {
-        emin = A[i + i * k];
-        imin = i;
-      }
-    simin = imin;
     outs[0] = emin;
     outs[1] = (double)k;
     outs[2] = bad ? 1.0 : 0.0;
   }
-  __syncthreads();
-  const int imin = simin;
-  const int nc = zv ? 4 * r : 2 * r;
-  for (int e = t; e < nc; e += 64) coef[e] = 0.0;
-  __syncthreads();
-  for (int jj = t; jj < k; jj += 64) {
-    double cre = 0.0, cim = 0.0;
-    if (ritz) {
-      const double sg = Q[0 + imin * k] >= 0.0 ? 1.0 : -1.0;
-      cre = sg * Q[jj + imin * k];
-    } else {
-      for (int i = 0; i < k; ++i) {
-        const double lam = A[i + i * k];
-        const double mag = exp(pf_re * lam) * Q[0 + i * k];
-        cre += Q[jj + i * k] * (mag * cos(pf_im * lam));
-        cim += Q[jj + i * k] * (mag * sin(pf_im * lam));
-      }
+  double cre = 0.0, cim = 0.0;
+  if (ritz) {
+    if (t < k) cre = Q[imin * 64] >= 0.0 ? Q[imin * 64 + t] : -Q[imin * 64 + t];
+    if (emin != emin) cre = emin;
+  } else {
+    const double mag = t < k ? exp(pf_re * d) * Q[t * 64] : 0.0;
+    const double wr = mag * cos(pf_im * d), wi = mag * sin(pf_im * d);
+    for (int i = 0; i < k; ++i) {
+      const double q = Q[i * 64 + t];
+      cre += q * lane_get(wr, i);
+      cim += q * lane_get(wi, i);
     }
-    if (!zv) {
-      coef[jj] = cre;
-      coef[r + jj] = cim;
-    } else {
-      coef[2 * jj] = cre;           // Re out += Re c Re v - Im c Im v
-      coef[2 * jj + 1] = -cim;
-      coef[2 * r + 2 * jj] = cim;   // Im out += Im c Re v + Re c Im v
-      coef[2 * r + 2 * jj + 1] = cre;
-    }
+  }
+  if (t >= k) cre = cim = 0.0;
+  if (t >= r) return;
+  if (!zv) {
+    coef[t] = cre;
+    coef[r + t] = cim;
+  } else {
+    coef[2 * t] = cre;           // Re out += Re c Re v - Im c Im v
+    coef[2 * t + 1] = -cim;
+    coef[2 * r + 2 * t] = cim;   // Im out += Im c Re v + Re c Im v
+    coef[2 * r + 2 * t + 1] = cre;
   }
 }
 
@@ -959,29 +1079,17 @@ void launch_comb_dev(Context& c, double* out, const double* a, const double* b, 
   HIP_OK(hipGetLastError());
 }
 
-void launch_cgs_pass(Context& c, double* w, const double* V, int64_t nv, int64_t n, int k, int cplx,
-                     double* partial, double* coef) {
-  if (n <= 0 || k <= 0) return;
-  const int nblk = (int)std::min<int64_t>(kDotBlocks, std::max<int64_t>(1, (n + kThreads - 1) / kThreads));
-  hipLaunchKernelGGL(k_vdots_partial, dim3(nblk, k), dim3(kThreads), 0, c.stream, V, nv, w, n, cplx, partial);
-  HIP_OK(hipGetLastError());
-  hipLaunchKernelGGL(k_vdots_final, dim3(k), dim3(kThreads), 0, c.stream, partial, nblk, coef);
-  HIP_OK(hipGetLastError());
-  hipLaunchKernelGGL(k_cgs_sub, dim3(grid_for(n)), dim3(kThreads), 0, c.stream, w, V, nv, n, k, cplx, coef);
-  HIP_OK(hipGetLastError());
-}
-
 void launch_krylov_coef(Context& c, const double* sc, int r, double pf_re, double pf_im, int ritz, int zv,
                         double* coef, double* outs) {
   if (r < 1 || r > 64) throw Error(-1, "launch_krylov_coef: Krylov dimension must be 1..64");
-  const size_t lds = (size_t)2 * r * r * sizeof(double);
-  hipLaunchKernelGGL(k_krylov_coef, dim3(1), dim3(64), lds, c.stream, sc, r, pf_re, pf_im, ritz, zv, coef, outs);
+  hipLaunchKernelGGL(k_krylov_coef, dim3(1), dim3(64), 0, c.stream, sc, r, pf_re, pf_im, ritz, zv, coef, outs);
   HIP_OK(hipGetLastError());
 }
 
-void launch_combine(Context& c, double* out, const double* V, int64_t ld, int64_t n, const double* coef, int k) {
+void launch_combine(Context& c, double* out, double* out2, const double* V, int64_t ld, int64_t n,
+                    const double* coef, int k) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_combine, dim3(grid_for(n)), dim3(kThreads), 0, c.stream, out, V, ld, n, coef, k);
+  hipLaunchKernelGGL(k_combine, dim3(grid_for(n)), dim3(kThreads), 0, c.stream, out, out2, V, ld, n, coef, k);
   HIP_OK(hipGetLastError());
 }
 
