@@ -1073,27 +1073,9 @@ dmrj_tensor* lanczos2(Context& c, const Tensor& L, const Tensor& R, const Tensor
   issue_gemm_arith(c, theta);
   auto step = [&]() {
     issue_heff(c, h1, !graph);
-    {
-      const double* xs[2] = {th->data, th->data};
-      const double* ys[2] = {th->data, y1};
-      launch_dots(c, 2, xs, ys, n, c.scal + S_TT);
-    }
-    launch_lz_scalar(c, 1);
-    launch_axpy_dev(c, y1, th->data, n, c.scal + S_CAXPY);  // y1 := psi2
-    {
-      const double* xs[1] = {y1};
-      launch_dots(c, 1, xs, xs, n, c.scal + S_PP);
-    }
-    launch_lz_scalar(c, 2);
-    launch_scale_dev(c, y1, n, c.scal + S_INVB);
+    launch_lanczos(c, th->data, y1, y2, n, false);  // y1 := psi2
     issue_heff(c, h2, !graph);
-    {
-      const double* xs[1] = {y1};
-      const double* ys[1] = {y2};
-      launch_dots(c, 1, xs, ys, n, c.scal + S_PHP);
-    }
-    launch_lz_scalar(c, 3);
-    launch_comb_dev(c, y2, th->data, y1, n, c.scal + S_CA, c.scal + S_CB);
+    launch_lanczos(c, th->data, y1, y2, n, true);   // y2 := the Ritz vector
     if (correct) {
       // FP64 residual correction of the energy: Rayleigh quotient of the Ritz
       // vector with an FP64 H_eff application; the residual norm

@@ -494,10 +494,13 @@ void launch_dots_buf(Context& c, int npairs, const double* const* xs, const doub
                      double* out, double* partial);
 void launch_dots(Context& c, int npairs, const double* const* xs, const double* const* ys,
                  int64_t n, double* out);
+// The inner products, scalars and vector updates of the two-vector Lanczos
+// step after its first / second H_eff application; one launch up to kLzShort
+// elements, else three / two.
+constexpr int kLzShort = 16384;
+void launch_lanczos(Context& c, const double* th, double* y1, double* y2, int64_t n, bool second);
 void launch_axpy_dev(Context& c, double* y, const double* x, int64_t n, const double* coef);
 void launch_scale_dev(Context& c, double* x, int64_t n, const double* coef);
-void launch_comb_dev(Context& c, double* out, const double* a, const double* b, int64_t n,
-                     const double* ca, const double* cb);
 void launch_lz_scalar(Context& c, int stage);
 void launch_combine(Context& c, double* out, double* out2, const double* V, int64_t ld, int64_t n,
                     const double* coef, int k);

@@ -621,17 +621,8 @@ __global__ void k_scale_dev(double* x, int64_t n, const double* coef) {
     x[i] *= c;
 }
 
-__global__ void k_comb_dev(double* out, const double* a, const double* b, int64_t n,
-                           const double* ca, const double* cb) {
-  const double u = *ca, v = *cb;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    out[i] = u * a[i] + v * b[i];
-}
-
 // Scalar steps of algs/DMRG.jl:57-90 on device scalars.
-__global__ void k_lz_scalar(double* s, int stage) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__device__ inline void lz_scalar(double* s, int stage) {
   if (stage == 0) {            // normalise the orthogonality-centre tensor
     s[S_INVOC] = 1.0 / sqrt(s[S_OC]);
   } else if (stage == 1) {     // alpha1 = <AA|Hpsi>, AA = theta/|theta|
@@ -672,6 +663,184 @@ __global__ void k_lz_scalar(double* s, int stage) {
     s[S_E] = e;
     s[S_NEGE] = -e;
   }
+}
+
+__global__ void k_lz_scalar(double* s, int stage) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) lz_scalar(s, stage);
+}
+
+// The vector work of the two-vector Lanczos step (algs/DMRG.jl:57-90) between
+// its H_eff applications, th the state, y1 = H th, then y2 = H psi2:
+//   0: tt = |th|^2 and <th, y1>
+//   1: scalars of stage 1, y1 -= alpha1 th / |th|, |y1|^2
+//   2: scalars of stage 2, y1 /= beta1 (psi2)
+//   3: <y1, y2>
+//   4: scalars of stage 3, y2 := the Ritz vector
+// A launch begins with the sums of the one before it (every work-group sums all
+// partials).  Short vectors: steps 0 to 2 and steps 3 and 4 in one work-group
+// each, the vector in registers: eleven launches became two or five, 35 of 460
+// us of a bond step at m = 16 and 0.7 of 25.7 ms of a sweep at m = 64.  Up to
+// 16384 elements one work-group and five launches measure the same in a sweep,
+// the single launch costs the host less.
+constexpr int kLzThreads = 1024;
+
+__device__ inline double2 lz_block_sum(double a, double b, double2* red) {
+  a = wave_sum(a);
+  b = wave_sum(b);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_double2(a, b);
+  __syncthreads();
+  double2 t = make_double2(0.0, 0.0);
+#pragma unroll
+  for (int i = 0; i < kLzThreads / 64; ++i) {
+    t.x += red[i].x;
+    t.y += red[i].y;
+  }
+  return t;
+}
+
+template <int STEP>
+__global__ __launch_bounds__(kLzThreads) void k_lz_step(const double* __restrict__ th, double* __restrict__ y1,
+                                                        double* __restrict__ y2, int64_t n, double* __restrict__ s,
+                                                        double* __restrict__ partial) {
+  __shared__ double2 red[kLzThreads / 64];
+  __shared__ double loc[S_COUNT];
+  const int tid = threadIdx.x;
+  const int64_t stride = (int64_t)gridDim.x * kLzThreads, e0 = blockIdx.x * (int64_t)kLzThreads + tid;
+  double* part = partial + (STEP & 1 ? 2 * kDotPartials : 0);        // read by the odd steps' successors
+  const double* prev = partial + (STEP & 1 ? 0 : 2 * kDotPartials);  // written by the step before
+  if constexpr (STEP == 1 || STEP == 2 || STEP == 4) {
+    const double* p = STEP == 4 ? partial + 2 * kDotPartials : prev;
+    const bool in = tid < (int)gridDim.x;
+    const double2 t = lz_block_sum(in ? p[tid] : 0.0, STEP == 1 && in ? p[kDotPartials + tid] : 0.0, red);
+    if (tid < S_COUNT) loc[tid] = s[tid];
+    __syncthreads();
+    if (tid == 0) {
+      if constexpr (STEP == 1) {
+        loc[S_TT] = t.x;
+        loc[S_TH] = t.y;
+      }
+      if constexpr (STEP == 2) loc[S_PP] = t.x;
+      if constexpr (STEP == 4) loc[S_PHP] = t.x;
+      lz_scalar(loc, STEP == 4 ? 3 : STEP);
+    }
+    __syncthreads();
+  }
+  double a = 0.0, b = 0.0;
+  if constexpr (STEP == 0) {
+#pragma unroll 4
+    for (int64_t e = e0; e < n; e += stride) {
+      const double x = th[e];
+      a += x * x;
+      b += x * y1[e];
+    }
+  } else if constexpr (STEP == 1) {
+    const double c = loc[S_CAXPY];
+#pragma unroll 4
+    for (int64_t e = e0; e < n; e += stride) {
+      const double y = y1[e] + c * th[e];
+      y1[e] = y;
+      a += y * y;
+    }
+  } else if constexpr (STEP == 2) {
+    const double c = loc[S_INVB];
+#pragma unroll 4
+    for (int64_t e = e0; e < n; e += stride) y1[e] *= c;
+  } else if constexpr (STEP == 3) {
+#pragma unroll 4
+    for (int64_t e = e0; e < n; e += stride) a += y1[e] * y2[e];
+  } else {
+    const double u = loc[S_CA], v = loc[S_CB];
+#pragma unroll 4
+    for (int64_t e = e0; e < n; e += stride) y2[e] = u * th[e] + v * y1[e];
+  }
+  if constexpr (STEP == 0 || STEP == 1 || STEP == 3) {
+    const double2 t = lz_block_sum(a, b, red);
+    if (tid == 0) {
+      part[blockIdx.x] = t.x;
+      if constexpr (STEP == 0) part[kDotPartials + blockIdx.x] = t.y;
+    }
+  }
+  // the scalars last: other work-groups may still read the old ones (they do
+  // not use what this step sets)
+  if constexpr (STEP == 1 || STEP == 2 || STEP == 4)
+    if (blockIdx.x == 0 && tid < S_COUNT) s[tid] = loc[tid];
+}
+
+template <int E>
+__global__ __launch_bounds__(kLzThreads) void k_lz_short(const double* __restrict__ th, double* __restrict__ y1,
+                                                         double* __restrict__ y2, int n, double* __restrict__ s,
+                                                         int second) {
+  __shared__ double2 red[kLzThreads / 64];
+  __shared__ double loc[S_COUNT];
+  const int tid = threadIdx.x;
+  if (tid < S_COUNT) loc[tid] = s[tid];
+  double y[E], a = 0.0, b = 0.0;
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const int e = tid + u * kLzThreads;
+    y[u] = e < n ? y1[e] : 0.0;
+    const double x = e < n ? (second ? y2 : th)[e] : 0.0;
+    a += second ? 0.0 : x * x;
+    b += x * y[u];
+  }
+  const double2 t = lz_block_sum(a, b, red);
+  if (tid == 0) {
+    loc[second ? S_PHP : S_TH] = t.y;
+    if (!second) loc[S_TT] = t.x;
+    lz_scalar(loc, second ? 3 : 1);
+  }
+  __syncthreads();
+  if (!second) {
+    const double c = loc[S_CAXPY];
+    a = 0.0;
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const int e = tid + u * kLzThreads;
+      y[u] += c * (e < n ? th[e] : 0.0);
+      a += y[u] * y[u];
+    }
+    const double2 p = lz_block_sum(a, 0.0, red);
+    if (tid == 0) {
+      loc[S_PP] = p.x;
+      lz_scalar(loc, 2);
+    }
+    __syncthreads();
+  }
+  const double c0 = second ? loc[S_CA] : 0.0, c1 = loc[second ? S_CB : S_INVB];
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const int e = tid + u * kLzThreads;
+    if (e < n) {
+      if (second)
+        y2[e] = c0 * th[e] + c1 * y[u];
+      else
+        y1[e] = y[u] * c1;
+    }
+  }
+  if (tid < S_COUNT) s[tid] = loc[tid];
+}
+
+// After the first (second = false) or the second H_eff application.
+void launch_lanczos(Context& c, const double* th, double* y1, double* y2, int64_t n, bool second) {
+  const dim3 t(kLzThreads);
+  if (n <= 4 * kLzThreads) {
+    hipLaunchKernelGGL(k_lz_short<4>, dim3(1), t, 0, c.stream, th, y1, y2, (int)n, c.scal, second ? 1 : 0);
+  } else if (n <= kLzShort) {
+    hipLaunchKernelGGL(k_lz_short<kLzShort / kLzThreads>, dim3(1), t, 0, c.stream, th, y1, y2, (int)n, c.scal,
+                       second ? 1 : 0);
+  } else {
+    const dim3 g((unsigned)std::min<int64_t>(kDotPartials, (n + 4 * kLzThreads - 1) / (4 * kLzThreads)));
+    if (!second) {
+      hipLaunchKernelGGL(k_lz_step<0>, g, t, 0, c.stream, th, y1, y2, n, c.scal, c.partial);
+      hipLaunchKernelGGL(k_lz_step<1>, g, t, 0, c.stream, th, y1, y2, n, c.scal, c.partial);
+      hipLaunchKernelGGL(k_lz_step<2>, g, t, 0, c.stream, th, y1, y2, n, c.scal, c.partial);
+    } else {
+      hipLaunchKernelGGL(k_lz_step<3>, g, t, 0, c.stream, th, y1, y2, n, c.scal, c.partial);
+      hipLaunchKernelGGL(k_lz_step<4>, g, t, 0, c.stream, th, y1, y2, n, c.scal, c.partial);
+    }
+  }
+  HIP_OK(hipGetLastError());
 }
 
 // Lane-layout probes of v_mfma_f64_16x16x4f64 (one wave, in-bounds):
@@ -1068,14 +1237,6 @@ void launch_axpy_dev(Context& c, double* y, const double* x, int64_t n, const do
 void launch_scale_dev(Context& c, double* x, int64_t n, const double* coef) {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_scale_dev, dim3(grid_for(n)), dim3(kThreads), 0, c.stream, x, n, coef);
-  HIP_OK(hipGetLastError());
-}
-
-void launch_comb_dev(Context& c, double* out, const double* a, const double* b, int64_t n,
-                     const double* ca, const double* cb) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_comb_dev, dim3(grid_for(n)), dim3(kThreads), 0, c.stream, out, a, b, n, ca,
-                     cb);
   HIP_OK(hipGetLastError());
 }
 

@@ -1,5 +1,5 @@
-"""The Krylov iteration (algs/time.jl:182-202) at the lengths where its kernels
-change: one work-group up to 4096 stored elements, above that several, whose
+"""The Krylov iteration (algs/time.jl:182-202) and the two-vector Lanczos step
+(algs/DMRG.jl:57-90) at the lengths where their kernels change.  Krylov: one work-group up to 4096 stored elements, above that several, whose
 pieces hold 1024 elements, up to 512 work-groups; and over the Krylov
 dimensions the coefficient kernel takes (1..64).
 
@@ -42,6 +42,20 @@ def chain(rng, dl, dr, cplx):
     return left, mid, right
 
 
+def environments(pkg, ctx, A, k, mpo):
+    """Device and oracle environments around the two sites k, k + 1 (0-based)."""
+    N = len(A)
+    gL, oL = pkg.network.makeBoundary(ctx, True), np.ones((1, 1, 1))
+    for i in range(k):
+        gL = pkg.Lupdate(gL, pkg.site_from_dense(ctx, A[i]), mpo, i + 1)
+        oL = od.Lupdate(oL, A[i], mpo.H[i])
+    gR, oR = pkg.network.makeBoundary(ctx, False), np.ones((1, 1, 1))
+    for i in range(N - 1, k + 1, -1):
+        gR = pkg.Rupdate(gR, pkg.site_from_dense(ctx, A[i]), mpo, i + 1)
+        oR = od.Rupdate(oR, A[i], mpo.H[i])
+    return gL, oL, gR, oR
+
+
 @pytest.mark.parametrize("dl,dr,cplx,r,pf", [
     (1, 2, False, 3, -0.25), (2, 2, False, 1, -0.25), (8, 8, False, 64, -0.25), (5, 9, False, 17, -0.3j),
     (31, 33, False, 12, -0.25), (32, 32, False, 12, -0.25), (32, 33, False, 12, -0.25), (29, 71, False, 5, -0.3j),
@@ -52,16 +66,9 @@ def test_krylov_sizes(pkg, ctx, dl, dr, cplx, r, pf):
     rng = np.random.default_rng(dl * 1000 + dr)
     left, mid, right = chain(rng, dl, dr, cplx)
     A = left + mid + right
-    N, k = len(A), len(left)
-    mpo = pkg.makeMPO(pkg.heisenbergMPO(), 2, N)
-    gL, oL = pkg.network.makeBoundary(ctx, True), np.ones((1, 1, 1))
-    for i in range(k):
-        gL = pkg.Lupdate(gL, pkg.site_from_dense(ctx, A[i]), mpo, i + 1)
-        oL = od.Lupdate(oL, A[i], mpo.H[i])
-    gR, oR = pkg.network.makeBoundary(ctx, False), np.ones((1, 1, 1))
-    for i in range(N - 1, k + 1, -1):
-        gR = pkg.Rupdate(gR, pkg.site_from_dense(ctx, A[i]), mpo, i + 1)
-        oR = od.Rupdate(oR, A[i], mpo.H[i])
+    k = len(left)
+    mpo = pkg.makeMPO(pkg.heisenbergMPO(), 2, len(A))
+    gL, oL, gR, oR = environments(pkg, ctx, A, k, mpo)
     h = C.c_void_p()
     dev = [pkg.site_from_dense(ctx, m) for m in mid]
     ctx.call("dmrj_theta2", dev[0].h, dev[1].h, C.byref(h))
@@ -74,3 +81,26 @@ def test_krylov_sizes(pkg, ctx, dl, dr, cplx, r, pf):
     print("n", oth.size, "r", r, "err %.1e" % err, "energy %.1e" % abs(e - we), flush=True)
     assert err <= 1e-12
     assert abs(e - we) <= 1e-12 * max(1.0, abs(we))
+
+
+@pytest.mark.parametrize("dl,dr", [(1, 1), (2, 3), (15, 17), (31, 33), (32, 32), (32, 33), (63, 65), (64, 64), (64, 65),
+                                   (130, 129), (367, 366)])
+def test_lanczos_sizes(pkg, ctx, dl, dr):
+    """The two-vector Lanczos step where its vector kernels change: 4096 and
+    16384 elements in one work-group, above that several."""
+    rng = np.random.default_rng(dl * 1000 + dr)
+    left, mid, right = chain(rng, dl, dr, False)
+    A = left + mid + right
+    k = len(left)
+    mpo = pkg.makeMPO(pkg.heisenbergMPO(), 2, len(A))
+    gL, oL, gR, oR = environments(pkg, ctx, A, k, mpo)
+    dev = [pkg.site_from_dense(ctx, m) for m in mid]
+    h, e = C.c_void_p(), C.c_double()
+    ctx.call("dmrj_lanczos2", gL.h, gR.h, dev[0].h, dev[1].h, mpo.device(ctx, k + 1), mpo.device(ctx, k + 2), 0,
+             C.byref(h), C.byref(e))
+    got = pkg.DeviceTensor(ctx, h).to_dense()[0]
+    want_e, want = od.simplelanczos(oL, oR, mid[0], mid[1], mpo.H[k], mpo.H[k + 1])
+    err = min(np.max(np.abs(got - want)), np.max(np.abs(got + want))) / np.max(np.abs(want))
+    print("n", got.size, "energy %.1e" % abs(e.value - want_e), "state %.1e" % err, flush=True)
+    assert abs(e.value - want_e) <= 1e-12 * max(1.0, abs(want_e))
+    assert err <= 1e-12
