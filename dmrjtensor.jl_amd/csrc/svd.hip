@@ -971,7 +971,46 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       reorth_basis(c, rj);
       complete_basis(c, cj);
     }
+    // complex: vectors whose columns ended below the solver's floor are
+    // orthogonal to the others to 1e-14 floor / sigma only, which the other
+    // factor's product would multiply by the largest sigma; there is no
+    // completion here, they are projected off the others
+    std::vector<double*> scratch;
+    if (z) {
+      std::vector<GemmTask> t1, t2;
+      std::vector<GemmSeg> s1, s2;
+      const double low = std::max(szero, 2e-11 * std::sqrt(aa2));
+      hoff = 0;
+      for (int si : order) {
+        Sec& s = secs[si];
+        int c0 = s.qj >= 0 ? s.keep : 0;
+        while (c0 > 0 && hs[hoff + c0 - 1] <= low) --c0;
+        hoff += s.kmin;
+        const int nz = s.keep - c0;
+        if (c0 == 0 || nz == 0) continue;
+        double* co = (double*)c.alloc.alloc((int64_t)2 * c0 * nz * sizeof(double));
+        scratch.push_back(co);
+        planes.add(co, (int64_t)c0 * nz, true);
+        if (dir > 0) {  // U1 -= U0 (U0^H U1)
+          double* u1 = s.U + (int64_t)c0 * s.R;
+          t1.push_back({co, c0, c0, nz, (int)s1.size(), 1, 0.0});
+          s1.push_back({s.U, u1, s.R, s.R, (int)s.R, 1 | kSegConjA, 1.0});
+          t2.push_back({u1, s.R, (int)s.R, nz, (int)s2.size(), 1, 1.0});
+          s2.push_back({s.U, co, s.R, c0, c0, 0, -1.0});
+        } else {  // V1^H -= (V1^H V0) V0^H
+          t1.push_back({co, nz, nz, c0, (int)s1.size(), 1, 0.0});
+          s1.push_back({s.Vt + c0, s.Vt, s.kmin, s.kmin, (int)s.C, 2 | kSegConjB, 1.0});
+          t2.push_back({s.Vt + c0, s.kmin, nz, (int)s.C, (int)s2.size(), 1, 1.0});
+          s2.push_back({co, s.Vt, nz, s.kmin, c0, 0, -1.0});
+        }
+      }
+      complexify_gemm(t1, s1, planes);
+      complexify_gemm(t2, s2, planes);
+      launch_gemm(c, t1, s1, -1);
+      launch_gemm(c, t2, s2, -1);
+    }
     issue_gemm_arith(c, gp);
+    for (double* p : scratch) c.alloc.release(p);
     issue_copy(c, sp);
   }
   for (auto& s : secs) {

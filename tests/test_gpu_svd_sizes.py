@@ -136,3 +136,27 @@ def test_complex_svd_sectors_of_different_sizes(pkg, ctx, direction):
     Rt = pkg.DeviceTensor(ctx, r).to_dense(1)[0]
     assert np.all(np.isfinite(L)) and np.all(np.isfinite(Rt))
     assert np.max(np.abs(np.tensordot(L, Rt, axes=(2, 0)) - A)) <= 8 * 2 * m * EPS
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("shape", [(210, 16), (16, 230), (40, 33), (33, 70), (130, 257), (280, 300)])
+def test_complex_svd_rank_deficient(pkg, ctx, shape, direction):
+    """Groups of equal columns and zero rows: the vectors of the vanishing
+    singular values must not bring weight into the product of the factors."""
+    R, Cc = shape
+    rng = np.random.default_rng(R * 31 + Cc)
+    M = np.exp(2j * np.pi * rng.random(R))[:, None] * _matrix("equal", R, Cc, rng)
+    M = M * np.exp(2j * np.pi * rng.random(Cc))[None, :]
+    n = max(R, Cc)
+    want = np.linalg.svd(M, compute_uv=False)
+    for scale in (1.0, 1e-150, 1e100):
+        t = pkg.site2_from_dense(ctx, (M * scale).reshape(R, 1, 1, Cc))
+        l, r, te, kk = C.c_void_p(), C.c_void_p(), C.c_double(), C.c_int64()
+        sv = np.zeros(512)
+        ctx.call("dmrj_svd_trunc2", t.h, 0, 2, 0.0, direction, C.byref(l), C.byref(r), C.byref(te), C.byref(kk),
+                 pkg._lib.dptr(sv), 512)
+        L = pkg.DeviceTensor(ctx, l).to_dense()[0].reshape(R, -1)
+        Rt = pkg.DeviceTensor(ctx, r).to_dense()[0].reshape(-1, Cc)
+        assert kk.value == min(R, Cc)
+        assert np.max(np.abs(sv[:kk.value] * np.linalg.norm(want) - want)) <= 2 * n * EPS
+        assert np.max(np.abs(L @ Rt * np.linalg.norm(want) - M)) <= 8 * n * EPS
