@@ -616,7 +616,8 @@ struct SmallSvdJob {
   int R, C;
 };
 // runs on c.side; join with hipStreamWaitEvent(c.stream, c.side_out) when it returns true
-bool launch_svd_small(Context& c, const std::vector<SmallSvdJob>& jobs, size_t lds_bytes);
+// scale 0: k_svd_small (real); else k_svd_tiny (sides up to 16), which works on the matrices times scale, a power of two
+bool launch_svd_small(Context& c, const std::vector<SmallSvdJob>& jobs, size_t lds_bytes, bool cplx, double scale);
 struct AugJob {
   const double* A;
   const double* W;
@@ -626,7 +627,7 @@ struct AugJob {
   int R, C, N, kmin;
 };
 void launch_aug_extract(Context& c, const std::vector<AugJob>& jobs);
-size_t small_svd_lds(int R, int C);
+size_t small_svd_lds(int R, int C, bool cplx);
 constexpr size_t kSmallSvdMaxLds = 60 * 1024;  // bytes of dynamic LDS per sector
 double gemm_flops(const std::vector<GemmTask>& tasks, const std::vector<GemmSeg>& segs);
 

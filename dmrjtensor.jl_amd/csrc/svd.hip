@@ -93,6 +93,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     int bj = 0, rowsX = 0, ncolsX = 0;
     int qr = 0;  // one-factor sector solved through its LQ / QR triangle (X: K x K factor)
     int qj = -1;   // index in the QR-preconditioned Jacobi batch
+    bool tiny = false;  // both factors from the one-launch Jacobi kernel, orthonormal to working precision
     int gram = 0;  // orthonormal factor = eigenvectors of the Gram matrix (orthonormal to working precision)
     std::vector<int> perm;
     std::vector<double> hn;
@@ -190,20 +191,30 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   const int psvd = c.prof_begin();
   double svd_flops = 0.0;
   // small sectors: one batched Jacobi launch.  With the default backend it
-  // takes sides up to 16, above which the launches of the blocked solver are
-  // the shorter chain: bond step with sectors to 55, 2.43 ms with this kernel
-  // up to 64, 1.01 up to 32, 0.77 up to 16; to 80 (m=80 Hubbard) 2.90, 0.91,
-  // 0.88; to 18 (m=16 Heisenberg) 0.43, 0.45, 0.46.
-  const int small_side = c.svd_backend == 0 ? 16 : 64;
+  // takes sides up to 16 (k_svd_tiny), above which the launches of the blocked
+  // solver are the shorter chain (sides up to 64 in such a kernel: 2.43 ms for a
+  // bond step with sectors to 55, up to 32: 1.01, up to 16: 0.77).
+  const int small_side = z || c.svd_backend == 0 ? 16 : 64;
+  // the kernel for sides up to 16 works on the matrices scaled to norm one by
+  // a power of two (exact); not where the squared norm under- or overflows
+  const bool in_range = aa2 > 1e-305 && aa2 < 1e305;
+  double tiny_scale = 0.0;
+  if (small_side == 16 && in_range) {
+    int ex = 0;
+    (void)std::frexp(std::sqrt(aa2), &ex);
+    tiny_scale = std::ldexp(1.0, -ex);
+  }
   std::vector<SmallSvdJob> small;
   size_t small_lds = 0;
   std::vector<char> is_small(secs.size(), 0);
   for (int si : order) {
     Sec& s = secs[si];
-    if (z || s.kmin == 0 || s.kmin > small_side || c.svd_backend == 1 || c.svd_backend == 2) continue;
-    const size_t l = small_svd_lds((int)s.R, (int)s.C);
-    if (l > kSmallSvdMaxLds) continue;
+    if (s.kmin == 0 || s.kmin > small_side || (z ? tiny_scale == 0.0 : c.svd_backend == 1 || c.svd_backend == 2))
+      continue;
+    const size_t l = small_svd_lds((int)s.R, (int)s.C, z);
+    if (l + (z ? 4096 : 0) > kSmallSvdMaxLds) continue;
     is_small[si] = 1;
+    s.tiny = tiny_scale != 0.0;
     small_lds = std::max(small_lds, l);
     small.push_back({s.M, s.U, s.s, s.Vt, (int)s.R, (int)s.C});
     const double mm = (double)std::max(s.R, s.C), nn = (double)std::min(s.R, s.C);
@@ -216,7 +227,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   // sweep limit) and tensors whose squared norm under- or overflows go to the
   // eigensolves of the augmented matrices.
   QjBatch qj(c, z);
-  if ((z || c.svd_backend == 0) && aa2 > 1e-305 && aa2 < 1e305) {
+  if ((z || c.svd_backend == 0) && in_range) {
     for (int si : order) {
       Sec& s = secs[si];
       if (s.kmin == 0 || is_small[si] || !qj_fits(s.R, s.C, z)) continue;
@@ -232,7 +243,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     }
     qj_prepare(qj);
   }
-  const bool small_on_side = launch_svd_small(c, small, small_lds);
+  const bool small_on_side = launch_svd_small(c, small, small_lds, z, tiny_scale);
   // every exit from here on, exceptions included, orders the main stream
   // after the side-stream kernel, so no later synchronisation of the main
   // stream can release memory that kernel still uses
@@ -947,9 +958,11 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       Sec& s = secs[si];
       if (s.keep > 0) {
         int c0 = s.keep;
-        while (c0 > 0 && hs[hoff + c0 - 1] <= szero) --c0;
+        // (the one-launch kernel's vectors are orthonormal whatever their weight;
+        // only vanishing columns, below the range of the products, are not)
+        while (c0 > 0 && hs[hoff + c0 - 1] <= (s.tiny ? 1e-60 * smax : szero)) --c0;
         int c1 = c0;
-        if (!s.gram && s.qj < 0)  // Gram eigenvectors and Jacobi columns need no re-orthonormalisation
+        if (!s.gram && !s.tiny && s.qj < 0)  // Gram eigenvectors and Jacobi columns need no re-orthonormalisation
           while (c1 > 1 && hs[hoff + c1 - 1] < ssmall) --c1;
         const int nv = (int)(dir > 0 ? s.R : s.C);
         if (c1 < c0 && c1 >= 1) {

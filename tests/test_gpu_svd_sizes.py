@@ -160,3 +160,41 @@ def test_complex_svd_rank_deficient(pkg, ctx, shape, direction):
         assert kk.value == min(R, Cc)
         assert np.max(np.abs(sv[:kk.value] * np.linalg.norm(want) - want)) <= 2 * n * EPS
         assert np.max(np.abs(L @ Rt * np.linalg.norm(want) - M)) <= 8 * n * EPS
+
+def _factors(pkg, ctx, M, direction):
+    R, Cc = M.shape
+    t = pkg.site2_from_dense(ctx, M.reshape(R, 1, 1, Cc))
+    l, r, te, kk = C.c_void_p(), C.c_void_p(), C.c_double(), C.c_int64()
+    sv = np.zeros(64)
+    ctx.call("dmrj_svd_trunc2", t.h, 0, 2, 0.0, direction, C.byref(l), C.byref(r), C.byref(te), C.byref(kk),
+             pkg._lib.dptr(sv), 64)
+    L = pkg.DeviceTensor(ctx, l).to_dense()[0].reshape(R, -1)
+    Rt = pkg.DeviceTensor(ctx, r).to_dense()[0].reshape(-1, Cc)
+    return L, Rt, sv[:kk.value]
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("kind", ["flat", "graded", "equal", "isometric"])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("shape", [(1, 1), (1, 7), (6, 1), (2, 2), (3, 2), (5, 16), (16, 16), (16, 15), (13, 8), (16, 33),
+                                   (31, 7), (16, 200), (210, 16), (16, 440), (452, 16)])
+def test_svd_small_sides(pkg, ctx, shape, cplx, kind, direction):
+    """Sides up to 16: one launch of cyclic Jacobi while the sector fits into
+    LDS.  Pairs are orthogonal to 4 eps, sums over the longer side add their
+    rounding; the accumulated factor ends in a Newton-Schulz step."""
+    R, Cc = shape
+    rng = np.random.default_rng(R * 31 + Cc)
+    M = _matrix(kind, R, Cc, rng)
+    if cplx:  # unitary phases: the same singular values
+        M = np.exp(2j * np.pi * rng.random(R))[:, None] * M * np.exp(2j * np.pi * rng.random(Cc))[None, :]
+    n, K = max(R, Cc), min(R, Cc)
+    want = np.linalg.svd(M, compute_uv=False)
+    for scale in (1.0, 1e-150, 1e100):
+        L, Rt, sv = _factors(pkg, ctx, M * scale, direction)
+        assert len(sv) == K
+        assert np.max(np.abs(sv - want / np.linalg.norm(want))) <= 2 * n * EPS
+        zero = want[want <= 1e-10 * want[0]]
+        assert np.max(np.abs(L @ Rt * np.linalg.norm(want) - M)) <= 8 * n * EPS + np.linalg.norm(zero)
+        big = want > 1e-10 * want[0] if cplx else np.full(K, True)
+        Q = (L if direction > 0 else Rt.conj().T)[:, big]
+        assert np.max(np.abs(Q.conj().T @ Q - np.eye(big.sum()))) <= (8 + 2 * np.sqrt(n)) * EPS + 4 * K * EPS
