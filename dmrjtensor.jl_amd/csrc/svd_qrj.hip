@@ -35,9 +35,10 @@
 // and 7 to 8 sweeps of K/16 rounds of 15 to 45 us.  Bond step at the middle of
 // an m=1024 Heisenberg chain (sectors to 508): 31.0 ms with the batched
 // eigensolve of the augmented matrices, five launches per column of R + C,
-// 7.1 ms with this; m=2048 Hubbard (sectors to 1164): 134 and 31 ms.  A third
-// factorisation (of A2) saves a sweep and costs its panels: 7.3 and 30.7 ms, and
-// 1.06 against 0.98 ms at a single 100 x 100 sector.
+// 6.5 ms with this; m=2048 Hubbard (sectors to 1164): 134 and 28.6 ms.  A third
+// factorisation (of A2) saves a sweep and costs its panels (7.3 against 7.1 ms,
+// 30.7 against 31, 1.06 against 0.98 at a single 100 x 100 sector, when rounds
+// were 5% slower).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -101,10 +102,14 @@ __device__ __forceinline__ double fast_rcp(double x) {
   return fma(y * e, 1.0 + e, y);
 }
 
-// Tangent of the Jacobi rotation from its cotangent of the double angle
-// f >= 0 (1e-38 for the pairs of columns furthest apart: no overflow in f^2).
-__device__ __forceinline__ float jacobi_tangent(float f) {
-  return __builtin_amdgcn_rcpf(f + (f < 1e15f ? __builtin_amdgcn_sqrtf(fmaf(f, f, 1.0f)) : f));
+// Generator of the Jacobi rotation from its cotangent of the double angle
+// f >= 0 (1e-38 for the pairs of columns furthest apart: no overflow in f^2):
+// the x for which the unitary polynomial of the round turns by the angle of the
+// tangent t = 1 / (f + sqrt(f^2 + 1)), x = t - t^3 / 4 + ..., to 0.003 rad.
+__device__ __forceinline__ float jacobi_generator(float f) {
+  const float t = __builtin_amdgcn_rcpf(f + (f < 1e15f ? __builtin_amdgcn_sqrtf(fmaf(f, f, 1.0f)) : f));
+  const float t2 = t * t;
+  return t * (1.0f - t2 * (0.25f - 0.096f * t2));
 }
 
 // The wave's number in its work-group, in a scalar register.
@@ -559,7 +564,7 @@ template <bool Z>
 __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs, int step, double tol2,
                                                   double floor2) {
   // waves, row blocks in flight per wave, planes, leading dimension and size of a 32 x 32 matrix in LDS
-  constexpr int kW = 8, kU = Z ? 2 : 4, kP = Z ? 2 : 1, kLd = 33, kM = 32 * kLd, kT = kTile<Z>;
+  constexpr int kW = 8, kU = 2, kS = Z ? 1 : 2, kP = Z ? 2 : 1, kLd = 33, kM = 32 * kLd, kT = kTile<Z>;
   __shared__ double red[kW * 3 * kT];   // partial Gram tiles, then four matrices
   __shared__ double G[kP * kM];
   __shared__ double cn[32];
@@ -580,30 +585,45 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
   double* Yq = jb.A[2] + (int64_t)q * rb * kT;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   {
+    // real: the next row blocks are in flight while the current ones are multiplied
     Tile<Z> pp = {kZero4, kZero4}, pq = pp, qq = pp;
-    for (int b0 = w; b0 < rb; b0 += kU * kW) {
-      double x[kU][4 * kP], y[kU][4 * kP];
+    double x[kS][kU][4 * kP], y[kS][kU][4 * kP];
+    auto load = [&](int s, int b0) {
 #pragma unroll
       for (int u = 0; u < kU; ++u) {
         const int64_t o = (int64_t)min(b0 + u * kW, rb - 1) * kT + lane;
 #pragma unroll
         for (int r = 0; r < 4 * kP; ++r) {
-          x[u][r] = Yp[o + 64 * r];
-          y[u][r] = Yq[o + 64 * r];
+          x[s][u][r] = Yp[o + 64 * r];
+          y[s][u][r] = Yq[o + 64 * r];
         }
       }
+    };
+    auto add = [&](int s, int b0) {
 #pragma unroll
       for (int u = 0; u < kU; ++u)
         if (b0 + u * kW < rb) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const double xr = x[u][r], yr = y[u][r], xi = Z ? x[u][(4 + r) % (4 * kP)] : 0.0,
-                         yi = Z ? y[u][(4 + r) % (4 * kP)] : 0.0;
+            const double xr = x[s][u][r], yr = y[s][u][r], xi = Z ? x[s][u][(4 + r) % (4 * kP)] : 0.0,
+                         yi = Z ? y[s][u][(4 + r) % (4 * kP)] : 0.0;
             mac_h<Z>(pp, xr, xi, xr, xi);
             mac_h<Z>(pq, xr, xi, yr, yi);
             mac_h<Z>(qq, yr, yi, yr, yi);
           }
         }
+    };
+    load(0, w);
+    for (int b0 = w; b0 < rb; b0 += kS * kU * kW) {
+      if constexpr (kS == 2) {
+        if (b0 + kU * kW < rb) load(1, b0 + kU * kW);
+        add(0, b0);
+        if (b0 + 2 * kU * kW < rb) load(0, b0 + 2 * kU * kW);
+        add(kS - 1, b0 + kU * kW);
+      } else {
+        add(0, b0);
+        if (b0 + kU * kW < rb) load(0, b0 + kU * kW);
+      }
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -639,18 +659,40 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
   }
   if (!__syncthreads_or(act)) return;
   if (tid == 0) *jb.last = step;
-  // Inner solve, all pairs at once: X holds the Jacobi tangents of every pair
-  // (scaled down where a column of X exceeds kCap in the 2-norm), V the
-  // unitary polar factor of I + X by Newton-Schulz steps V += V (I - V^H V) / 2
-  // on the matrix cores, repeated on V^H G V while the rotations were large.
-  // Its off-diagonal rest is of second order, as after a cyclic sweep of
-  // rotations, at a fraction of the latency: a sweep is 31 dependent rounds of
-  // LDS traffic, 46000 cycles, this 8000 to 33000, and one outer sweep fewer
-  // on the sectors of an m=1024 Heisenberg state.  (A cosine applied to a
+  // rows for the final product, the first block's fetched before the inner
+  // solve and each next one's while the current is multiplied
+  double2_t rows[2][4 * kP];
+  auto fetch = [&](int s, int b) {
+    const int64_t o = (int64_t)b * kT + c * 16 + 4 * g;
+#pragma unroll
+    for (int h = 0; h < kP; ++h) {
+      rows[s][4 * h + 0] = *(const double2_t*)(Yp + o + 256 * h);
+      rows[s][4 * h + 1] = *(const double2_t*)(Yp + o + 256 * h + 2);
+      rows[s][4 * h + 2] = *(const double2_t*)(Yq + o + 256 * h);
+      rows[s][4 * h + 3] = *(const double2_t*)(Yq + o + 256 * h + 2);
+    }
+  };
+  fetch(0, min(w, rb - 1));
+  // Inner solve, all pairs at once: X holds the Jacobi rotations of every pair
+  // as a skew matrix (scaled down where a column of X exceeds kCap in the
+  // 2-norm), V a unitary matrix near I + X, from a polynomial and
+  // Newton-Schulz steps V += V (I - V^H V) / 2 on the matrix cores, repeated on
+  // V^H G V while the rotations were large.  Its off-diagonal rest is of second
+  // order, as after a cyclic sweep of rotations, at a fraction of the latency:
+  // a sweep is 31 dependent rounds of LDS traffic, 46000 cycles, this 9000 on
+  // average (20000 where the rotations are large), and one outer sweep fewer on
+  // the sectors of an m=1024 Heisenberg state.  (A cosine applied to a
   // column would also scale it by its rounding error, and those factors add up
   // over the rounds: 3e-14 of the singular values of a 200 x 200 Gaussian
   // matrix, against 1.5e-15.)
-  constexpr double kCap = 0.7, kSmall = 0.25;
+  // The rest of an average round at 400 columns: 9200 cycles the Gram tiles,
+  // 2000 their sum, 11100 the product, for 5400 and 7200 of FP64 MFMA time of
+  // the CU's busiest SIMD; their loads are therefore in flight ahead.  Bond
+  // steps with this and the polynomial against neither: 200 x 400 dense 4.23 to
+  // 4.05 ms, m=510 Hubbard 2.90 to 2.70, m=2048 Hubbard 30.6 to 28.6.  Slicing
+  // the rows of a pair over several work-groups (partial Gram tiles in a launch
+  // of their own) was no faster at any size.
+  constexpr double kCap = 0.85, kSmall = 0.25;
   constexpr int kRepeats = 2, kNewton = 12;
   double* V = red;             // this repeat's factor
   double* Vt = V + kP * kM;    // the products so far
@@ -702,52 +744,67 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
         const double ri = fast_rsqrt(go ? q2 : 1.0);   // 1 / |g_ij|
         const float f = (float)(0.5 * d * ri);
         const bool neg = f < 0.0f || (f == 0.0f && i > j);
-        const double t = go ? (double)jacobi_tangent(fabsf(f)) * ri : 0.0;
+        const double t = go ? (double)jacobi_generator(fabsf(f)) * ri : 0.0;
         V[i * kLd + j] = i == j ? 1.0 : neg ? -t * x : t * x;
         V[kM + i * kLd + j] = i == j ? 0.0 : neg ? -t * y : t * y;
       } else {
         const bool go = i != j && x * x > fmax(eps2 * gi * gj, 1e-280);
         const float f = (float)(d * __builtin_amdgcn_rcp(go ? 2.0 * x : 1.0));
         const bool neg = f < 0.0f || (f == 0.0f && (i > j) != (x < 0.0));
-        const float t = jacobi_tangent(fabsf(f));
+        const float t = jacobi_generator(fabsf(f));
         V[i * kLd + j] = i == j ? 1.0 : go ? (double)(neg ? -t : t) : 0.0;
       }
       const unsigned long long m = __ballot(gj > gi || (gj == gi && j < i));
       if (j == 0) order[__popc((unsigned)(lane < 32 ? m : m >> 32))] = i;
     }
     __syncthreads();
-    // X is skew: I - V^H V = X^2, and V + X^2 / 2 is unitary up to X^4 / 4
+    // X is skew, S = V^H V - I = X^H X = -X^2, and
+    //   (I - S/2 + S^2/8) + X (I - S/4 + S^2/32)
+    // is unitary up to S^5 / 1024 (the coefficients cancel S to S^4), so few
+    // Newton-Schulz steps are left where |X|_2 is near one
     Tile<Z> v = zero, e = zero;
     if (mine) {
-      v = get(V);
       e = mul(V, true, V, zero);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const bool one = ti == tj && 4 * r + g == c;
-        e.r[r] = (one ? 1.0 : 0.0) - e.r[r];
-        if (one) cn[16 * ti + c] = -e.r[r];  // squared norms of the columns of X
-      }
+      for (int r = 0; r < 4; ++r)
+        if (ti == tj && 4 * r + g == c) {
+          e.r[r] -= 1.0;
+          cn[16 * ti + c] = e.r[r];  // squared norms of the columns of X
+        }
+      put(E, e);
     }
     __syncthreads();
     double mx = 0.0;
 #pragma unroll
     for (int k = 0; k < 32; ++k) mx = fmax(mx, cn[k]);
     const bool large = mx > kSmall * kSmall;
+    const double a2 = mx > cap * cap ? cap * cap / mx : 1.0, a1 = sqrt(a2);
     if (mine) {
-      const double a2 = mx > cap * cap ? cap * cap / mx : 1.0, a1 = sqrt(a2);
+      const Tile<Z> q = mul(E, true, E, zero);
+      Tile<Z> d;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const bool one = ti == tj && 4 * r + g == c;
-        v.r[r] = (one ? 1.0 : a1 * v.r[r]) + 0.5 * a2 * e.r[r];
-        if constexpr (Z) v.i[r] = a1 * v.i[r] - 0.5 * a2 * e.i[r];
+        const double one = ti == tj && 4 * r + g == c ? 1.0 : 0.0;
+        d.r[r] = one - a2 * (0.25 * e.r[r] - 0.03125 * a2 * q.r[r]);
+        v.r[r] = one - a2 * (0.5 * e.r[r] - 0.125 * a2 * q.r[r]) - a1 * d.r[r];
+        if constexpr (Z) {
+          d.i[r] = -a2 * (0.25 * e.i[r] - 0.03125 * a2 * q.i[r]);
+          v.i[r] = -a2 * (0.5 * e.i[r] - 0.125 * a2 * q.i[r]) - a1 * d.i[r];
+        }
+        d.r[r] *= a1;
+        d.i[r] *= a1;
       }
-      put(V, v);
+      put(Tm, d);
     }
+    __syncthreads();
+    if (mine) v = mul(V, false, Tm, v);  // V = I + X, the surplus D is in v already
+    __syncthreads();
+    if (mine) put(V, v);
     __syncthreads();
     // Newton-Schulz steps as many as |X|_2^2 = 2 mx asks for, the last one
     // checked: the deviation it found is squared by its update
-    double dev = fmin(2.0 * mx, 1.0);
-    dev *= 0.25 * dev;
+    double dev = fmin(2.0 * a2 * mx, 1.0);
+    dev = dev * dev * dev * dev * dev * (1.0 / 1024);
     bool conv = dev < 1e-17;
     for (int nt = 0; nt < kNewton && !conv; ++nt) {
       int big = 0;
@@ -804,41 +861,30 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
       vb[h][k] = Vt[e];
       vi[h][k] = Z ? Vt[(kP - 1) * kM + e] : 0.0;
     }
-  constexpr int kV = Z ? 1 : 2;  // row blocks in flight per wave
-  for (int b0 = w; b0 < rb; b0 += kV * kW) {
-    double2_t x[kV][4 * kP];
+  auto turn = [&](int s, int b) {
+    Tile<Z> yp = zero, yq = zero;
 #pragma unroll
-    for (int u = 0; u < kV; ++u) {
-      const int64_t o = (int64_t)min(b0 + u * kW, rb - 1) * kT + c * 16 + 4 * g;
+    for (int k = 0; k < 8; ++k) {
+      const double xr = rows[s][k >> 1][k & 1], xi = Z ? rows[s][4 * (kP - 1) + (k >> 1)][k & 1] : 0.0;
+      mac<Z>(yp, xr, xi, vb[0][k], vi[0][k]);
+      mac<Z>(yq, xr, xi, vb[1][k], vi[1][k]);
+    }
+    const int64_t o = (int64_t)b * kT + lane;
 #pragma unroll
-      for (int h = 0; h < kP; ++h) {
-        x[u][4 * h + 0] = *(const double2_t*)(Yp + o + 256 * h);
-        x[u][4 * h + 1] = *(const double2_t*)(Yp + o + 256 * h + 2);
-        x[u][4 * h + 2] = *(const double2_t*)(Yq + o + 256 * h);
-        x[u][4 * h + 3] = *(const double2_t*)(Yq + o + 256 * h + 2);
+    for (int r = 0; r < 4; ++r) {
+      Yp[o + 64 * r] = yp.r[r];
+      Yq[o + 64 * r] = yq.r[r];
+      if constexpr (Z) {
+        Yp[o + 256 + 64 * r] = yp.i[r];
+        Yq[o + 256 + 64 * r] = yq.i[r];
       }
     }
-#pragma unroll
-    for (int u = 0; u < kV; ++u)
-      if (b0 + u * kW < rb) {
-        Tile<Z> yp = zero, yq = zero;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const double xr = x[u][k >> 1][k & 1], xi = Z ? x[u][4 * (kP - 1) + (k >> 1)][k & 1] : 0.0;
-          mac<Z>(yp, xr, xi, vb[0][k], vi[0][k]);
-          mac<Z>(yq, xr, xi, vb[1][k], vi[1][k]);
-        }
-        const int64_t o = (int64_t)(b0 + u * kW) * kT + lane;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          Yp[o + 64 * r] = yp.r[r];
-          Yq[o + 64 * r] = yq.r[r];
-          if constexpr (Z) {
-            Yp[o + 256 + 64 * r] = yp.i[r];
-            Yq[o + 256 + 64 * r] = yq.i[r];
-          }
-        }
-      }
+  };
+  for (int b = w; b < rb; b += 2 * kW) {
+    if (b + kW < rb) fetch(1, b + kW);
+    turn(0, b);
+    if (b + 2 * kW < rb) fetch(0, b + 2 * kW);
+    if (b + kW < rb) turn(1, b + kW);
   }
 }
 
