@@ -64,13 +64,12 @@ __device__ __forceinline__ double4_t mfma(double a, double b, double4_t c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// The value of lane J of every row of 16 lanes (DPP row_newbcast).
+// The value of lane J of every row of 16 lanes (DPP row_newbcast, one 64-bit
+// move: a panel step 2% shorter than with two 32-bit ones).
 template <int J>
 __device__ __forceinline__ double row_bcast(double x) {
-  const int2 v = __builtin_bit_cast(int2, x);
-  int2 r;
-  r.x = __builtin_amdgcn_update_dpp(0, v.x, 0x150 + J, 0xf, 0xf, true);
-  r.y = __builtin_amdgcn_update_dpp(0, v.y, 0x150 + J, 0xf, 0xf, true);
+  const long long v = __builtin_bit_cast(long long, x);
+  const long long r = __builtin_amdgcn_update_dpp(v, v, 0x150 + J, 0xf, 0xf, true);
   return __builtin_bit_cast(double, r);
 }
 
@@ -484,55 +483,62 @@ __global__ __launch_bounds__(NW * 64) void k_qj_qr(const QjJob* __restrict__ job
   }
 }
 
-// Squared column norms of A0 (columns of M for dir > 0, rows for dir < 0): 64
-// columns a group.
+// Squared column norms of A0 (columns of M for dir > 0, rows for dir < 0): 16
+// columns and 16 interleaved sequences of rows a group, which reads whole
+// 128-byte lines in both directions (a wave a column or 64 columns a wave:
+// 42 us at 400 x 400, 5 now).
+template <bool Z>
 __global__ __launch_bounds__(256) void k_qj_norms0(const QjJob* __restrict__ jobs) {
-  __shared__ double part[4][64];
+  __shared__ double part[256];
   const QjJob& jb = jobs[blockIdx.y];
-  const int j0 = blockIdx.x * 64;
+  const int j0 = blockIdx.x * 16, lo = threadIdx.x & 15, hi = threadIdx.x >> 4;
   if (j0 >= jb.o) return;
   if (j0 == 0 && threadIdx.x == 0) *jb.last = -1;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const double* Mi = jb.M + jb.plane;  // imaginary plane (the real one itself for real tensors)
-  if (jb.dir < 0) {
-    double acc = 0.0;
-    if (j0 + lane < jb.o)
-      for (int i = w; i < jb.n; i += 4) {
-        const int64_t e = (int64_t)(j0 + lane) + (int64_t)i * jb.R;
-        acc += jb.M[e] * jb.M[e] + Mi[e] * Mi[e];
-      }
-    part[w][lane] = acc;
-    __syncthreads();
-    if (w == 0 && j0 + lane < jb.o) jb.nrm[j0 + lane] = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
-  } else {
-    for (int k = w; k < 64 && j0 + k < jb.o; k += 4) {
-      double acc = 0.0;
-      for (int i = lane; i < jb.n; i += 64) {
-        const int64_t e = (int64_t)i + (int64_t)(j0 + k) * jb.R;
-        acc += jb.M[e] * jb.M[e] + Mi[e] * Mi[e];
-      }
-      for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-      if (lane == 0) jb.nrm[j0 + k] = acc;
+  const int col = jb.dir > 0 ? hi : lo, i0 = jb.dir > 0 ? lo : hi, n = jb.n;
+  const int64_t cs = jb.dir > 0 ? jb.R : 1, is = jb.dir > 0 ? 1 : jb.R;
+  double acc = 0.0;
+  if (j0 + col < jb.o) {
+    const double* m = jb.M + (j0 + col) * cs;
+    const int64_t plane = jb.plane;
+#pragma unroll 8
+    for (int i = i0; i < n; i += 16) {
+      const double x = m[i * is], y = Z ? m[plane + i * is] : 0.0;
+      acc += Z ? x * x + y * y : x * x;
     }
+  }
+  part[col * 16 + i0] = acc;
+  __syncthreads();
+  if (threadIdx.x < 16 && j0 + (int)threadIdx.x < jb.o) {
+    double t = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t += part[threadIdx.x * 16 + i];
+    jb.nrm[j0 + threadIdx.x] = t;
   }
 }
 
-// perm[rank of column j] = j, norms descending, ties by index.
+// perm[rank of column j] = j, norms descending, ties by index: 16 columns a
+// group, a sixteenth of the comparisons a thread (a column a thread: 57 us at
+// 1024 columns, 6 now).
 __global__ __launch_bounds__(256) void k_qj_rank(const QjJob* __restrict__ jobs) {
+  __shared__ int part[256];
   const QjJob& jb = jobs[blockIdx.y];
-  const int j = blockIdx.x * 256 + threadIdx.x;
-  if (blockIdx.x * 256 >= jb.o) return;
-  __shared__ double buf[256];
-  const double x = j < jb.o ? jb.nrm[j] : 0.0;
+  const int lo = threadIdx.x & 15, hi = threadIdx.x >> 4, o = jb.o, j = blockIdx.x * 16 + lo;
+  if ((int)blockIdx.x * 16 >= o) return;
+  const double* nrm = jb.nrm;
+  const double x = j < o ? nrm[j] : 0.0;
   int rank = 0;
-  for (int k0 = 0; k0 < jb.o; k0 += 256) {
-    __syncthreads();
-    if (k0 + threadIdx.x < jb.o) buf[threadIdx.x] = jb.nrm[k0 + threadIdx.x];
-    __syncthreads();
-    const int kn = min(256, jb.o - k0);
-    for (int k = 0; k < kn; ++k) rank += buf[k] > x || (buf[k] == x && k0 + k < j);
+#pragma unroll 8
+  for (int k = hi; k < o; k += 16) {
+    const double y = nrm[k];
+    rank += (y > x) | ((y == x) & (k < j));
   }
-  if (j < jb.o) jb.perm[rank] = j;
+  part[hi * 16 + lo] = rank;
+  __syncthreads();
+  if (hi == 0 && j < o) {
+#pragma unroll
+    for (int k = 1; k < 16; ++k) rank += part[k * 16 + lo];
+    jb.perm[rank] = j;
+  }
 }
 
 // Panels of A0: sorted columns, scaled, zero-padded.
@@ -1086,8 +1092,12 @@ bool qj_solve(QjBatch& q, double norm2) {
   c.stage_flush();
   launch_fill(c, q.work + nn, q.nd, 0.0);
   const int pk = up16(maxK) / 16;
-  hipLaunchKernelGGL(k_qj_norms0, dim3((maxo + 63) / 64, nj), dim3(256), 0, c.stream, dj);
-  hipLaunchKernelGGL(k_qj_rank, dim3((maxo + 255) / 256, nj), dim3(256), 0, c.stream, dj);
+  const dim3 go((maxo + 15) / 16, nj);
+  if (z)
+    hipLaunchKernelGGL(k_qj_norms0<true>, go, dim3(256), 0, c.stream, dj);
+  else
+    hipLaunchKernelGGL(k_qj_norms0<false>, go, dim3(256), 0, c.stream, dj);
+  hipLaunchKernelGGL(k_qj_rank, go, dim3(256), 0, c.stream, dj);
   const dim3 gg(up16(maxo) / 16, nj, std::min(16, up16(maxn) / 16));
   if (z)
     hipLaunchKernelGGL(k_qj_gather<true>, gg, dim3(256), 0, c.stream, dj, scale);
