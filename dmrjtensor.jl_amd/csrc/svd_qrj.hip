@@ -819,10 +819,10 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           e.r[r] = (ti == tj && 4 * r + g == c ? 0.5 : 0.0) - 0.5 * e.r[r];
-          big |= fabs(e.r[r]) > 5e-9;
+          big |= !(fabs(e.r[r]) <= 5e-9);  // (not a number after a divergence)
           if constexpr (Z) {
             e.i[r] *= -0.5;
-            big |= fabs(e.i[r]) > 5e-9;
+            big |= !(fabs(e.i[r]) <= 5e-9);
           }
         }
         put(E, e);
@@ -838,8 +838,8 @@ __global__ __launch_bounds__(512) void k_qj_round(const QjJob* __restrict__ jobs
       __syncthreads();
     }
     if (!conv) {
-      // |X|_2 above 1.8, where the steps do not converge (32 columns of equal
-      // norms and products): at a quarter of the cap |X|_2 <= 0.7
+      // |X|_2 above 2.1, where the steps do not converge (32 columns of nearly
+      // equal norms and products): at a quarter of the cap |X|_2 <= 1.2
       if (cap < kCap) return;
       cap *= 0.25;
       continue;

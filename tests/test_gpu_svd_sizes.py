@@ -198,3 +198,32 @@ def test_svd_small_sides(pkg, ctx, shape, cplx, kind, direction):
         big = want > 1e-10 * want[0] if cplx else np.full(K, True)
         Q = (L if direction > 0 else Rt.conj().T)[:, big]
         assert np.max(np.abs(Q.conj().T @ Q - np.eye(big.sum()))) <= (8 + 2 * np.sqrt(n)) * EPS + 4 * K * EPS
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("shape", [(32, 40), (48, 64), (96, 160), (160, 96), (300, 280)])
+def test_svd_large_rotations(pkg, ctx, shape, cplx, direction):
+    """A step matrix: its panels hold columns of nearly equal norms and inner
+    products, whose simultaneous rotations have a spectral norm above the range
+    of the inner solve's Newton-Schulz steps; the solve has to notice the
+    divergence (overflow to not-a-number included) and shorten them."""
+    R, Cc = shape
+    rng = np.random.default_rng(R + Cc)
+    M = np.tril(np.ones((R, Cc))) + 1e-3 * rng.standard_normal((R, Cc))
+    if cplx:
+        M = np.exp(2j * np.pi * rng.random(R))[:, None] * M * np.exp(2j * np.pi * rng.random(Cc))[None, :]
+    M = M / np.linalg.norm(M)
+    n, K = max(R, Cc), min(R, Cc)
+    t = pkg.site2_from_dense(ctx, M.reshape(R, 1, 1, Cc))
+    l, r, te, kk = C.c_void_p(), C.c_void_p(), C.c_double(), C.c_int64()
+    sv = np.zeros(512)
+    ctx.call("dmrj_svd_trunc2", t.h, 0, 2, 0.0, direction, C.byref(l), C.byref(r), C.byref(te), C.byref(kk),
+             pkg._lib.dptr(sv), 512)
+    L = pkg.DeviceTensor(ctx, l).to_dense()[0].reshape(R, -1)
+    Rt = pkg.DeviceTensor(ctx, r).to_dense()[0].reshape(-1, Cc)
+    assert kk.value == K
+    assert np.max(np.abs(sv[:K] - np.linalg.svd(M, compute_uv=False))) <= 2 * n * EPS
+    assert np.max(np.abs(L @ Rt - M)) <= 8 * n * EPS
+    Q = L if direction > 0 else Rt.conj().T
+    assert np.max(np.abs(Q.conj().T @ Q - np.eye(K))) <= 1e-13 + 4 * n * EPS
