@@ -194,12 +194,17 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   // takes sides up to 16 (k_svd_tiny), above which the launches of the blocked
   // solver are the shorter chain (sides up to 64 in such a kernel: 2.43 ms for a
   // bond step with sectors to 55, up to 32: 1.01, up to 16: 0.77).
-  const int small_side = z || c.svd_backend == 0 ? 16 : 64;
+  // Backend 5 goes the same way: its Gram eigensolve was the fast route, now it
+  // is the slower one at every size (bond steps, block Jacobi against Gram:
+  // m=32 Heisenberg 0.37 and 0.63 ms, m=1024 6.4 and 13.2, m=510 Hubbard 2.7
+  // and 7.2, m=2048 28.4 and 45.7) and keeps what the block Jacobi leaves.
+  const bool jacobi = z || c.svd_backend == 0 || c.svd_backend == 5;
+  const int small_side = jacobi ? 16 : 64;
   // the kernel for sides up to 16 works on the matrices scaled to norm one by
   // a power of two (exact); not where the squared norm under- or overflows
   const bool in_range = aa2 > 1e-305 && aa2 < 1e305;
   double tiny_scale = 0.0;
-  if (small_side == 16 && in_range) {
+  if (jacobi && in_range) {
     int ex = 0;
     (void)std::frexp(std::sqrt(aa2), &ex);
     tiny_scale = std::ldexp(1.0, -ex);
@@ -220,14 +225,14 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     const double mm = (double)std::max(s.R, s.C), nn = (double)std::min(s.R, s.C);
     svd_flops += 4.0 * mm * nn * nn + 8.0 * nn * nn * nn;
   }
-  // larger sectors of the default backend and all complex ones: QR-preconditioned block Jacobi
+  // larger sectors of backends 0 and 5 and all complex ones: QR-preconditioned block Jacobi
   // (svd_qrj.hip) for the vectors of the side that must come out orthonormal;
   // the other factor by the grouped GEMM below.  Sectors it does not take
   // (longer than its register-resident slabs, or not converged within its
   // sweep limit) and tensors whose squared norm under- or overflows go to the
   // eigensolves of the augmented matrices.
   QjBatch qj(c, z);
-  if ((z || c.svd_backend == 0) && in_range) {
+  if (jacobi && in_range) {
     for (int si : order) {
       Sec& s = secs[si];
       if (s.kmin == 0 || is_small[si] || !qj_fits(s.R, s.C, z)) continue;
@@ -374,7 +379,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       const double mm = (double)std::max(s.R, s.C), nn = (double)s.kmin;
       svd_flops += 4.0 * mm * nn * nn + 8.0 * nn * nn * nn;
     }
-  // large sectors, backend 5: batched symmetric eigensolve of the Gram matrix
+  // what backend 5 has left: batched symmetric eigensolve of the Gram matrix
   // of the side that must come out orthonormal (M M^T for dir > 0, M^T M for
   // dir < 0: size n = R or C instead of R + C); eigenvalues sigma^2 carry an
   // absolute error ~eps |M|^2; the other factor by the grouped GEMM below

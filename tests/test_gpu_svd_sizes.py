@@ -227,3 +227,27 @@ def test_svd_large_rotations(pkg, ctx, shape, cplx, direction):
     assert np.max(np.abs(L @ Rt - M)) <= 8 * n * EPS
     Q = L if direction > 0 else Rt.conj().T
     assert np.max(np.abs(Q.conj().T @ Q - np.eye(K))) <= 1e-13 + 4 * n * EPS
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("shape", [(16, 12), (72, 40), (40, 2048), (2049, 20), (20, 2049)])
+def test_backend5_routes(pkg, ctx, shape, direction):
+    """Backend 5: the block Jacobi up to 2048 rows or columns (as the default),
+    the Gram eigensolve, sigma^2 to n eps |M|^2, above."""
+    R, Cc = shape
+    M = _matrix("flat", R, Cc, np.random.default_rng(R + Cc))
+    n, K = max(R, Cc), min(R, Cc)
+    ctx.set_svd_backend(5)
+    try:
+        L, Rt, sv = _factors(pkg, ctx, M, direction)
+    finally:
+        ctx.set_svd_backend(0)
+    want = np.linalg.svd(M, compute_uv=False)
+    assert len(sv) == K
+    if n > 2048:
+        assert np.max(np.abs(sv ** 2 - want ** 2)) <= 4 * n * EPS
+    else:
+        assert np.max(np.abs(sv - want)) <= 2 * n * EPS
+    assert np.max(np.abs(L @ Rt - M)) <= 8 * n * EPS
+    Q = L if direction > 0 else Rt.T
+    assert np.max(np.abs(Q.T @ Q - np.eye(K))) <= 1e-13 + 4 * n * EPS
