@@ -282,7 +282,10 @@ __device__ __forceinline__ void panel_column(Tile<Z> (&a)[TPW], int nt, bool top
   const double alphaz = Z ? row_bcast<J>(prz) : 0.0;
   double tau = 0.0, tauz = 0.0, beta = alpha, scale = 0.0, scalez = 0.0;
   const double xa = Z ? fma(alphaz, alphaz, xn) : xn;
-  if (xa > 0.0) {
+  // a residual below 1e-145 of the norm counts as zero (its elements are
+  // dropped, coef = -1 below): squares near the subnormal range have too few
+  // bits for a unitary reflector, and the reciprocals would overflow
+  if (xa > 1e-290) {
     const double h = fma(alpha, alpha, xa);
     const double ri = copysign(fast_rsqrt(h), -alpha);  // 1 / beta
     beta = h * ri;
