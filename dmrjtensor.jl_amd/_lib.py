@@ -42,6 +42,7 @@ SIGNATURES = {
     "dmrj_ctx_flops": [_p, _dp, C.c_int],
     "dmrj_ctx_profile": [_p, C.c_int],
     "dmrj_ctx_set_svd_backend": [_p, C.c_int],
+    "dmrj_ctx_set_jacobi_sweeps": [_p, C.c_int],
     "dmrj_ctx_set_env_precision": [_p, C.c_int],
     "dmrj_ctx_last_residual": [_p, _dp],
     "dmrj_selftest_mfma_bf16": [_p, C.POINTER(C.c_float)],
@@ -186,6 +187,9 @@ class Context:
 
     def set_svd_backend(self, mode):
         self.call("dmrj_ctx_set_svd_backend", int(mode))
+
+    def set_jacobi_sweeps(self, limit):
+        self.call("dmrj_ctx_set_jacobi_sweeps", int(limit))
 
     def set_gemm_cfg(self, cfg):
         self.call("dmrj_ctx_set_gemm_cfg", int(cfg))

@@ -1748,6 +1748,13 @@ int dmrj_ctx_set_svd_backend(dmrj_ctx* c, int mode) {
   });
 }
 
+int dmrj_ctx_set_jacobi_sweeps(dmrj_ctx* c, int limit) {
+  return guard(c, [&] {
+    if (limit < 0 || limit > 40) throw Error(DMRJ_ERR_ARG, "block Jacobi sweep limit must be 0..40");
+    c->jacobi_sweeps = limit;
+  });
+}
+
 int dmrj_ctx_set_eig_batching(dmrj_ctx* c, int mode) {
   return guard(c, [&] {
     if (mode < 0 || mode > 3) throw Error(DMRJ_ERR_ARG, "eigensolve batching mode must be 0..3");

@@ -236,6 +236,7 @@ struct Context {
   // block Jacobi for large ones, 1 = gesdd,
   // 2 = gesvd, 3 = batched Jacobi for small sectors + gesvd
   int svd_backend = 0;
+  int jacobi_sweeps = 40;  // sweep limit of the QR-preconditioned block Jacobi (0: not used)
   double bj_calls = 0, bj_sweeps = 0;  // block-Jacobi SVD calls and sweeps
   int env_prec = 0;  // precision of environment updates
   int last_gemm_cfg = -1;
@@ -413,7 +414,9 @@ struct QjSector {
   // vectors have n elements), K = min(n, o)
   const double* M = nullptr;
   int R = 0, o = 0, n = 0, K = 0, dir = 0, index = 0;
-  // set by qj_solve: singular values descending, their columns, reciprocals
+  // set by qj_solve: converged to finite values; singular values descending,
+  // their columns, reciprocals
+  bool ok = false;
   std::vector<double> sigma, inv;
   std::vector<int> col;
   // set by the caller before qj_vectors
@@ -437,7 +440,7 @@ struct QjBatch {
 };
 bool qj_fits(int64_t R, int64_t C, bool cplx);  // sector sizes the register-resident kernels take
 void qj_prepare(QjBatch& q);
-bool qj_solve(QjBatch& q, double norm2);
+void qj_solve(QjBatch& q, double norm2);
 void qj_vectors(QjBatch& q);
 
 // A new tensor handle of the given kind (0 site, 1 left env, 2 right env) and

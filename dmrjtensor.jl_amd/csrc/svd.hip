@@ -232,7 +232,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   // sweep limit) and tensors whose squared norm under- or overflows go to the
   // eigensolves of the augmented matrices.
   QjBatch qj(c, z);
-  if (jacobi && in_range) {
+  if (jacobi && in_range && c.jacobi_sweeps > 0) {
     for (int si : order) {
       Sec& s = secs[si];
       if (s.kmin == 0 || is_small[si] || !qj_fits(s.R, s.C, z)) continue;
@@ -370,8 +370,10 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       }
     }
   }
-  if (!qj.sec.empty() && qj_solve(qj, aa2))
+  if (!qj.sec.empty()) {
+    qj_solve(qj, aa2);
     for (size_t b = 0; b < qj.sec.size(); ++b) {
+      if (!qj.sec[b].ok) continue;
       Sec& s = secs[qj.sec[b].index];
       s.qj = (int)b;
       s.bj = 1;
@@ -379,6 +381,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       const double mm = (double)std::max(s.R, s.C), nn = (double)s.kmin;
       svd_flops += 4.0 * mm * nn * nn + 8.0 * nn * nn * nn;
     }
+  }
   // what backend 5 has left: batched symmetric eigensolve of the Gram matrix
   // of the side that must come out orthonormal (M M^T for dir > 0, M^T M for
   // dir < 0: size n = R or C instead of R + C); eigenvalues sigma^2 carry an
@@ -469,7 +472,11 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   int nqr = 0;
   if (z) {
     // complex, what the block Jacobi has left: batched Hermitian eigensolves
-    // of [[0, M], [M^H, 0]] (eigenvalues +-sigma), batched by size (eig_classes)
+    // of [[0, M], [M^H, 0]] (eigenvalues +-sigma).  Sectors of equal size share
+    // a batch, whatever the batching mode, and none is padded: rocSOLVER's
+    // zheevd (divide and conquer) returns not-a-number vectors with a success
+    // code where rows of the matrix vanish.  Sectors with such rows of their
+    // own are solved again by zheev (QR iterations), which does not.
     std::vector<int> big;
     for (int si : order) {
       Sec& s = secs[si];
@@ -482,7 +489,10 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       naug = (int)big.size();
       std::vector<int> nsz(naug);
       for (int b = 0; b < naug; ++b) nsz[b] = (int)(secs[big[b]].R + secs[big[b]].C);
-      const std::vector<int> cls = eig_classes(nsz, c.eig_batching);
+      std::vector<int> cls;
+      for (int b = 0; b < naug; ++b)
+        if (b == 0 || nsz[b] != nsz[b - 1] || c.eig_batching == 2) cls.push_back(b);
+      cls.push_back(naug);
       const int ncls = (int)cls.size() - 1;
       std::vector<int64_t> aoff(ncls + 1, 0), voff(ncls + 1, 0);
       for (int k = 0; k < ncls; ++k) {
@@ -518,6 +528,37 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
         if (st != rocblas_status_success) throw Error(DMRJ_ERR_SOLVER, "rocsolver_zheevd_strided_batched failed");
       }
       launch_aug_extract_z(c, jobs);
+      double* chk = (double*)c.alloc.alloc(2 * naug * sizeof(double));  // squared norms of the factors
+      std::vector<double> hchk(2 * naug);
+      for (int retry = 0; retry < 2; ++retry) {
+        for (int b = 0; b < naug; ++b) {
+          const Sec& s = secs[big[b]];
+          const double* xs[1] = {s.U};
+          launch_dots(c, 1, xs, xs, 2 * s.R * s.kmin, chk + 2 * b);
+          xs[0] = s.Vt;
+          launch_dots(c, 1, xs, xs, 2 * s.kmin * s.C, chk + 2 * b + 1);
+        }
+        HIP_OK(hipMemcpyAsync(hchk.data(), chk, 2 * naug * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+        HIP_OK(hipStreamSynchronize(c.stream));
+        std::vector<AugJobZ> again;
+        for (int k = 0; k < ncls; ++k)
+          for (int b = cls[k]; b < cls[k + 1]; ++b) {
+            if (std::isfinite(hchk[2 * b]) && std::isfinite(hchk[2 * b + 1])) continue;
+            if (retry) throw Error(DMRJ_ERR_SOLVER, "rocsolver Hermitian eigensolver returned non-finite vectors");
+            const AugJobZ& jb = jobs[b];
+            launch_fill(c, (double*)jb.Z, 2 * (int64_t)jb.N * jb.N, 0.0);
+            launch_aug_place_z(c, {jb});
+            rocblas_status st = rocsolver_zheev(hb, rocblas_evect_original, rocblas_fill_upper, jb.N,
+                                                (rocblas_double_complex*)jb.Z, jb.N,
+                                                augW + voff[k] + (int64_t)(b - cls[k]) * jb.N,
+                                                augE + voff[k] + (int64_t)(b - cls[k]) * jb.N, auginfo + b);
+            if (st != rocblas_status_success) throw Error(DMRJ_ERR_SOLVER, "rocsolver_zheev failed");
+            again.push_back(jb);
+          }
+        if (again.empty()) break;
+        launch_aug_extract_z(c, again);
+      }
+      c.alloc.release(chk);
     }
   } else if (c.svd_backend == 0) {
     std::vector<int> big, qrs;

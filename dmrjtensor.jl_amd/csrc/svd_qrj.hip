@@ -1072,10 +1072,9 @@ void qj_prepare(QjBatch& q) {
 }
 
 // Factorisations, Jacobi sweeps and column norms of all sectors; sigma and
-// col of every sector receive the column norms (unscaled) in descending order
-// and the column each belongs to.  Returns false when a sector did not
-// converge within the sweep limit.
-bool qj_solve(QjBatch& q, double norm2) {
+// col of every sector that converged within the sweep limit (ok) receive the
+// column norms (unscaled) in descending order and the column each belongs to.
+void qj_solve(QjBatch& q, double norm2) {
   Context& c = q.c;
   std::vector<QjSector>& sec = q.sec;
   const int nj = (int)sec.size();
@@ -1137,7 +1136,7 @@ bool qj_solve(QjBatch& q, double norm2) {
   const int chunk = nbmax / 2;
   const double tol = std::max(1e-14, 4.0 * 2.220446049250313e-16 * std::sqrt((double)maxK));
   const double fl = 1e-11;  // relative to |AA|, which the scaling puts in [1/2, 1)
-  constexpr int kMaxSweeps = 40;
+  const int limit = c.jacobi_sweeps * (nbmax - 1);
   int step = 0;
   bool done = false;
   int* hlast = (int*)c.host_sigma((nj + 1) / 2 + 1);
@@ -1148,21 +1147,22 @@ bool qj_solve(QjBatch& q, double norm2) {
       else
         hipLaunchKernelGGL(k_qj_round<false>, dim3(nbmax / 2, nj), dim3(512), 0, c.stream, dj, step, tol * tol, fl * fl);
   };
-  for (int k = 0; k < 10 && step < 5 * (nbmax - 1); ++k) rounds();  // five sweeps are always needed
-  while (!done && step < kMaxSweeps * (nbmax - 1)) {
+  while (step < std::min(limit, 5 * (nbmax - 1))) rounds();  // five sweeps are always needed
+  for (bool more = true; more && !done;) {
     const int upto = step;
     HIP_OK(hipMemcpyAsync(hlast, q.ints, nj * sizeof(int), hipMemcpyDeviceToHost, c.stream));
     HIP_OK(hipEventRecord(c.poll, c.stream));
-    rounds();
+    more = step < limit;
+    if (more) rounds();
     HIP_OK(hipEventSynchronize(c.poll));
     done = true;
     for (int j = 0; j < nj; ++j) {
       const int nb = (std::max(2, up16(sec[j].K) / 16) + 1) & ~1;
-      done = done && upto - 1 - hlast[j] >= nb - 1;
+      sec[j].ok = upto - 1 - hlast[j] >= nb - 1;
+      done = done && sec[j].ok;
     }
   }
   HIP_OK(hipGetLastError());
-  if (!done) return false;
   if (z)
     hipLaunchKernelGGL(k_qj_norms2<true>, dim3(pk, nj), dim3(256), 0, c.stream, dj);
   else
@@ -1173,6 +1173,8 @@ bool qj_solve(QjBatch& q, double norm2) {
   for (int j = 0; j < nj; ++j) {
     QjSector& s = sec[j];
     const double* v = h + (q.jobs[j].nrm - q.work);
+    for (int i = 0; i < up16(s.K); ++i) s.ok = s.ok && std::isfinite(v[i]);
+    if (!s.ok) continue;
     s.col.resize(up16(s.K));
     for (int i = 0; i < (int)s.col.size(); ++i) s.col[i] = i;
     std::stable_sort(s.col.begin(), s.col.end(), [&](int a, int b) { return v[a] > v[b]; });
@@ -1184,7 +1186,6 @@ bool qj_solve(QjBatch& q, double norm2) {
       s.inv[i] = v[s.col[i]] > 0.0 ? 1.0 / v[s.col[i]] : 0.0;
     }
   }
-  return true;
 }
 
 // The first `keep` vectors of every sector (keep, out, es, vs set by the

@@ -64,8 +64,8 @@ int dmrj_ctx_sync(dmrj_ctx* ctx);
 int dmrj_version(void);
 /* memory statistics: bytes live, bytes cached, peak bytes */
 int dmrj_ctx_memstats(dmrj_ctx* ctx, int64_t* out3);
-/* Batching of the SVD's batched symmetric eigensolves (backend 5, complex
- * tensors and what backend 0 leaves to them; no
+/* Batching of the SVD's batched symmetric eigensolves, which take what the
+ * block Jacobi of backends 0 and 5 leaves (dmrj_ctx_set_svd_backend; no
  * counterpart in the reference, whose SVD runs sector by sector): 1 (default)
  * = sectors sorted by size and cut into batches, each padded to its own
  * largest size, where a cost model of the tridiagonalisation (fixed latency
@@ -73,7 +73,8 @@ int dmrj_ctx_memstats(dmrj_ctx* ctx, int64_t* out3);
  * outweighs the extra steps; 0 = one batch padded to the largest sector;
  * 2 = one batch per sector; 3 = batches of two sectors in size order (a test
  * mode: every batch offset path is taken on small problems).  Every mode
- * gives a backward-stable result; the bits differ between modes. */
+ * gives a backward-stable result; the bits differ between modes.  Complex
+ * sectors are not padded: those of equal size share a batch (mode 2: none do). */
 int dmrj_ctx_set_eig_batching(dmrj_ctx* ctx, int mode);
 /* force a GEMM tile shape (0: 32x32, 1: 64x64, 2: 128x128, 3: 64x128,
  * 4: 128x64, -1: automatic) */
@@ -118,11 +119,11 @@ int dmrj_ctx_graph_stats(dmrj_ctx* ctx, double* out2);
 int dmrj_ctx_marker(dmrj_ctx* ctx, int id);
 /* SVD backend of dmrj_svd_trunc2 / dmrj_twostep: 0 (default) = batched
  * one-sided Jacobi for sectors with min(R,C) <= 16, QR-preconditioned block
- * Jacobi for the larger ones (FP64 on the matrix cores); a sector longer
- * than 2048 on a side, or one that does not converge within the sweep limit,
- * takes a batched symmetric eigensolve of the augmented matrix [[0,M],[M^T,0]]
+ * Jacobi for the larger ones (FP64 on the matrix cores); the sectors longer
+ * than 2048 on a side, and those that do not converge within the sweep limit,
+ * take a batched symmetric eigensolve of the augmented matrix [[0,M],[M^T,0]]
  * (if at least 1.5 times longer than the side that must come out orthonormal,
- * of its K x K LQ / QR triangle);
+ * of their K x K LQ / QR triangle);
  * 1 = rocSOLVER gesdd per sector, 2 = gesvd per sector, 3 = batched Jacobi +
  * gesvd, 4 = batched Jacobi for small sectors + batched block one-sided
  * Jacobi (columns of M or M^T in LDS-resident block pairs) for the larger
@@ -135,10 +136,15 @@ int dmrj_ctx_marker(dmrj_ctx* ctx, int id);
  * size min-side instead of R + C), the other factor by a grouped GEMM with
  * M: exactly orthonormal factor, singular values with absolute error
  * ~eps |M|^2 (for those sectors not the FP64 drop-in's accuracy: small sigma
- * and truncation errors near a cutoff differ from LAPACK's).  Complex tensors of
- * sides up to 1024 always use the QR-preconditioned block Jacobi, longer ones a
- * batched Hermitian eigensolve of [[0,M],[M^H,0]]. */
+ * and truncation errors near a cutoff differ from LAPACK's).  Complex tensors
+ * always go as with 0: one-sided Jacobi to 16, block Jacobi to 1024, and what
+ * is longer or has not converged through Hermitian eigensolves of
+ * [[0,M],[M^H,0]] (vectors that come back non-finite are DMRJ_ERR_SOLVER). */
 int dmrj_ctx_set_svd_backend(dmrj_ctx* ctx, int mode);
+/* Sweep limit of the QR-preconditioned block Jacobi, 0..40 (default 40; 7 to 8
+ * are needed): sectors that have not converged by then take the eigensolves
+ * named above, 0 = all of them do.  No reference counterpart. */
+int dmrj_ctx_set_jacobi_sweeps(dmrj_ctx* ctx, int limit);
 /* out2 = {SVD calls that used the block one-sided Jacobi, total sweeps of
  * those calls}; reset != 0 clears the counters.  No reference counterpart. */
 int dmrj_ctx_svd_stats(dmrj_ctx* ctx, double* out2, int reset);

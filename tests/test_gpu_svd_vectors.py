@@ -59,3 +59,117 @@ def test_residuals_below_the_range_of_squares(pkg, ctx, tiny, cplx, direction):
     assert np.max(np.abs(sv - want)) <= 2 * n * EPS
     assert np.max(np.abs(L @ Rt - M)) <= 8 * n * EPS
     assert _isometry(L, Rt, direction) <= 1e-13 + 4 * n * EPS
+
+
+def _charged(cplx, rng, dims, rdims=None, edit=None):
+    """A two-site tensor of spins 1/2 whose bonds hold dims[q] (right: rdims[q])
+    states of charge q, and the matrix of its centre sectors; edit(Q, sector)
+    changes a sector."""
+    ql, qr = (np.array([[c] for c in sorted(d) for _ in range(d[c])], dtype=np.int32) for d in (dims, rdims or dims))
+    qp = np.array([[1], [-1]], dtype=np.int32)
+    row = (ql[:, 0][:, None] + qp[:, 0][None, :]).ravel()
+    col = (qr[:, 0][None, :] - qp[:, 0][:, None]).ravel()
+    M = np.zeros((len(row), len(col)), dtype=complex if cplx else float)
+    sectors = {}
+    for Q in sorted(set(row) & set(col)):
+        at = np.ix_(np.flatnonzero(row == Q), np.flatnonzero(col == Q))
+        S = rng.standard_normal((len(at[0]), at[1].size)) / len(row)
+        if cplx:
+            S = _phases(S, rng)
+        M[at] = S if edit is None else edit(int(Q), S)
+        sectors[int(Q)] = at
+    return M.reshape(len(ql), 2, 2, len(qr)), (ql, qp, qp, qr, 1), M, sectors
+
+
+DIMS = {-4: 7, -2: 12, 0: 40, 2: 27, 4: 3}
+
+
+def _check_sectors(M, sectors, L, Rt, sv, direction):
+    """Values, products and the isometry, every sector to its own norm."""
+    n = max(at[0].size + at[1].size for at in sectors.values()) // 2
+    P = L @ Rt
+    norm = np.linalg.norm(M)
+    assert np.all(np.isfinite(L)) and np.all(np.isfinite(Rt))
+    want = []
+    for at in sectors.values():
+        w = np.linalg.svd(M[at], compute_uv=False)
+        want += [(x, np.linalg.norm(w)) for x in w]
+        assert np.max(np.abs(P[at] * norm - M[at])) <= 16 * n * EPS * np.linalg.norm(w)
+    want.sort(key=lambda p: -p[0])
+    assert len(sv) == len(want)
+    for got, (w, scale) in zip(sv, want):
+        assert abs(got * norm - w) <= 4 * n * EPS * scale
+    assert _isometry(L, Rt, direction) <= 1e-13 + 4 * n * EPS
+
+
+WIDE = {-4: 15, -2: 30, 0: 90, 2: 55, 4: 8}
+TWINS = {-2: 20, 0: 31, 2: 20}   # sectors of 20, 51, 51 and 20 rows
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("bonds", [(DIMS, DIMS), (DIMS, WIDE), (TWINS, TWINS)], ids=["square", "wide", "twins"])
+@pytest.mark.parametrize("batching", [0, 1, 2, 3])
+@pytest.mark.parametrize("kind", ["complex"])
+def test_eigensolves_of_several_sectors(pkg, ctx, kind, batching, bonds, direction):
+    """What the block Jacobi leaves to the eigensolves (all of it here): sectors
+    of six sizes, or of two sizes twice, in one call, every way of batching
+    them.  The Gram form is accurate to n eps in the squares of the values."""
+    A, charges, M, sectors = _charged(kind == "complex", np.random.default_rng(29), *bonds)
+    t = pkg.site2_from_dense(ctx, A, *charges)
+    ctx.set_jacobi_sweeps(0)
+    ctx.set_eig_batching(batching)
+    ctx.set_svd_backend(5 if kind == "gram" else 0)
+    try:
+        L, Rt, sv = _svd(pkg, ctx, t, 1, direction)
+    finally:
+        ctx.set_jacobi_sweeps(40)
+        ctx.set_eig_batching(1)
+        ctx.set_svd_backend(0)
+    if kind != "gram":
+        _check_sectors(M, sectors, L, Rt, sv, direction)
+        return
+    norm, n = np.linalg.norm(M), max(M.shape)
+    want = np.sort(np.concatenate([np.linalg.svd(M[at], compute_uv=False) for at in sectors.values()]))[::-1] / norm
+    assert np.max(np.abs(sv ** 2 - want ** 2)) <= 4 * n * EPS
+    assert np.max(np.abs(L @ Rt * norm - M)) <= 8 * n * EPS * norm
+    assert _isometry(L, Rt, direction) <= 1e-13 + 4 * n * EPS
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("shape", [(40, 33), (33, 70), (130, 257)])
+def test_eigensolve_of_sectors_with_zero_rows(pkg, ctx, shape, cplx, direction):
+    """Rows and columns of zeros in what is left to the eigensolves: finite
+    factors whose product is the tensor."""
+    R, Cc = shape
+    rng = np.random.default_rng(R + Cc)
+    M = np.zeros((R, Cc))
+    M[1:1 + R // 3, :Cc // 4] = rng.standard_normal((R // 3, Cc // 4))
+    if cplx:
+        M = _phases(M, rng)
+    M = M / np.linalg.norm(M)
+    n = max(R, Cc)
+    ctx.set_jacobi_sweeps(0)
+    try:
+        L, Rt, sv = _dense(pkg, ctx, M, direction)
+    finally:
+        ctx.set_jacobi_sweeps(40)
+    assert np.max(np.abs(sv - np.linalg.svd(M, compute_uv=False))) <= 4 * n * EPS
+    assert np.max(np.abs(L @ Rt - M)) <= 16 * n * EPS
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("limit", [1, 2, 4])
+def test_sectors_that_do_not_converge(pkg, ctx, limit, cplx, direction):
+    """Sweep limits that the diagonal sector keeps and the others do not: what
+    has converged stays, the others take the eigensolves."""
+    A, charges, M, sectors = _charged(cplx, np.random.default_rng(31), DIMS,
+                                      edit=lambda q, S: np.diag(np.linspace(0.3, 1.0, len(S))) if q == -1 else S)
+    t = pkg.site2_from_dense(ctx, A, *charges)
+    ctx.set_jacobi_sweeps(limit)
+    try:
+        L, Rt, sv = _svd(pkg, ctx, t, 1, direction)
+    finally:
+        ctx.set_jacobi_sweeps(40)
+    _check_sectors(M, sectors, L, Rt, sv, direction)
