@@ -109,7 +109,7 @@ TWINS = {-2: 20, 0: 31, 2: 20}   # sectors of 20, 51, 51 and 20 rows
 @pytest.mark.parametrize("direction", [1, -1])
 @pytest.mark.parametrize("bonds", [(DIMS, DIMS), (DIMS, WIDE), (TWINS, TWINS)], ids=["square", "wide", "twins"])
 @pytest.mark.parametrize("batching", [0, 1, 2, 3])
-@pytest.mark.parametrize("kind", ["complex"])
+@pytest.mark.parametrize("kind", ["real", "gram", "complex"])
 def test_eigensolves_of_several_sectors(pkg, ctx, kind, batching, bonds, direction):
     """What the block Jacobi leaves to the eigensolves (all of it here): sectors
     of six sizes, or of two sizes twice, in one call, every way of batching
