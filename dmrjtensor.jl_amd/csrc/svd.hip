@@ -185,6 +185,26 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
       throw Error(DMRJ_ERR_NUMERIC, "two-site tensor holds NaN/Inf; SVD not attempted");
     }
   }
+  // A tensor whose squared norm leaves the normal range is gathered again
+  // times 2^512 or 2^-512: products of its elements would lose their digits in
+  // every solver (sectors of 3 .. 67 rows, norm 3e-154: factors off by the norm
+  // itself).  All that follows is in these units but the discarded weight.
+  double unit = 1.0;
+  if (aa2 <= 1e-305 || aa2 >= 1e305) {
+    unit = std::ldexp(1.0, aa2 < 1.0 ? 512 : -512);
+    for (CopyOp& g : gather) g.alpha = unit;
+    launch_copy(c, gather);
+    aa2 = 0.0;
+    for (int si : order) {
+      const Sec& s = secs[si];
+      if (s.kmin == 0) continue;
+      const double* xs[1] = {s.M};
+      launch_dots(c, 1, xs, xs, s.R * s.C * zf, c.scal + S_CHK);
+      HIP_OK(hipMemcpyAsync(&c.hscal[S_CHK], c.scal + S_CHK, sizeof(double), hipMemcpyDeviceToHost, c.stream));
+      HIP_OK(hipStreamSynchronize(c.stream));
+      aa2 += c.hscal[S_CHK];
+    }
+  }
   auto* hb = (rocblas_handle)c.rocblas;
   rocblas_int* info = (rocblas_int*)c.alloc.alloc(sizeof(rocblas_int) * std::max<size_t>(1, secs.size()));
   int nsvd = 0;
@@ -201,7 +221,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   const bool jacobi = z || c.svd_backend == 0 || c.svd_backend == 5;
   const int small_side = jacobi ? 16 : 64;
   // the kernel for sides up to 16 works on the matrices scaled to norm one by
-  // a power of two (exact); not where the squared norm under- or overflows
+  // a power of two (exact); not where there is no norm
   const bool in_range = aa2 > 1e-305 && aa2 < 1e305;
   double tiny_scale = 0.0;
   if (jacobi && in_range) {
@@ -229,8 +249,8 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   // (svd_qrj.hip) for the vectors of the side that must come out orthonormal;
   // the other factor by the grouped GEMM below.  Sectors it does not take
   // (longer than its register-resident slabs, or not converged within its
-  // sweep limit) and tensors whose squared norm under- or overflows go to the
-  // eigensolves of the augmented matrices.
+  // sweep limit) and tensors of zeros go to the eigensolves of the augmented
+  // matrices.
   QjBatch qj(c, z);
   if (jacobi && in_range && c.jacobi_sweeps > 0) {
     for (int si : order) {
@@ -851,7 +871,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   const int64_t n = (int64_t)ents.size();
   int64_t keep = n;
   double acc = 0.0;
-  while (keep > 0 && acc + ents[keep - 1].v * ents[keep - 1].v < cutoff) {
+  while (keep > 0 && (acc + ents[keep - 1].v * ents[keep - 1].v) / unit / unit < cutoff) {
     acc += ents[keep - 1].v * ents[keep - 1].v;
     --keep;
   }
@@ -861,7 +881,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
   double terr = 0.0, kept2 = 0.0;
   for (int64_t i = keep; i < n; ++i) terr += ents[i].v * ents[i].v;
   for (int64_t i = 0; i < keep; ++i) kept2 += ents[i].v * ents[i].v;
-  res.truncerr = terr;
+  res.truncerr = terr / unit / unit;
   const double renorm = kept2 > 0 ? 1.0 / std::sqrt(kept2) : 1.0;
   // kept counts per sector (values within a sector are descending, so the
   // kept set of a sector is a prefix)

@@ -173,3 +173,25 @@ def test_sectors_that_do_not_converge(pkg, ctx, limit, cplx, direction):
     finally:
         ctx.set_jacobi_sweeps(40)
     _check_sectors(M, sectors, L, Rt, sv, direction)
+
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("scale", [1e-170, 3e-154, 1e153])
+def test_squared_norm_out_of_range(pkg, ctx, scale, cplx, direction):
+    """Norms whose squares are no normal numbers, sectors of 3 .. 67 rows; and the
+    weight that a truncation discards, in the tensor's own units."""
+    A, charges, M, sectors = _charged(cplx, np.random.default_rng(37), DIMS)
+    f = scale / np.linalg.norm(M)
+    t = pkg.site2_from_dense(ctx, A * f, *charges)
+    L, Rt, sv = _svd(pkg, ctx, t, 1, direction)
+    _check_sectors(M, sectors, L, Rt, sv, direction)
+    te, kept = C.c_double(), 100
+    l, r, kk = C.c_void_p(), C.c_void_p(), C.c_int64()
+    ctx.call("dmrj_svd_trunc2", t.h, kept, 2, 0.0, direction, C.byref(l), C.byref(r), C.byref(te), C.byref(kk),
+             pkg._lib.dptr(sv), len(sv))
+    want = np.sort(np.concatenate([np.linalg.svd(M[at], compute_uv=False) for at in sectors.values()]))[::-1]
+    want = want / np.linalg.norm(want) * scale
+    # (squares of 1e-154 are subnormal: half a unit of 5e-324)
+    assert abs(te.value - np.sum(want[kept:] ** 2)) <= 1e-12 * np.sum(want[kept:] ** 2) + 1e-322
