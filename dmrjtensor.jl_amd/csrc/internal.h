@@ -400,7 +400,8 @@ struct QjJob {
   int64_t plane;          // distance of its imaginary plane (0 for real tensors)
   double* A[3];           // working panels: n x o, o x K, K x K
   double* T[2];           // triangular factors of the block reflectors, 256 doubles a panel
-  double* nrm;            // column norms: of A0 (squares, o), then of A2 (16 per panel)
+  double* nrm;            // column norms: of A0 (squares, o), then of A2 (16 per panel); behind o's
+                          // last panel of 16 the power of two that scaled the sector
   int* perm;              // o: column of A0 at every place of the sorted order
   int* last;              // last Jacobi round that rotated
   const int* kcol;        // kept columns of A2, in the order of the vectors

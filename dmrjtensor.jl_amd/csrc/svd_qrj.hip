@@ -282,7 +282,7 @@ __device__ __forceinline__ void panel_column(Tile<Z> (&a)[TPW], int nt, bool top
   const double alphaz = Z ? row_bcast<J>(prz) : 0.0;
   double tau = 0.0, tauz = 0.0, beta = alpha, scale = 0.0, scalez = 0.0;
   const double xa = Z ? fma(alphaz, alphaz, xn) : xn;
-  // a residual below 1e-145 of the norm counts as zero (its elements are
+  // a residual below 1e-145 of the sector's norm counts as zero (its elements are
   // dropped, coef = -1 below): squares near the subnormal range have too few
   // bits for a unitary reflector, and the reciprocals would overflow
   if (xa > 1e-290) {
@@ -486,12 +486,12 @@ __global__ __launch_bounds__(NW * 64) void k_qj_qr(const QjJob* __restrict__ job
   }
 }
 
-// Squared column norms of A0 (columns of M for dir > 0, rows for dir < 0): 16
+// Squared column norms of scale A0 (columns of M for dir > 0, rows for dir < 0): 16
 // columns and 16 interleaved sequences of rows a group, which reads whole
 // 128-byte lines in both directions (a wave a column or 64 columns a wave:
 // 42 us at 400 x 400, 5 now).
 template <bool Z>
-__global__ __launch_bounds__(256) void k_qj_norms0(const QjJob* __restrict__ jobs) {
+__global__ __launch_bounds__(256) void k_qj_norms0(const QjJob* __restrict__ jobs, double scale) {
   __shared__ double part[256];
   const QjJob& jb = jobs[blockIdx.y];
   const int j0 = blockIdx.x * 16, lo = threadIdx.x & 15, hi = threadIdx.x >> 4;
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(256) void k_qj_norms0(const QjJob* __restrict__ job
     const int64_t plane = jb.plane;
 #pragma unroll 8
     for (int i = i0; i < n; i += 16) {
-      const double x = m[i * is], y = Z ? m[plane + i * is] : 0.0;
+      const double x = scale * m[i * is], y = Z ? scale * m[plane + i * is] : 0.0;
       acc += Z ? x * x + y * y : x * x;
     }
   }
@@ -544,12 +544,40 @@ __global__ __launch_bounds__(256) void k_qj_rank(const QjJob* __restrict__ jobs)
   }
 }
 
-// Panels of A0: sorted columns, scaled, zero-padded.
+// Panels of A0: sorted columns, scaled, zero-padded.  `scale` brings the norm
+// of the tensor to order one, the factor found here that of the sector: what
+// the solver counts as zero is relative to the sector's own norm, so the values
+// and vectors of a weak sector are as accurate as a strong one's (a factor for
+// the whole tensor left sectors below 1e-11 of its norm unrotated).  The factor
+// goes to the host behind the column norms.  Every group sums all norms itself;
+// sectors below 1e-140 of the tensor's norm keep its factor.
 template <bool Z>
 __global__ __launch_bounds__(256) void k_qj_gather(const QjJob* __restrict__ jobs, double scale) {
+  __shared__ double part[256], sums[16];
   const QjJob& jb = jobs[blockIdx.y];
   const int p = blockIdx.x;
   if (p >= blocks16(jb.o)) return;
+  {
+    double t = 0.0;
+    for (int j = threadIdx.x; j < jb.o; j += 256) t += jb.nrm[j];
+    part[threadIdx.x] = t;
+    __syncthreads();
+    if (threadIdx.x < 16) {
+      t = 0.0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) t += part[threadIdx.x * 16 + i];
+      sums[threadIdx.x] = t;
+    }
+    __syncthreads();
+    t = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t += sums[i];
+    int ex = 0;
+    if (t > 1e-280) (void)frexp(sqrt(t), &ex);
+    const double factor = ldexp(1.0, -ex);
+    if (p == 0 && blockIdx.z == 0 && threadIdx.x == 0) jb.nrm[16 * blocks16(jb.o)] = factor;
+    scale *= factor;
+  }
   const int rb = blocks16(jb.n), c = threadIdx.x & 15, rr = threadIdx.x >> 4;
   const int col = p * 16 + c < jb.o ? jb.perm[p * 16 + c] : -1;
   double* dst = jb.A[0] + (int64_t)p * rb * kTile<Z> + threadIdx.x;
@@ -1026,7 +1054,7 @@ void qj_prepare(QjBatch& q) {
   const int nj = (int)sec.size();
   // largest first: a launch's grid covers the jobs that still take part
   std::stable_sort(sec.begin(), sec.end(), [](const QjSector& a, const QjSector& b) { return a.o > b.o; });
-  // doubles: the norms of all sectors (one copy to the host), then the
+  // doubles: the norms and the factor of all sectors (one copy to the host), then the
   // matrices; ints: the round counters of all sectors, then the orders
   const bool z = q.cplx;
   const int zf = z ? 2 : 1;
@@ -1036,7 +1064,7 @@ void qj_prepare(QjBatch& q) {
   for (int j = 0; j < nj; ++j) {
     const int64_t o = up16(sec[j].o), n = up16(sec[j].n), K = up16(sec[j].K), Kc = kcols(sec[j].K);
     nof[j] = nn;
-    nn += o;
+    nn += o + 16;
     dof[j] = nd;
     nd += zf * (n * o + o * Kc + K * Kc + 2 * 16 * K);
     iof[j] = ni;
@@ -1078,7 +1106,7 @@ void qj_solve(QjBatch& q, double norm2) {
   Context& c = q.c;
   std::vector<QjSector>& sec = q.sec;
   const int nj = (int)sec.size();
-  // powers of two, exact: norms of order one whatever the tensor's scale
+  // powers of two, exact: norms of order one whatever the tensor's scale (k_qj_gather adds the sector's)
   int ex = 0;
   (void)std::frexp(std::sqrt(norm2), &ex);
   const double scale = std::ldexp(1.0, -ex);
@@ -1096,9 +1124,9 @@ void qj_solve(QjBatch& q, double norm2) {
   const int pk = up16(maxK) / 16;
   const dim3 go((maxo + 15) / 16, nj);
   if (z)
-    hipLaunchKernelGGL(k_qj_norms0<true>, go, dim3(256), 0, c.stream, dj);
+    hipLaunchKernelGGL(k_qj_norms0<true>, go, dim3(256), 0, c.stream, dj, scale);
   else
-    hipLaunchKernelGGL(k_qj_norms0<false>, go, dim3(256), 0, c.stream, dj);
+    hipLaunchKernelGGL(k_qj_norms0<false>, go, dim3(256), 0, c.stream, dj, scale);
   hipLaunchKernelGGL(k_qj_rank, go, dim3(256), 0, c.stream, dj);
   const dim3 gg(up16(maxo) / 16, nj, std::min(16, up16(maxn) / 16));
   if (z)
@@ -1135,7 +1163,7 @@ void qj_solve(QjBatch& q, double norm2) {
   const int nbmax = (std::max(2, pk) + 1) & ~1;
   const int chunk = nbmax / 2;
   const double tol = std::max(1e-14, 4.0 * 2.220446049250313e-16 * std::sqrt((double)maxK));
-  const double fl = 1e-11;  // relative to |AA|, which the scaling puts in [1/2, 1)
+  const double fl = 1e-11;  // relative to the sector's norm, which the scaling puts in [1/2, 1)
   const int limit = c.jacobi_sweeps * (nbmax - 1);
   int step = 0;
   bool done = false;
@@ -1173,6 +1201,7 @@ void qj_solve(QjBatch& q, double norm2) {
   for (int j = 0; j < nj; ++j) {
     QjSector& s = sec[j];
     const double* v = h + (q.jobs[j].nrm - q.work);
+    const double factor = v[up16(s.o)];
     for (int i = 0; i < up16(s.K); ++i) s.ok = s.ok && std::isfinite(v[i]);
     if (!s.ok) continue;
     s.col.resize(up16(s.K));
@@ -1182,7 +1211,7 @@ void qj_solve(QjBatch& q, double norm2) {
     s.sigma.resize(s.K);
     s.inv.resize(s.K);
     for (int i = 0; i < s.K; ++i) {
-      s.sigma[i] = v[s.col[i]] / scale;
+      s.sigma[i] = v[s.col[i]] / factor / scale;
       s.inv[i] = v[s.col[i]] > 0.0 ? 1.0 / v[s.col[i]] : 0.0;
     }
   }

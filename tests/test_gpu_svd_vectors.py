@@ -195,3 +195,19 @@ def test_squared_norm_out_of_range(pkg, ctx, scale, cplx, direction):
     want = want / np.linalg.norm(want) * scale
     # (squares of 1e-154 are subnormal: half a unit of 5e-324)
     assert abs(te.value - np.sum(want[kept:] ** 2)) <= 1e-12 * np.sum(want[kept:] ** 2) + 1e-322
+
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("weak", [1e-6, 1e-20, 1e-40])
+@pytest.mark.parametrize("Q", [5, 1, -1])
+def test_weak_sector(pkg, ctx, Q, weak, cplx, direction):
+    """One charge sector far below the others: its values and vectors are
+    accurate to its own norm (sectors of 3, 43 .. 67 and 19 .. 52 rows)."""
+    A, charges, M, sectors = _charged(cplx, np.random.default_rng(23), DIMS,
+                                      edit=lambda q, S: S * (weak if q == Q else 1.0))
+    assert Q in sectors
+    t = pkg.site2_from_dense(ctx, A, *charges)
+    L, Rt, sv = _svd(pkg, ctx, t, 1, direction)
+    _check_sectors(M, sectors, L, Rt, sv, direction)
