@@ -1013,7 +1013,12 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     // sectors, whose factor is a set of eigenvectors) re-orthonormalised in
     // place, then an orthonormal
     // completion for numerically zero singular values (sigma <= 1e-10
-    // sigma_max); the latter carry no weight
+    // sigma_max); the latter carry no weight.  Block Jacobi columns are
+    // orthogonal to the pair tolerance, 1e-14, down to the solver's floor, 1e-11
+    // of the sector's norm, and to 1e-14 floor / sigma below it, which the other
+    // factor's product would multiply by the largest sigma: they are
+    // re-orthonormalised below twice the floor and replaced where they are no
+    // more than rounding, 1e-14 of that norm.
     double smax = 0.0;
     for (int64_t i = 0; i < n; ++i) smax = std::max(smax, ents[i].v);
     const double szero = 1e-10 * smax;
@@ -1023,13 +1028,17 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     for (int si : order) {
       Sec& s = secs[si];
       if (s.keep > 0) {
+        double sn = 0.0;  // the sector's norm
+        for (int l = 0; l < s.kmin; ++l) sn += hs[hoff + l] * hs[hoff + l];
+        sn = std::sqrt(sn);
         int c0 = s.keep;
         // (the one-launch kernel's vectors are orthonormal whatever their weight;
         // only vanishing columns, below the range of the products, are not)
-        while (c0 > 0 && hs[hoff + c0 - 1] <= (s.tiny ? 1e-60 * smax : szero)) --c0;
+        const double zero = s.tiny ? 1e-60 * smax : s.qj >= 0 ? 1e-14 * sn : szero;
+        while (c0 > 0 && hs[hoff + c0 - 1] <= zero) --c0;
         int c1 = c0;
-        if (!s.gram && !s.tiny && s.qj < 0)  // Gram eigenvectors and Jacobi columns need no re-orthonormalisation
-          while (c1 > 1 && hs[hoff + c1 - 1] < ssmall) --c1;
+        const double weak = s.gram || s.tiny ? 0.0 : s.qj >= 0 ? 2e-11 * sn : ssmall;
+        while (c1 > 1 && hs[hoff + c1 - 1] < weak) --c1;
         const int nv = (int)(dir > 0 ? s.R : s.C);
         if (c1 < c0 && c1 >= 1) {
           if (dir > 0)

@@ -211,3 +211,27 @@ def test_weak_sector(pkg, ctx, Q, weak, cplx, direction):
     t = pkg.site2_from_dense(ctx, A, *charges)
     L, Rt, sv = _svd(pkg, ctx, t, 1, direction)
     _check_sectors(M, sectors, L, Rt, sv, direction)
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("shape", [(90, 64), (200, 230), (500, 480)])
+def test_truncation_inside_a_weak_tail(pkg, ctx, shape, cplx, direction):
+    """A flat spectrum and a tail of 1e-10 to 1e-13 of the largest value, cut in its
+    middle: what is kept is the best approximation, to the rounding of the
+    solver, and the factor an isometry."""
+    R, Cc = shape
+    rng = np.random.default_rng(R + 3 * Cc)
+    K, n = min(R, Cc), max(R, Cc)
+    s = np.ones(K)
+    s[K // 2:] = np.logspace(-10, -13, K - K // 2)
+    U, V = (np.linalg.qr(rng.standard_normal((d, K)) + (1j * rng.standard_normal((d, K)) if cplx else 0.0))[0]
+            for d in (R, Cc))
+    M = (U * s) @ V.conj().T / np.linalg.norm(s)
+    t = pkg.site2_from_dense(ctx, M.reshape(R, 1, 1, Cc))
+    keep = 3 * K // 4
+    L, Rt, sv = _svd(pkg, ctx, t, 0, direction, keep)
+    assert len(sv) == keep
+    best = np.linalg.norm(np.linalg.svd(M, compute_uv=False)[keep:])
+    assert np.linalg.norm(L @ Rt - M, 2) <= best + 16 * n * EPS
+    assert _isometry(L, Rt, direction) <= 1e-13 + 4 * n * EPS
