@@ -387,7 +387,8 @@ struct CompleteJob {
   double* Q;          // canonical factor: element r of vector c at Q[c vs + r es]
   int64_t vs, es;
   int n, c0, keep;    // vectors c0 .. keep-1 are replaced
-  // scratch, set by complete_basis
+  int64_t plane = 0;  // distance of the imaginary parts (0: real), the same kind in all jobs of a call
+  // scratch, set by complete_basis (complex: two planes each)
   double* W = nullptr;     // n x 32 candidates
   double* coef = nullptr;  // keep x 32
   double* d = nullptr;     // n residuals

@@ -85,8 +85,8 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     int64_t R = 0, C = 0;
     double *M = nullptr, *U = nullptr, *Vt = nullptr, *s = nullptr, *E = nullptr;
     int kmin = 0, keep = 0;
-    // sectors solved for one orthonormal factor (block Jacobi, backend 4, or
-    // Gram eigensolve, backend 5); the other factor comes from a GEMM with M.
+    // sectors solved for one orthonormal factor (block Jacobi, Gram and complex
+    // augmented eigensolves); the other factor comes from a GEMM with M.
     // colsrc / coldiv: source column (rowsX elements) and divisor of the k-th
     // largest singular vector of that side
     double* X = nullptr;
@@ -534,6 +534,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
           const int64_t j = b - cls[k];
           jobs.push_back({s.M, aug + aoff[k] + 2 * j * NNk, augW + voff[k] + j * Nk, s.U, s.s, s.Vt, (int)s.R,
                           (int)s.C, Nk, s.kmin});
+          s.bj = 1;                // the other factor from the grouped GEMM below
           is_small[big[b]] = 1;  // handled
           const double n2 = (double)Nk;
           svd_flops += 4.0 * 9.0 * n2 * n2 * n2;
@@ -830,7 +831,7 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
           s.colsrc.push_back(s.X + (int64_t)l * s.kmin);
           s.coldiv.push_back(1.0);
         }
-      } else if (s.bj) {
+      } else if (s.bj && !z) {
         // block-Jacobi sector: column norms sorted descending (stable), the
         // largest kmin are the singular values
         s.perm.resize(s.ncolsX);
@@ -925,13 +926,13 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
           q.es = dir > 0 ? 1 : s.kmin;
           q.vs = dir > 0 ? s.R : 1;
           q.oplane = s.kmin * (dir > 0 ? s.R : s.C);
-          if (z) {
-            planes.add(s.M, s.R * s.C, true);
-            planes.add(s.U, s.R * s.kmin, true);
-            planes.add(s.Vt, s.kmin * s.C, true);
-          }
         }
-        for (int k = 0; k < s.keep && s.qj < 0; ++k) {
+        if (z) {
+          planes.add(s.M, s.R * s.C, true);
+          planes.add(s.U, s.R * s.kmin, true);
+          planes.add(s.Vt, s.kmin * s.C, true);
+        }
+        for (int k = 0; k < s.keep && s.qj < 0 && !z; ++k) {
           const double* src = s.colsrc[k];
           if (dir > 0)
             gat.push_back({src, s.U + (int64_t)k * s.R, 1, s.coldiv[k], s.rowsX, 0});
@@ -1018,7 +1019,8 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
     // of the sector's norm, and to 1e-14 floor / sigma below it, which the other
     // factor's product would multiply by the largest sigma: they are
     // re-orthonormalised below twice the floor and replaced where they are no
-    // more than rounding, 1e-14 of that norm.
+    // more than rounding, 1e-14 of that norm.  (Complex eigensolves: the bounds
+    // of the real ones, relative to the sector's norm.)
     double smax = 0.0;
     for (int64_t i = 0; i < n; ++i) smax = std::max(smax, ents[i].v);
     const double szero = 1e-10 * smax;
@@ -1034,71 +1036,31 @@ SvdResult svd_trunc(Context& c, const Tensor& AA, int64_t m, int64_t minm, doubl
         int c0 = s.keep;
         // (the one-launch kernel's vectors are orthonormal whatever their weight;
         // only vanishing columns, below the range of the products, are not)
-        const double zero = s.tiny ? 1e-60 * smax : s.qj >= 0 ? 1e-14 * sn : szero;
+        const double zero = s.tiny ? 1e-60 * smax : s.qj >= 0 ? 1e-14 * sn : z ? 1e-10 * sn : szero;
         while (c0 > 0 && hs[hoff + c0 - 1] <= zero) --c0;
         int c1 = c0;
-        const double weak = s.gram || s.tiny ? 0.0 : s.qj >= 0 ? 2e-11 * sn : ssmall;
+        const double weak = s.gram || s.tiny ? 0.0 : s.qj >= 0 ? 2e-11 * sn : z ? 1e-2 * sn : ssmall;
         while (c1 > 1 && hs[hoff + c1 - 1] < weak) --c1;
         const int nv = (int)(dir > 0 ? s.R : s.C);
+        const int64_t plane = z ? (int64_t)s.kmin * nv : 0;
         if (c1 < c0 && c1 >= 1) {
           if (dir > 0)
-            rj.push_back({s.U, s.R, 1, nv, c1, c0});
+            rj.push_back({s.U, s.R, 1, nv, c1, c0, plane});
           else
-            rj.push_back({s.Vt, 1, s.kmin, nv, c1, c0});
+            rj.push_back({s.Vt, 1, s.kmin, nv, c1, c0, plane});
         }
         if (c0 < s.keep) {
           if (dir > 0)
-            cj.push_back({s.U, s.R, 1, nv, c0, s.keep});
+            cj.push_back({s.U, s.R, 1, nv, c0, s.keep, plane});
           else
-            cj.push_back({s.Vt, 1, s.kmin, nv, c0, s.keep});
+            cj.push_back({s.Vt, 1, s.kmin, nv, c0, s.keep, plane});
         }
       }
       hoff += s.kmin;
     }
-    if (!z) {
-      reorth_basis(c, rj);
-      complete_basis(c, cj);
-    }
-    // complex: vectors whose columns ended below the solver's floor are
-    // orthogonal to the others to 1e-14 floor / sigma only, which the other
-    // factor's product would multiply by the largest sigma; there is no
-    // completion here, they are projected off the others
-    std::vector<double*> scratch;
-    if (z) {
-      std::vector<GemmTask> t1, t2;
-      std::vector<GemmSeg> s1, s2;
-      const double low = std::max(szero, 2e-11 * std::sqrt(aa2));
-      hoff = 0;
-      for (int si : order) {
-        Sec& s = secs[si];
-        int c0 = s.qj >= 0 ? s.keep : 0;
-        while (c0 > 0 && hs[hoff + c0 - 1] <= low) --c0;
-        hoff += s.kmin;
-        const int nz = s.keep - c0;
-        if (c0 == 0 || nz == 0) continue;
-        double* co = (double*)c.alloc.alloc((int64_t)2 * c0 * nz * sizeof(double));
-        scratch.push_back(co);
-        planes.add(co, (int64_t)c0 * nz, true);
-        if (dir > 0) {  // U1 -= U0 (U0^H U1)
-          double* u1 = s.U + (int64_t)c0 * s.R;
-          t1.push_back({co, c0, c0, nz, (int)s1.size(), 1, 0.0});
-          s1.push_back({s.U, u1, s.R, s.R, (int)s.R, 1 | kSegConjA, 1.0});
-          t2.push_back({u1, s.R, (int)s.R, nz, (int)s2.size(), 1, 1.0});
-          s2.push_back({s.U, co, s.R, c0, c0, 0, -1.0});
-        } else {  // V1^H -= (V1^H V0) V0^H
-          t1.push_back({co, nz, nz, c0, (int)s1.size(), 1, 0.0});
-          s1.push_back({s.Vt + c0, s.Vt, s.kmin, s.kmin, (int)s.C, 2 | kSegConjB, 1.0});
-          t2.push_back({s.Vt + c0, s.kmin, nz, (int)s.C, (int)s2.size(), 1, 1.0});
-          s2.push_back({co, s.Vt, nz, s.kmin, c0, 0, -1.0});
-        }
-      }
-      complexify_gemm(t1, s1, planes);
-      complexify_gemm(t2, s2, planes);
-      launch_gemm(c, t1, s1, -1);
-      launch_gemm(c, t2, s2, -1);
-    }
+    reorth_basis(c, rj);
+    complete_basis(c, cj);
     issue_gemm_arith(c, gp);
-    for (double* p : scratch) c.alloc.release(p);
     issue_copy(c, sp);
   }
   for (auto& s : secs) {

@@ -334,73 +334,113 @@ __device__ int cb_argmax(const double* d, int n, const int* excl, int nex, doubl
 // Exact greedy step: v = e_j after two classical Gram-Schmidt passes against
 // vectors 0 .. c-1 of Q; returns |v|.  Loops are ordered so that consecutive
 // lanes read consecutive addresses for both layouts (es == 1: vectors are
-// columns; vs == 1: rows).
+// columns; vs == 1: rows).  Complex (Z): imaginary planes of v, coef and Q, and
+// inner products sum conj(q) v.
+template <bool Z>
 __device__ double complete_candidate(const CompleteJob& jb, double* v, double* coef, int c, int j, double* red) {
   const int n = jb.n;
+  const int64_t vp = (int64_t)kCB * n, cp = (int64_t)kCB * jb.keep, qp = jb.plane;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   constexpr int kWaves = kBjThreads / 64;
-  for (int r = threadIdx.x; r < n; r += kBjThreads) v[r] = (r == j) ? 1.0 : 0.0;
+  for (int r = threadIdx.x; r < n; r += kBjThreads) {
+    v[r] = (r == j) ? 1.0 : 0.0;
+    if constexpr (Z) v[vp + r] = 0.0;
+  }
   __syncthreads();
+  // (a, b) += conj(q) v and (a, b) -= coef q, element by element
+  auto dot = [&](const double* q, int r, double& a, double& b) {
+    a += q[0] * v[r];
+    if constexpr (Z) {
+      a += q[qp] * v[vp + r];
+      b += q[0] * v[vp + r] - q[qp] * v[r];
+    }
+  };
+  auto sub = [&](int p, const double* q, double& a, double& b) {
+    a -= coef[p] * q[0];
+    if constexpr (Z) {
+      a += coef[cp + p] * q[qp];
+      b -= coef[p] * q[qp] + coef[cp + p] * q[0];
+    }
+  };
   for (int pass = 0; pass < 2; ++pass) {
     if (jb.es == 1) {
       for (int p = wave; p < c; p += kWaves) {
         const double* q = jb.Q + (int64_t)p * jb.vs;
-        double a = 0.0;
-        for (int r = lane; r < n; r += 64) a += q[r] * v[r];
-        for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
-        if (lane == 0) coef[p] = a;
+        double a = 0.0, b = 0.0;
+        for (int r = lane; r < n; r += 64) dot(q + r, r, a, b);
+        for (int o = 32; o > 0; o >>= 1) {
+          a += __shfl_down(a, o, 64);
+          if constexpr (Z) b += __shfl_down(b, o, 64);
+        }
+        if (lane == 0) {
+          coef[p] = a;
+          if constexpr (Z) coef[cp + p] = b;
+        }
       }
     } else {
       for (int p = threadIdx.x; p < c; p += kBjThreads) {
-        double a = 0.0;
-        for (int r = 0; r < n; ++r) a += jb.Q[(int64_t)p * jb.vs + (int64_t)r * jb.es] * v[r];
+        double a = 0.0, b = 0.0;
+        for (int r = 0; r < n; ++r) dot(jb.Q + (int64_t)p * jb.vs + (int64_t)r * jb.es, r, a, b);
         coef[p] = a;
+        if constexpr (Z) coef[cp + p] = b;
       }
     }
     __syncthreads();
     if (jb.es == 1) {
       for (int r = threadIdx.x; r < n; r += kBjThreads) {
-        double a = v[r];
-        for (int p = 0; p < c; ++p) a -= coef[p] * jb.Q[(int64_t)p * jb.vs + r];
+        double a = v[r], b = Z ? v[vp + r] : 0.0;
+        for (int p = 0; p < c; ++p) sub(p, jb.Q + (int64_t)p * jb.vs + r, a, b);
         v[r] = a;
+        if constexpr (Z) v[vp + r] = b;
       }
     } else {
       for (int r = wave; r < n; r += kWaves) {
         const double* q = jb.Q + (int64_t)r * jb.es;  // element r of every vector, contiguous over p
-        double a = 0.0;
-        for (int p = lane; p < c; p += 64) a += coef[p] * q[p];
-        for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
-        if (lane == 0) v[r] -= a;
+        double a = 0.0, b = 0.0;
+        for (int p = lane; p < c; p += 64) sub(p, q + p, a, b);
+        for (int o = 32; o > 0; o >>= 1) {
+          a += __shfl_down(a, o, 64);
+          if constexpr (Z) b += __shfl_down(b, o, 64);
+        }
+        if (lane == 0) {
+          v[r] += a;
+          if constexpr (Z) v[vp + r] += b;
+        }
       }
     }
     __syncthreads();
   }
   double a = 0.0;
-  for (int r = threadIdx.x; r < n; r += kBjThreads) a += v[r] * v[r];
+  for (int r = threadIdx.x; r < n; r += kBjThreads) a += v[r] * v[r] + (Z ? v[vp + r] * v[vp + r] : 0.0);
   return sqrt(cb_block_sum(a, red));
 }
 
 // Q vectors c .. c+s-1 = W columns 0 .. s-1; d_r -= sum of their squares.
+template <bool Z>
 __device__ void cb_store(const CompleteJob& jb, int c, int s) {
   const int n = jb.n;
   if (s <= 0) return;
-  if (jb.es == 1) {
-    for (int u = 0; u < s; ++u)
-      for (int r = threadIdx.x; r < n; r += kBjThreads)
-        jb.Q[(int64_t)(c + u) * jb.vs + r] = jb.W[(int64_t)u * n + r];
-  } else {
-    for (int64_t e = threadIdx.x; e < (int64_t)s * n; e += kBjThreads) {
-      const int u = (int)(e % s), r = (int)(e / s);
-      jb.Q[(int64_t)(c + u) * jb.vs + (int64_t)r * jb.es] = jb.W[(int64_t)u * n + r];
+  for (int h = 0; h < (Z ? 2 : 1); ++h) {
+    double* Q = jb.Q + h * jb.plane;
+    const double* W = jb.W + h * (int64_t)kCB * n;
+    if (jb.es == 1) {
+      for (int u = 0; u < s; ++u)
+        for (int r = threadIdx.x; r < n; r += kBjThreads)
+          Q[(int64_t)(c + u) * jb.vs + r] = W[(int64_t)u * n + r];
+    } else {
+      for (int64_t e = threadIdx.x; e < (int64_t)s * n; e += kBjThreads) {
+        const int u = (int)(e % s), r = (int)(e / s);
+        Q[(int64_t)(c + u) * jb.vs + (int64_t)r * jb.es] = W[(int64_t)u * n + r];
+      }
     }
-  }
-  for (int r = threadIdx.x; r < n; r += kBjThreads) {
-    double a = jb.d[r];
-    for (int u = 0; u < s; ++u) {
-      const double q = jb.W[(int64_t)u * n + r];
-      a -= q * q;
+    for (int r = threadIdx.x; r < n; r += kBjThreads) {
+      double a = jb.d[r];
+      for (int u = 0; u < s; ++u) {
+        const double q = W[(int64_t)u * n + r];
+        a -= q * q;
+      }
+      jb.d[r] = a;
     }
-    jb.d[r] = a;
   }
   __syncthreads();
 }
@@ -408,6 +448,7 @@ __device__ void cb_store(const CompleteJob& jb, int c, int s) {
 // b < 0: residuals d of all unit vectors and the first candidate block.
 // b >= 0: finish block b (its candidates in W have been projected against
 // vectors 0 .. c0 + kCB b - 1), then set up the candidates of block b + 1.
+template <bool Z>
 __global__ __launch_bounds__(kBjThreads) void k_complete_block(const CompleteJob* __restrict__ jobs, int njobs,
                                                                int b) {
   __shared__ double red[4];
@@ -417,6 +458,7 @@ __global__ __launch_bounds__(kBjThreads) void k_complete_block(const CompleteJob
   for (int ji = blockIdx.x; ji < njobs; ji += gridDim.x) {
     const CompleteJob jb = jobs[ji];
     const int n = jb.n;
+    const int64_t wp = (int64_t)kCB * n;
     int cnext;
     if (b < 0) {
       if (jb.es == 1) {
@@ -425,6 +467,10 @@ __global__ __launch_bounds__(kBjThreads) void k_complete_block(const CompleteJob
           for (int p = 0; p < jb.c0; ++p) {
             const double q = jb.Q[(int64_t)p * jb.vs + j];
             a -= q * q;
+            if constexpr (Z) {
+              const double y = jb.Q[jb.plane + (int64_t)p * jb.vs + j];
+              a -= y * y;
+            }
           }
           jb.d[j] = a;
         }
@@ -433,7 +479,10 @@ __global__ __launch_bounds__(kBjThreads) void k_complete_block(const CompleteJob
         for (int j = wave; j < n; j += kBjThreads / 64) {
           const double* q = jb.Q + (int64_t)j * jb.es;  // contiguous over p
           double a = 0.0;
-          for (int p = lane; p < jb.c0; p += 64) a += q[p] * q[p];
+          for (int p = lane; p < jb.c0; p += 64) {
+            a += q[p] * q[p];
+            if constexpr (Z) a += q[jb.plane + p] * q[jb.plane + p];
+          }
           for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
           if (lane == 0) jb.d[j] = 1.0 - a;
         }
@@ -450,33 +499,52 @@ __global__ __launch_bounds__(kBjThreads) void k_complete_block(const CompleteJob
         for (int pass = 0; pass < 2; ++pass)
           for (int u = 0; u < s; ++u) {
             const double* wu = jb.W + (int64_t)u * n;
-            double a = 0.0;
-            for (int r = threadIdx.x; r < n; r += kBjThreads) a += wu[r] * wt[r];
+            double a = 0.0, ai = 0.0;
+            for (int r = threadIdx.x; r < n; r += kBjThreads) {
+              a += wu[r] * wt[r];
+              if constexpr (Z) {
+                a += wu[wp + r] * wt[wp + r];
+                ai += wu[r] * wt[wp + r] - wu[wp + r] * wt[r];
+              }
+            }
             a = cb_block_sum(a, red);
-            for (int r = threadIdx.x; r < n; r += kBjThreads) wt[r] -= a * wu[r];
+            if constexpr (Z) ai = cb_block_sum(ai, red);
+            for (int r = threadIdx.x; r < n; r += kBjThreads) {
+              wt[r] -= a * wu[r];
+              if constexpr (Z) {
+                wt[r] += ai * wu[wp + r];
+                wt[wp + r] -= a * wu[wp + r] + ai * wu[r];
+              }
+            }
             __syncthreads();
           }
         double a = 0.0;
-        for (int r = threadIdx.x; r < n; r += kBjThreads) a += wt[r] * wt[r];
+        for (int r = threadIdx.x; r < n; r += kBjThreads) a += wt[r] * wt[r] + (Z ? wt[wp + r] * wt[wp + r] : 0.0);
         const double nrm2 = cb_block_sum(a, red);
         if (nrm2 >= 1e-4 && nrm2 >= 0.1 * jb.seld[t]) {
           const double inv = 1.0 / sqrt(nrm2);
           double* ws = jb.W + (int64_t)s * n;
-          for (int r = threadIdx.x; r < n; r += kBjThreads) ws[r] = wt[r] * inv;
+          for (int r = threadIdx.x; r < n; r += kBjThreads) {
+            ws[r] = wt[r] * inv;
+            if constexpr (Z) ws[wp + r] = wt[wp + r] * inv;
+          }
           __syncthreads();
           ++s;
         }
       }
-      cb_store(jb, cb, s);
+      cb_store<Z>(jb, cb, s);
       // places left by dropped candidates: exact greedy steps against all
       // vectors so far (W is free now: column 0 serves as the work vector)
       for (int col = cb + s; col < cb + nb; ++col) {
         const int j = cb_argmax(jb.d, n, cand_sh, 0, bv, bi);
-        const double nrm = complete_candidate(jb, jb.W, jb.coef, col, j, red);
+        const double nrm = complete_candidate<Z>(jb, jb.W, jb.coef, col, j, red);
         const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
-        for (int r = threadIdx.x; r < n; r += kBjThreads) jb.W[r] *= inv;
+        for (int r = threadIdx.x; r < n; r += kBjThreads) {
+          jb.W[r] *= inv;
+          if constexpr (Z) jb.W[wp + r] *= inv;
+        }
         __syncthreads();
-        cb_store(jb, col, 1);
+        cb_store<Z>(jb, col, 1);
       }
       cnext = cb + nb;
     }
@@ -491,7 +559,10 @@ __global__ __launch_bounds__(kBjThreads) void k_complete_block(const CompleteJob
       }
       __syncthreads();
     }
-    for (int64_t e = threadIdx.x; e < (int64_t)nbn * n; e += kBjThreads) jb.W[e] = 0.0;
+    for (int64_t e = threadIdx.x; e < (int64_t)nbn * n; e += kBjThreads) {
+      jb.W[e] = 0.0;
+      if constexpr (Z) jb.W[wp + e] = 0.0;
+    }
     __syncthreads();
     if (threadIdx.x < nbn) jb.W[(int64_t)threadIdx.x * n + cand_sh[threadIdx.x]] = 1.0;
     __syncthreads();
@@ -500,26 +571,40 @@ __global__ __launch_bounds__(kBjThreads) void k_complete_block(const CompleteJob
 
 void complete_basis(Context& c, std::vector<CompleteJob>& jobs) {
   if (jobs.empty()) return;
+  const bool z = jobs[0].plane != 0;
   std::vector<double*> scratch;
+  BufMap planes;
   int nblk = 0;
   for (CompleteJob& j : jobs) {
     if (j.c0 < 0 || j.keep > j.n || j.c0 >= j.keep) throw Error(DMRJ_ERR_STATE, "completion job out of range");
-    const int64_t sz = (int64_t)kCB * j.n + (int64_t)kCB * j.keep + j.n + 2 * kCB;
+    const int64_t zf = z ? 2 : 1, wn = zf * kCB * j.n, cn = zf * kCB * j.keep;
+    const int64_t sz = wn + cn + j.n + 2 * kCB;
     double* p = (double*)c.alloc.alloc(sz * (int64_t)sizeof(double));
     scratch.push_back(p);
     j.W = p;
-    j.coef = j.W + (int64_t)kCB * j.n;
-    j.d = j.coef + (int64_t)kCB * j.keep;
+    j.coef = j.W + wn;
+    j.d = j.coef + cn;
     j.seld = j.d + j.n;
     j.cand = reinterpret_cast<int*>(j.seld + kCB);
+    if (z) {
+      planes.add(j.Q, j.plane, true);
+      planes.add(j.W, (int64_t)kCB * j.n, true);
+      planes.add(j.coef, (int64_t)kCB * j.keep, true);
+    }
     nblk = std::max(nblk, (j.keep - j.c0 + kCB - 1) / kCB);
   }
   auto* dj = (CompleteJob*)c.upload(jobs.data(), jobs.size() * sizeof(CompleteJob));
   const unsigned grid = (unsigned)std::min<size_t>(jobs.size(), 1024);
-  hipLaunchKernelGGL(k_complete_block, dim3(grid), dim3(kBjThreads), 0, c.stream, dj, (int)jobs.size(), -1);
-  HIP_OK(hipGetLastError());
+  auto block = [&](int b) {
+    if (z)
+      hipLaunchKernelGGL(k_complete_block<true>, dim3(grid), dim3(kBjThreads), 0, c.stream, dj, (int)jobs.size(), b);
+    else
+      hipLaunchKernelGGL(k_complete_block<false>, dim3(grid), dim3(kBjThreads), 0, c.stream, dj, (int)jobs.size(), b);
+    HIP_OK(hipGetLastError());
+  };
+  block(-1);
   for (int b = 0; b < nblk; ++b) {
-    // W -= Q (Q^T W) twice; op(Q^T) is cb x n, op(Q) n x cb
+    // W -= Q (Q^H W) twice; op(Q^H) is cb x n, op(Q) n x cb
     std::vector<GemmTask> t1, t2;
     std::vector<GemmSeg> s1, s2;
     for (const CompleteJob& j : jobs) {
@@ -529,17 +614,20 @@ void complete_basis(Context& c, std::vector<CompleteJob>& jobs) {
       const bool cols = j.es == 1;
       const int64_t ldq = cols ? j.vs : j.es;
       t1.push_back({j.coef, j.keep, cb, nb, (int)s1.size(), 1, 0.0});
-      s1.push_back({j.Q, j.W, ldq, j.n, j.n, cols ? 1 : 0, 1.0});
+      s1.push_back({j.Q, j.W, ldq, j.n, j.n, (cols ? 1 : 0) | (z ? kSegConjA : 0), 1.0});
       t2.push_back({j.W, j.n, j.n, nb, (int)s2.size(), 1, 1.0});
       s2.push_back({j.Q, j.coef, ldq, j.keep, cb, cols ? 0 : 1, -1.0});
+    }
+    if (z) {
+      complexify_gemm(t1, s1, planes);
+      complexify_gemm(t2, s2, planes);
     }
     if (!t1.empty())
       for (int pass = 0; pass < 2; ++pass) {
         launch_gemm(c, t1, s1, -1);
         launch_gemm(c, t2, s2, -1);
       }
-    hipLaunchKernelGGL(k_complete_block, dim3(grid), dim3(kBjThreads), 0, c.stream, dj, (int)jobs.size(), b);
-    HIP_OK(hipGetLastError());
+    block(b);
   }
   for (double* p : scratch) c.alloc.release(p);
 }
@@ -551,6 +639,7 @@ void complete_basis(Context& c, std::vector<CompleteJob>& jobs) {
 // at once, per sector:
 //   W = Q[:, c0:keep];  twice  W -= Q0 (Q0^T W)   (Q0 = the first c0 vectors)
 //   three times  G = W^T W,  W <- W (I - F),  F = strict_upper(G) + diag(G - I) / 2
+// (complex: conjugate transposes, every buffer with an imaginary plane).
 // The second step is the first-order form of the Cholesky-QR update
 // W <- W R^-1 (G = R^T R, R = I + F + O((G-I)^2)): F + F^T = G - I, so
 // (I - F)^T G (I - F) = I + O((G-I)^2) and each pass squares the deviation
@@ -559,7 +648,7 @@ void complete_basis(Context& c, std::vector<CompleteJob>& jobs) {
 // product is one grouped-GEMM launch over all sectors.
 struct ReorthJob {
   double* Q;
-  int64_t vs, es;
+  int64_t vs, es, plane;
   int n, c0, k;
   double* W;  // n x k (column-major)
   double* V;  // n x k, the other buffer of the W <- W (I - F) passes
@@ -569,7 +658,8 @@ struct ReorthJob {
 };
 constexpr int kReorthPasses = 3;
 
-// to_q = 0: W = Q[:, c0:keep]; to_q = 1: Q[:, c0:keep] = W.  Job blockIdx.y.
+// to_q = 0: W = Q[:, c0:keep]; to_q = 1: Q[:, c0:keep] = W.  Job blockIdx.y,
+// plane blockIdx.z.
 __global__ __launch_bounds__(256) void k_reorth_move(const ReorthJob* __restrict__ jobs, int to_q) {
   const ReorthJob jb = jobs[blockIdx.y];
   const int64_t tot = (int64_t)jb.n * jb.k;
@@ -582,8 +672,8 @@ __global__ __launch_bounds__(256) void k_reorth_move(const ReorthJob* __restrict
       r = (int)(e / jb.k);
       u = (int)(e % jb.k);
     }
-    double* q = jb.Q + (int64_t)(jb.c0 + u) * jb.vs + (int64_t)r * jb.es;
-    double* w = jb.W + (int64_t)u * jb.n + r;
+    double* q = jb.Q + blockIdx.z * jb.plane + (int64_t)(jb.c0 + u) * jb.vs + (int64_t)r * jb.es;
+    double* w = jb.W + blockIdx.z * tot + (int64_t)u * jb.n + r;
     if (to_q)
       *q = *w;
     else
@@ -592,14 +682,15 @@ __global__ __launch_bounds__(256) void k_reorth_move(const ReorthJob* __restrict
 }
 
 // T = I - F from G (both k x k column-major): T[u][t] = -G[u][t] (u < t),
-// 1.5 - G[t][t] / 2 (u = t), 0 (u > t).  Job blockIdx.y.
+// 1.5 - G[t][t] / 2 (u = t), 0 (u > t).  Job blockIdx.y, plane blockIdx.z (the
+// imaginary one has no diagonal).
 __global__ __launch_bounds__(256) void k_reorth_tri(const ReorthJob* __restrict__ jobs) {
   const ReorthJob jb = jobs[blockIdx.y];
   const int64_t tot = (int64_t)jb.k * jb.k;
   for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < tot; e += (int64_t)gridDim.x * 256) {
     const int u = (int)(e % jb.k), t = (int)(e / jb.k);
-    const double g = jb.G[e];
-    jb.T[e] = u < t ? -g : (u == t ? 1.5 - 0.5 * g : 0.0);
+    const double g = jb.G[blockIdx.z * tot + e];
+    jb.T[blockIdx.z * tot + e] = u < t ? -g : (u == t && blockIdx.z == 0 ? 1.5 - 0.5 * g : 0.0);
   }
 }
 
@@ -612,20 +703,32 @@ static unsigned reorth_chunks(const std::vector<ReorthJob>& rj, bool square) {
 void reorth_basis(Context& c, std::vector<CompleteJob>& jobs) {
   if (jobs.empty()) return;
   if (jobs.size() > 65535) throw Error(DMRJ_ERR_STATE, "too many sectors for re-orthonormalisation");
+  const bool z = jobs[0].plane != 0;
+  const unsigned zf = z ? 2 : 1;
+  BufMap planes;
   std::vector<ReorthJob> rj;
   std::vector<double*> scratch;
   for (const CompleteJob& j : jobs) {
     if (j.c0 < 1 || j.keep > j.n || j.c0 >= j.keep) throw Error(DMRJ_ERR_STATE, "re-orthonormalisation job out of range");
     const int k = j.keep - j.c0;
     const int64_t nk = (int64_t)j.n * k, kk = (int64_t)k * k;
-    double* p = (double*)c.alloc.alloc((2 * nk + (int64_t)j.c0 * k + 2 * kk) * (int64_t)sizeof(double));
+    const int64_t ck = (int64_t)j.c0 * k;
+    double* p = (double*)c.alloc.alloc(zf * (2 * nk + ck + 2 * kk) * (int64_t)sizeof(double));
     scratch.push_back(p);
-    rj.push_back({j.Q, j.vs, j.es, j.n, j.c0, k, p, p + nk, p + 2 * nk, p + 2 * nk + (int64_t)j.c0 * k,
-                  p + 2 * nk + (int64_t)j.c0 * k + kk});
+    rj.push_back({j.Q, j.vs, j.es, j.plane, j.n, j.c0, k, p, p + zf * nk, p + zf * 2 * nk, p + zf * (2 * nk + ck),
+                  p + zf * (2 * nk + ck + kk)});
+    if (z) {
+      planes.add(j.Q, j.plane, true);
+      planes.add(rj.back().W, nk, true);
+      planes.add(rj.back().V, nk, true);
+      planes.add(rj.back().C, ck, true);
+      planes.add(rj.back().G, kk, true);
+      planes.add(rj.back().T, kk, true);
+    }
   }
   const unsigned nj = (unsigned)rj.size();
   auto* dj = (ReorthJob*)c.upload(rj.data(), rj.size() * sizeof(ReorthJob));
-  hipLaunchKernelGGL(k_reorth_move, dim3(reorth_chunks(rj, false), nj), dim3(256), 0, c.stream, dj, 0);
+  hipLaunchKernelGGL(k_reorth_move, dim3(reorth_chunks(rj, false), nj, zf), dim3(256), 0, c.stream, dj, 0);
   HIP_OK(hipGetLastError());
   {
     // W -= Q0 (Q0^T W), twice
@@ -635,9 +738,13 @@ void reorth_basis(Context& c, std::vector<CompleteJob>& jobs) {
       const bool cols = j.es == 1;
       const int64_t ldq = cols ? j.vs : j.es;
       t1.push_back({j.C, j.c0, j.c0, j.k, (int)s1.size(), 1, 0.0});
-      s1.push_back({j.Q, j.W, ldq, j.n, j.n, cols ? 1 : 0, 1.0});
+      s1.push_back({j.Q, j.W, ldq, j.n, j.n, (cols ? 1 : 0) | (z ? kSegConjA : 0), 1.0});
       t2.push_back({j.W, j.n, j.n, j.k, (int)s2.size(), 1, 1.0});
       s2.push_back({j.Q, j.C, ldq, j.c0, j.c0, cols ? 0 : 1, -1.0});
+    }
+    if (z) {
+      complexify_gemm(t1, s1, planes);
+      complexify_gemm(t2, s2, planes);
     }
     for (int pass = 0; pass < 2; ++pass) {
       launch_gemm(c, t1, s1, -1);
@@ -651,18 +758,22 @@ void reorth_basis(Context& c, std::vector<CompleteJob>& jobs) {
     std::vector<GemmSeg> sg, sv;
     for (const ReorthJob& j : rj) {
       tg.push_back({j.G, j.k, j.k, j.k, (int)sg.size(), 1, 0.0});
-      sg.push_back({j.W, j.W, j.n, j.n, j.n, 1, 1.0});
+      sg.push_back({j.W, j.W, j.n, j.n, j.n, 1 | (z ? kSegConjA : 0), 1.0});
       tv.push_back({j.V, j.n, j.n, j.k, (int)sv.size(), 1, 0.0});
       sv.push_back({j.W, j.T, j.n, j.k, j.k, 0, 1.0});
     }
+    if (z) {
+      complexify_gemm(tg, sg, planes);
+      complexify_gemm(tv, sv, planes);
+    }
     launch_gemm(c, tg, sg, -1);
-    hipLaunchKernelGGL(k_reorth_tri, dim3(tri_chunks, nj), dim3(256), 0, c.stream, dj);
+    hipLaunchKernelGGL(k_reorth_tri, dim3(tri_chunks, nj, zf), dim3(256), 0, c.stream, dj);
     HIP_OK(hipGetLastError());
     launch_gemm(c, tv, sv, -1);
     for (ReorthJob& j : rj) std::swap(j.W, j.V);
     dj = (ReorthJob*)c.upload(rj.data(), rj.size() * sizeof(ReorthJob));
   }
-  hipLaunchKernelGGL(k_reorth_move, dim3(reorth_chunks(rj, false), nj), dim3(256), 0, c.stream, dj, 1);
+  hipLaunchKernelGGL(k_reorth_move, dim3(reorth_chunks(rj, false), nj, zf), dim3(256), 0, c.stream, dj, 1);
   HIP_OK(hipGetLastError());
   for (double* p : scratch) c.alloc.release(p);
 }

@@ -175,7 +175,6 @@ def test_sectors_that_do_not_converge(pkg, ctx, limit, cplx, direction):
     _check_sectors(M, sectors, L, Rt, sv, direction)
 
 
-
 @pytest.mark.parametrize("direction", [1, -1])
 @pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("scale", [1e-170, 3e-154, 1e153])
@@ -195,7 +194,6 @@ def test_squared_norm_out_of_range(pkg, ctx, scale, cplx, direction):
     want = want / np.linalg.norm(want) * scale
     # (squares of 1e-154 are subnormal: half a unit of 5e-324)
     assert abs(te.value - np.sum(want[kept:] ** 2)) <= 1e-12 * np.sum(want[kept:] ** 2) + 1e-322
-
 
 
 @pytest.mark.parametrize("direction", [1, -1])
@@ -235,3 +233,55 @@ def test_truncation_inside_a_weak_tail(pkg, ctx, shape, cplx, direction):
     best = np.linalg.norm(np.linalg.svd(M, compute_uv=False)[keep:])
     assert np.linalg.norm(L @ Rt - M, 2) <= best + 16 * n * EPS
     assert _isometry(L, Rt, direction) <= 1e-13 + 4 * n * EPS
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("sweeps", [40, 0], ids=["jacobi", "eigensolve"])
+@pytest.mark.parametrize("shape", [(9, 12), (16, 16), (210, 16), (16, 230), (40, 33), (33, 70), (130, 257), (280, 300)])
+def test_vanishing_values_keep_an_isometry(pkg, ctx, shape, sweeps, cplx, direction):
+    """Rank-deficient sectors, everything kept: equal columns (singular values
+    at the rounding level), zero rows and columns (exact zeros), one element.  The bounds
+    are those of the vectors with weight."""
+    R, Cc = shape
+    n = max(R, Cc)
+    for kind in ("equal", "zeros", "one"):
+        rng = np.random.default_rng(R * 17 + Cc)
+        if kind == "equal":
+            M = np.repeat(rng.standard_normal((R, -(-Cc // 4))), 4, axis=1)[:, :Cc]
+            M[rng.permutation(R)[:R // 5]] = 0.0
+        elif kind == "one":
+            M = np.zeros((R, Cc))
+            M[R // 2, Cc // 2] = 1.0
+        else:
+            M = np.zeros((R, Cc))
+            M[:R // 3, 1:1 + Cc // 4] = rng.standard_normal((R // 3, Cc // 4))
+        if cplx:
+            M = _phases(M, rng)
+        M = M / np.linalg.norm(M)
+        ctx.set_jacobi_sweeps(sweeps)
+        try:
+            L, Rt, sv = _dense(pkg, ctx, M, direction)
+        finally:
+            ctx.set_jacobi_sweeps(40)
+        assert len(sv) == min(R, Cc)
+        assert np.max(np.abs(sv - np.linalg.svd(M, compute_uv=False))) <= 2 * n * EPS
+        assert np.max(np.abs(L @ Rt - M)) <= 8 * n * EPS
+        assert _isometry(L, Rt, direction) <= 1e-13 + 4 * n * EPS
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("Q", [5, 1])
+def test_sector_of_zeros(pkg, ctx, Q, cplx, direction):
+    """A charge sector without weight that is kept all the same, and a tensor of
+    zeros: the factor is still an isometry."""
+    A, charges, M, sectors = _charged(cplx, np.random.default_rng(41), DIMS,
+                                      edit=lambda q, S: S * (0.0 if q == Q else 1.0))
+    t = pkg.site2_from_dense(ctx, A, *charges)
+    L, Rt, sv = _svd(pkg, ctx, t, 1, direction)
+    _check_sectors(M, sectors, L, Rt, sv, direction)
+    t = pkg.site2_from_dense(ctx, 0.0 * A, *charges)
+    L, Rt, sv = _svd(pkg, ctx, t, 1, direction)
+    assert np.all(sv == 0.0) and np.all(L @ Rt == 0.0)
+    assert _isometry(L, Rt, direction) <= 1e-13
