@@ -11,14 +11,14 @@ is capped by m alone).
 A "step" is one full mixed-precision DMRG sweep (2(L-1) two-site bond steps)
 at m = 2048: split-precision H_eff*psi (FP16x3 with per-block scaling by
 default, --mixed), FP64 environment updates, FP64 Lanczos scalars and 2x2
-Ritz solve on the device, the FP64 Gram-matrix SVD (backend 5), and the FP64
+Ritz solve on the device, the FP64 block Jacobi SVD (backend 5), and the FP64
 Rayleigh-quotient energy correction at the bond each sweep reports.  The ramp
 and --warmup sweeps at m = 2048 are untimed; exactly --steps sweeps are timed
 between two stream synchronisations, with all tensors resident in HBM, no
 per-kernel events and no autotuner trials inside the timed region.
 
 Then, from one copy each of the resulting state, --cmp-sweeps sweeps of the
-plain FP64 drop-in (FP64 everywhere, augmented-matrix SVD, backend 0) and of
+plain FP64 drop-in (FP64 everywhere, block Jacobi SVD, backend 0) and of
 the mixed form, both unprofiled: the sweep-time ratio and the relative energy
 and centre-bond spectrum deviation of the mixed sweeps from the FP64 ones.
 One more sweep of each, with HIP events on every grouped-GEMM launch, gives
@@ -81,7 +81,7 @@ def main():
     ap.add_argument("--mixed", default="f16x3", choices=["f16x3", "bf16x3"],
                     help="headline: arithmetic of the mixed form's H_eff*psi GEMMs")
     ap.add_argument("--mixed-svd", type=int, default=5,
-                    help="headline: SVD backend of the mixed form (5: FP64 Gram eigensolve)")
+                    help="headline: SVD backend of the mixed form (5: FP64 block Jacobi, Gram eigensolve of what it leaves)")
     ap.add_argument("--correction", default="sweep", choices=["sweep", "bond"],
                     help="headline: FP64 Rayleigh-quotient energy of the mixed form at the last bond of every "
                          "sweep or at every bond")
@@ -878,7 +878,7 @@ def bench_compare(pkg, ctx, args, psi, mpo, desc, L, m, base_params):
     best = rows[2]
     out = {
         "metric": "DMRG sweep time, mixed vs FP64 GPU from the same state, and |dE/E| against the FP64 drop-in",
-        "value": best["speedup_vs_fp64_dropin"], "unit": "x (sweep-time ratio, BF16x3 + FP64 env + Gram SVD)",
+        "value": best["speedup_vs_fp64_dropin"], "unit": "x (sweep-time ratio, BF16x3 + FP64 env + SVD backend 5)",
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(t_ref * 1e3, 3),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f64 / bf16x3 / f16x3",
         "data": "synthetic (seeded random product state)",

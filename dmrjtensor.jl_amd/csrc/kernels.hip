@@ -895,8 +895,8 @@ __global__ void k_combine(double* __restrict__ out, double* __restrict__ out2, c
 // Coefficients of the Krylov exponential / Ritz vector on the device (one
 // wave; the Krylov dimension is at most 64, typically 2..12):
 //   k = the Krylov dimension used (first beta_j <= 1e-10 ends the space),
-//   T = Q diag(lam) Q^T by the QL algorithm with implicit shifts (FP64, the
-//   tridiagonal of alpha in sc[0..], beta in sc[64..]),
+//   T = Q diag(lam) Q^T by the QL algorithm with implicit shifts (Dubrulle,
+//   Martin and Wilkinson, Numer. Math. 12 (1968); FP64, the tridiagonal of alpha in sc[0..], beta in sc[64..]),
 //   c = Q exp(pf lam) Q^T e1 with the complex prefactor pf = (pf_re, pf_im),
 //   or (ritz) the eigenvector of the lowest lam signed to c_1 >= 0.
 // coef: real Krylov vectors: c_re[0..r), c_im[r..2r); complex Krylov vectors

@@ -1,11 +1,11 @@
 // Truncated SVD of a two-site tensor (fsvd! of the reference's twostep,
 // algs/DMRG.jl:387-395): the tensor is cut into centre-charge sectors, every
 // sector is decomposed by the selected backend (batched one-sided Jacobi for
-// sectors up to 64, QR-preconditioned block Jacobi, batched symmetric
-// eigensolves of the augmented or Gram matrices, block one-sided Jacobi, or
-// rocSOLVER's SVDs), the singular
-// values of all sectors are sorted and truncated together, and the kept
-// vectors are split into the left and right tensors.
+// sectors up to 16, with backends 3 and 4 up to 64, QR-preconditioned block
+// Jacobi, batched symmetric eigensolves of the augmented or Gram matrices,
+// block one-sided Jacobi, or rocSOLVER's SVDs), the singular values of all
+// sectors are sorted and truncated together, and the kept vectors are split
+// into the left and right tensors.
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>

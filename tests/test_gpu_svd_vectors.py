@@ -285,3 +285,9 @@ def test_sector_of_zeros(pkg, ctx, Q, cplx, direction):
     L, Rt, sv = _svd(pkg, ctx, t, 1, direction)
     assert np.all(sv == 0.0) and np.all(L @ Rt == 0.0)
     assert _isometry(L, Rt, direction) <= 1e-13
+
+
+@pytest.mark.parametrize("limit", [-1, 41])
+def test_sweep_limit_out_of_range(pkg, ctx, limit):
+    with pytest.raises(Exception, match="sweep limit"):
+        ctx.set_jacobi_sweeps(limit)
